@@ -1127,48 +1127,80 @@ static void launch_attention(const AttnParams& P, const StepRows& R, hipStream_t
   else
     launch_attention_r<T, 1>(P, R, nbatch, vec, s);
 }
-// ---- prompt portions on the matrix cores (bfloat16 K/V pools). One wave per (tile of up to 32 query rows of one
-// sequence, query head); the host lists the tiles {first row, rows}. Keys go by 32 at a time:
-//   S^T[key][q] = K Q^T      v_mfma_f32_32x32x16_bf16, A = K rows read straight from the pool (16-byte pieces),
-//                            B = the tile's queries, kept in registers as bf16 high + low parts (two products,
-//                            so the float32 queries keep ~16 bits of mantissa);
-//   scale, cap, mask, running maximum and sum per query: lane (q, half) holds 16 keys of ITS query, so the
-//                            softmax statistics are per-lane values plus one exchange between the two halves;
-//   O^T[dv][q] += V^T P^T    A = V^T gathered from the wave's LDS copy of the 32 V rows, B = the weights, again
-//                            as high + low bf16 parts; O^T keeps each lane's query in the lane, so the running
-//                            rescale is a per-lane multiply.
-// The K operand rows are loaded in the order key(m) = m with bits 2 and 3 swapped: the accumulator registers
-// 0..7 / 8..15 of lane (q, half) then hold keys 8 half + 0..7 of the first / second 16-key group, which is the
-// operand layout of the second product, so the weights never move between lanes.
-constexpr int FL_LDV = 4;  // LDS row padding (elements): the two lane halves land in different banks
+// ---- prompt portions on the matrix cores (bfloat16 K/V pools). One block of four waves per (tile of up to 64 query
+// rows of one sequence, query head); the host lists the tiles {first row, rows}. Waves 0 / 1 hold the tile's query
+// rows 0..31 / 32..63 over the even 32-key groups of the tile's keys, waves 2 / 3 the same rows over the odd groups; the
+// two halves merge through LDS at the end. Per group:
+//   S^T[key][q] = K Q^T      v_mfma_f32_32x32x16_bf16, A = K rows from the block's LDS tile, B = the wave's queries, kept
+//                            in registers as bf16 high + low parts (two products, so the float32 queries keep ~16 bits
+//                            of mantissa);
+//   scale, cap, mask, running maximum and sum per query: lane (q, half) holds 16 keys of ITS query, so the softmax
+//                            statistics are per-lane values plus one exchange between the two halves. Scores are kept
+//                            times log2(e) (v_exp_f32 takes them as they are); groups that every query of the wave sees
+//                            whole skip the mask, groups none sees are skipped, and the rescale of the outputs is
+//                            skipped while no maximum moves;
+//   O^T[dv][q] += V^T P^T    A = V^T by transposed LDS reads of the row-major V tile, B = the weights, again as high +
+//                            low bf16 parts, straight from the accumulators: registers 8 s .. 8 s + 7 of lane (q, half)
+//                            are keys 16 s + 4 half + {0..3, 8..11}, and the transposed reads take the keys in that order.
+// What bounds it: the products (32 of 32 cycles per wave and group at 128 / 128) beside ~1,200 cycles of softmax VALU
+// work, two waves per SIMD sharing the two units. The K / V tile of 64 keys is double-buffered in LDS, the next one in
+// registers: every key row is read from the cache once per 64 queries in whole lines. (One wave per 32 queries with its K
+// rows straight from the cache and 16-bit gathers of V ran at one wave per SIMD and waited for all of it.) 64-row
+// tiles: 2,048 rows x 16 heads are 512 blocks, two per CU, a late (long) tile beside an early one; 128-row tiles leave
+// the last tiles' CUs twice the average work. Measured, 16 heads of 128 over 4 key/value heads, 2,048 rows, capped
+// scores: 330 -> 75 us (142 us while every thread looked its own pieces' rows up in the block table).
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ unsigned pack_bf(float a, float b) {  // round to nearest even (v_cvt_pk_bf16_f32)
   const bf16x2 v = {(__bf16)a, (__bf16)b};
   return __builtin_bit_cast(unsigned, v);
 }
-// float32 exp and tanh on the transcendental unit (v_exp_f32, 1 ulp): the error stays below 1e-6 of the cap
-__device__ __forceinline__ float fast_exp(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896341f); }
-__device__ __forceinline__ float fast_tanh(float x) {
-  const float e = __builtin_amdgcn_exp2f(fminf(x, 15.f) * 2.88539008177792681f);  // e^(2x)
-  return 1.f - 2.f * __builtin_amdgcn_rcpf(e + 1.f);
+// byte offset of 16-byte chunk ch of V row `row` (rows of VROW bytes, each 256-byte part swizzled on its own): the row
+// writes and the transposed reads both spread over the banks
+template <int VROW>
+__device__ __forceinline__ int flash_vswz(int row, int ch) {
+  return VROW * row + 256 * (ch >> 4) + 16 * ((ch & 15) ^ (((row & 3) << 2) | ((row >> 2) & 3)));
 }
+constexpr int FL_KEYS = 64;  // keys per LDS tile: two groups of 32
 template <int KD, int NV>
-__global__ __launch_bounds__(64) void flash_prefill_kernel(AttnParams P, StepRows R, const int* __restrict__ tiles) {
-  constexpr int D = 16 * KD, DV = 32 * NV, LDV = DV + FL_LDV;
-  __shared__ __attribute__((aligned(16))) uint16_t Vl[32 * LDV];
-  const int lane = threadIdx.x, q = lane & 31, hf = lane >> 5;
-  const int row0 = tiles[2 * blockIdx.x], nrows = tiles[2 * blockIdx.x + 1];
+struct FlashLds {
+  static constexpr int LDK = 16 * KD + 8;                            // halves; 16-byte rows offset by 4 banks
+  static constexpr int VROW = (32 * NV + 127) / 128 * 256;           // bytes
+  static constexpr int KB = FL_KEYS * LDK * 2, BUF = KB + FL_KEYS * VROW;
+  static constexpr int MERGE = 2 * (16 * NV + 2) * 64 * 4;           // the odd groups' outputs, maxima and sums
+  static constexpr int BYTES = 2 * BUF > MERGE ? 2 * BUF : MERGE;    // then the tiles' pool rows
+  static constexpr int ALL = BYTES + 2 * 2 * FL_KEYS * 4;
+};
+// registers: wide heads keep more of them live than two waves per SIMD leave each
+template <int KD, int NV>
+__global__ __launch_bounds__(256, (KD <= 8 && NV <= 4) ? 2 : 1) void flash_prefill_kernel(AttnParams P, StepRows R,
+                                                                                        const int* __restrict__ tiles, int ntiles) {
+  typedef FlashLds<KD, NV> L;
+  constexpr int D = 16 * KD, DV = 32 * NV, LDK = L::LDK, VROW = L::VROW, KCH = D / 8, VCH = DV / 8;
+  extern __shared__ __attribute__((aligned(16))) char flash_smem[];
+  const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, q = lane & 31, hf = lane >> 5;
+  const int qw = wv & 1, set = wv >> 1;
   const int vh = P.vheads > 1 ? P.vheads : 1;  // output heads: (query head, value head) pairs with vheads = G
-  const int oh = blockIdx.y, h = oh / vh, g = h / (P.H / P.G), gv = vh > 1 ? oh % vh : g;
+  // tiles from the last (longest) to the middle, then from the first up: a CU's two blocks are a long and a short one
+  const int NO = P.H * vh, rank = blockIdx.x / NO, half = (ntiles + 1) / 2;
+  const int tile = rank < half ? ntiles - 1 - rank : rank - half;
+  const int oh = blockIdx.x % NO, h = oh / vh, g = h / (P.H / P.G), gv = vh > 1 ? oh % vh : g;
+  const int row0 = tiles[2 * tile], nrows = tiles[2 * tile + 1];
   const int KG = P.kshared ? 1 : P.G, kg = P.kshared ? 0 : g;  // a shared key row: the K pool has one head
   const int koff = P.maps > 1 ? (h % P.maps) * D : 0;        // several maps per head sit side by side in a K row
   const int* bt = R.block_table + (long long)R.q_seq[row0] * R.max_blocks;
-  const int qrow = row0 + min(q, nrows - 1);
-  const int qlen = q < nrows ? R.q_len[qrow] : 0;
+  const int qi = 32 * qw + q;
+  const int qrow = row0 + min(qi, nrows - 1);
+  const int qlen = qi < nrows ? R.q_len[qrow] : 0;
   const int kfirst = attn_first_key(P, max(qlen, 1));        // this lane's query sees keys kfirst .. qlen - 1
-  const float slope = P.slopes ? P.slopes[h] : 0.f;
+  const float slope = P.slopes ? P.slopes[h] * 1.44269504088896341f : 0.f;
   const int kmax = R.q_len[row0 + nrows - 1];
   const int kmin = attn_first_key(P, R.q_len[row0]) & ~31;   // the first key any row of the tile sees
+  // the keys that any row of this wave sees (none: a wave past the tile's rows)
+  const int wrows = min(32, nrows - 32 * qw);
+  const int wmax = wrows > 0 ? R.q_len[row0 + 32 * qw + wrows - 1] : 0;
+  const int wmin = wrows > 0 ? attn_first_key(P, R.q_len[row0 + 32 * qw]) : 0;
   // queries: B operand, lane (q, hf) holds dims 16 kk + 8 hf + 0..7
   bf16x8 qhi[KD], qlo[KD];
   {
@@ -1187,139 +1219,193 @@ __global__ __launch_bounds__(64) void flash_prefill_kernel(AttnParams P, StepRow
       qlo[kk] = __builtin_bit_cast(bf16x8, lo);
     }
   }
-  const int m = lane & 31;
-  const int kperm = (m & 0x13) | ((m & 4) << 1) | ((m & 8) >> 1);  // bits 2 and 3 swapped
   f32x16 o[NV];
 #pragma unroll
   for (int j = 0; j < NV; ++j)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[j][r] = 0.f;
   float mi = -1e30f, li = 0.f;
-  const float inv_cap = P.softcap != 0.f ? 1.f / P.softcap : 0.f;
+  // score -> log2 domain: without a cap scale * log2(e); with one cap * log2(e) * tanh(score * scale / cap), the tanh as
+  // 1 - 2 / (2^(x * 2 log2(e)) + 1) on the transcendental unit (v_exp_f32, v_rcp_f32: within 1e-6 of the cap)
+  const bool capped = P.softcap != 0.f;
+  const float capl = P.softcap * 1.44269504088896341f, cin = capped ? P.scale / P.softcap * 2.88539008177792681f : 0.f;
+  const float sc1 = P.scale * 1.44269504088896341f;
   const uint16_t* kc = (const uint16_t*)P.kc;
   const uint16_t* vc = (const uint16_t*)P.vc;
   const long long ldk = P.ldk ? P.ldk : D, ldv = P.ldv ? P.ldv : DV;  // row strides of the pools
-  // The K fragments and V rows of the NEXT key group are requested before the current group is multiplied, so a
-  // group's global round trip passes behind the previous group's products and softmax.
-  constexpr int CH = DV / 8;            // 16-byte pieces per V row
-  constexpr int VPL = 32 * CH / 64;     // V pieces per lane per group
-  u32x4 kf_n[KD], vs_n[VPL];
-  auto fetch = [&](int t0) {
-    {
-      const int key = min(t0 + kperm, kmax - 1);
-      const long long rowidx = (long long)(bt[key / R.bs] * KG + kg) * R.bs + key % R.bs;
-      const uint16_t* kr = kc + rowidx * ldk + koff + 8 * hf;
+  constexpr int NK = (FL_KEYS * KCH + 255) / 256, NVC = (FL_KEYS * VCH + 255) / 256;  // 16-byte pieces per thread
+  u32x4 kr[NK], vr[NVC];
+  // the pool rows {key, value} of a tile's keys, found by one thread per key two tiles ahead (a look at the block table
+  // per piece would put that table's round trip, and the address arithmetic, into every thread's way)
+  int* rows = (int*)(flash_smem + L::BYTES);
+  const int kt = tid & (FL_KEYS - 1);
+  auto find = [&](int t0, int& key) {  // keys past the end: the last key's row, their weights are zero
+    key = min(t0 + kt, kmax - 1);
+    return bt[key / R.bs];
+  };
+  auto note = [&](int key, int blk, int b) {
+    const int off = key % R.bs;
+    rows[2 * FL_KEYS * b + kt] = (blk * KG + kg) * R.bs + off;
+    rows[2 * FL_KEYS * b + FL_KEYS + kt] = (blk * P.G + gv) * R.bs + off;
+  };
+  auto fetch = [&](int b) {
 #pragma unroll
-      for (int kk = 0; kk < KD; ++kk) kf_n[kk] = *(const u32x4*)(kr + 16 * kk);
+    for (int c = 0; c < NK; ++c) {
+      const int i = min(tid + 256 * c, FL_KEYS * KCH - 1);
+      kr[c] = *(const u32x4*)(kc + rows[2 * FL_KEYS * b + i / KCH] * ldk + koff + 8 * (i % KCH));
     }
 #pragma unroll
-    for (int i = 0; i < VPL; ++i) {  // keys past the end: the last key's row, their weights are zero
-      const int c = lane + 64 * i;
-      const int key = min(t0 + c / CH, kmax - 1), seg = c % CH;
-      const long long rowidx = (long long)(bt[key / R.bs] * P.G + gv) * R.bs + key % R.bs;
-      vs_n[i] = *(const u32x4*)(vc + rowidx * ldv + 8 * seg);
+    for (int c = 0; c < NVC; ++c) {
+      const int i = min(tid + 256 * c, FL_KEYS * VCH - 1);
+      vr[c] = *(const u32x4*)(vc + rows[2 * FL_KEYS * b + FL_KEYS + i / VCH] * ldv + 8 * (i % VCH));
     }
   };
-  fetch(kmin);
-  for (int t0 = kmin; t0 < kmax; t0 += 32) {
-    u32x4 kf_c[KD], vs_c[VPL];
+  int nkey, nblk;
+  if (wv == 0) {
+    nblk = find(kmin, nkey);
+    note(nkey, nblk, 0);
+    nblk = find(kmin + FL_KEYS, nkey);
+  }
+  __syncthreads();
+  fetch(0);
+  int buf = 0;
+  for (int t0 = kmin; t0 < kmax; t0 += FL_KEYS, buf ^= 1) {
+    char* kb = flash_smem + buf * L::BUF;
+    char* vb = kb + L::KB;
 #pragma unroll
-    for (int kk = 0; kk < KD; ++kk) kf_c[kk] = kf_n[kk];
-#pragma unroll
-    for (int i = 0; i < VPL; ++i) vs_c[i] = vs_n[i];
-    if (t0 + 32 < kmax) fetch(t0 + 32);
-    // V rows of this key group into LDS
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < VPL; ++i) {
-      const int c = lane + 64 * i;
-      unsigned* dst = (unsigned*)&Vl[(c / CH) * LDV + 8 * (c % CH)];
-      *(unsigned long long*)dst = (unsigned long long)vs_c[i][0] | ((unsigned long long)vs_c[i][1] << 32);
-      *(unsigned long long*)(dst + 2) = (unsigned long long)vs_c[i][2] | ((unsigned long long)vs_c[i][3] << 32);
+    for (int c = 0; c < NK; ++c) {
+      const int i = tid + 256 * c;
+      if (FL_KEYS * KCH % 256 == 0 || i < FL_KEYS * KCH) *(u32x4*)(kb + 2 * (i / KCH * LDK + 8 * (i % KCH))) = kr[c];
     }
-    // S^T = K Q^T
-    f32x16 sacc;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) sacc[r] = 0.f;
+    for (int c = 0; c < NVC; ++c) {
+      const int i = tid + 256 * c;
+      if (FL_KEYS * VCH % 256 == 0 || i < FL_KEYS * VCH) *(u32x4*)(vb + flash_vswz<VROW>(i / VCH, i % VCH)) = vr[c];
+    }
+    if (wv == 0) note(nkey, nblk, buf ^ 1);
+    // one barrier a tile: this buffer's readers of two tiles ago passed the last barrier after they were done
+    __syncthreads();
+    if (wv == 0) nblk = find(t0 + 2 * FL_KEYS, nkey);
+    if (t0 + FL_KEYS < kmax) fetch(buf ^ 1);
+    const int tg = t0 + 32 * set;  // this wave's group
+    if (tg >= wmax || tg + 32 <= wmin) continue;
+    const uint16_t* ks = (const uint16_t*)kb + (32 * set + q) * LDK + 8 * hf;
+    f32x16 s;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = 0.f;
 #pragma unroll
     for (int kk = 0; kk < KD; ++kk) {
-      const bf16x8 kf = __builtin_bit_cast(bf16x8, kf_c[kk]);
-      sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qhi[kk], sacc, 0, 0, 0);
-      sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qlo[kk], sacc, 0, 0, 0);
+      const bf16x8 kf = *(const bf16x8*)(ks + 16 * kk);
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qhi[kk], s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qlo[kk], s, 0, 0, 0);
     }
-    // register r of lane (q, hf) is key t0 + 16 (r >> 3) + 8 hf + (r & 7)
-    float pr[16];
-    float mx = -1e30f;
+    // register r of lane (q, hf) is key tg + (r & 3) + 8 (r >> 2) + 4 hf
+    if (capped) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      float sc = sacc[r] * P.scale;
-      if (P.softcap != 0.f) sc = P.softcap * fast_tanh(sc * inv_cap);
-      const int key = t0 + 16 * (r >> 3) + 8 * hf + (r & 7);
-      sc -= slope * (float)(qlen - 1 - key);
-      const bool vis = key < qlen && key >= kfirst;
-      pr[r] = vis ? sc : -1e30f;
-      mx = fmaxf(mx, pr[r]);
+      for (int r = 0; r < 16; ++r)
+        s[r] = capl - 2.f * capl * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(fminf(s[r] * cin, 43.2808512f)) + 1.f);
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] *= sc1;
     }
+    if (P.slopes) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] -= slope * (float)(qlen - 1 - (tg + (r & 3) + 8 * (r >> 2) + 4 * hf));
+    }
+    if (!__all(tg + 32 <= qlen && tg >= kfirst)) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int key = tg + (r & 3) + 8 * (r >> 2) + 4 * hf;
+        s[r] = key < qlen && key >= kfirst ? s[r] : -1e30f;
+      }
+    }
+    float mx = s[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
     mx = fmaxf(mx, xor_shfl<32>(mx));
     const float mn = fmaxf(mi, mx);
-    const float corr = fast_exp(fmaxf(mi - mn, -100.f));
+    const float corr = __builtin_amdgcn_exp2f(fmaxf(mi - mn, -140.f));
     float sum = 0.f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      pr[r] = pr[r] > -1e29f ? fast_exp(pr[r] - mn) : 0.f;
-      sum += pr[r];
+      s[r] = s[r] > -1e29f ? __builtin_amdgcn_exp2f(s[r] - mn) : 0.f;
+      sum += s[r];
     }
     sum += xor_shfl<32>(sum);
     li = li * corr + sum;
     mi = mn;
+    if (__any(corr != 1.f)) {
 #pragma unroll
-    for (int j = 0; j < NV; ++j)
+      for (int j = 0; j < NV; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) o[j][r] *= corr;
-    bf16x8 phi[2], plo[2];
+        for (int r = 0; r < 16; ++r) o[j][r] *= corr;
+    }
+    // O^T += V^T P^T: the 16-lane group gq reads value columns 16 (gq & 1) .. + 15 of four key rows at a time
+    typedef __attribute__((address_space(3))) s16x4 lds_s4;
+    const int gq = lane >> 4, qq = (lane & 15) >> 2, pp = lane & 3;
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
+    for (int ks2 = 0; ks2 < 2; ++ks2) {
       u32x4 hi, lo;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float a = pr[8 * ks + 2 * i], b = pr[8 * ks + 2 * i + 1];
+        const float a = s[8 * ks2 + 2 * i], b = s[8 * ks2 + 2 * i + 1];
         hi[i] = pack_bf(a, b);
         lo[i] = pack_bf(a - __uint_as_float(hi[i] << 16), b - __uint_as_float(hi[i] & 0xffff0000u));
       }
-      phi[ks] = __builtin_bit_cast(bf16x8, hi);
-      plo[ks] = __builtin_bit_cast(bf16x8, lo);
+      const bf16x8 phi = __builtin_bit_cast(bf16x8, hi), plo = __builtin_bit_cast(bf16x8, lo);
+      const int r0 = 32 * set + 16 * ks2 + 4 * hf + qq;
+#pragma unroll
+      for (int j = 0; j < NV; ++j) {
+        const int c0 = 4 * j + 2 * (gq & 1) + (pp >> 1);
+        const char* v0 = vb + flash_vswz<VROW>(r0, c0) + 8 * (pp & 1);
+        const char* v1 = vb + flash_vswz<VROW>(r0 + 8, c0) + 8 * (pp & 1);
+        const bf16x4 a = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)v0));
+        const bf16x4 b = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)v1));
+        const bf16x8 vf = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+        o[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, phi, o[j], 0, 0, 0);
+        o[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, plo, o[j], 0, 0, 0);
+      }
     }
-    __syncthreads();  // the V rows are in LDS
-    // O^T += V^T P^T: A operand lane (dv = 32 j + m, hf) holds V[16 ks + 8 hf + i][dv], i = 0..7
+  }
+  // the odd groups' share joins the even groups' (the tiles' buffers are free once everybody is here)
+  __syncthreads();
+  float* mg = (float*)flash_smem + (qw * (16 * NV + 2)) * 64 + lane;
+  if (set == 1) {
+    mg[0] = mi;
+    mg[64] = li;
 #pragma unroll
     for (int j = 0; j < NV; ++j)
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        const uint16_t* vp = &Vl[(16 * ks + 8 * hf) * LDV + 32 * j + m];
-        u32x4 vv;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) vv[i] = (unsigned)vp[(2 * i) * LDV] | ((unsigned)vp[(2 * i + 1) * LDV] << 16);
-        const bf16x8 vf = __builtin_bit_cast(bf16x8, vv);
-        o[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, phi[ks], o[j], 0, 0, 0);
-        o[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, plo[ks], o[j], 0, 0, 0);
-      }
+      for (int r = 0; r < 16; ++r) mg[64 * (2 + 16 * j + r)] = o[j][r];
   }
-  if (q < nrows) {  // register r of tile j: value dim 32 j + (r & 3) + 8 (r >> 2) + 4 hf of this lane's query
-    if (P.sink) li += expf(P.sink[h] - mi);  // the sink: a term of the denominator without key or value
+  __syncthreads();
+  if (set == 0 && qi < nrows) {  // register r of tile j: value dim 32 j + (r & 3) + 8 (r >> 2) + 4 hf of this lane's query
+    const float m1 = mg[0], mn = fmaxf(mi, m1);
+    const float c0 = __builtin_amdgcn_exp2f(fmaxf(mi - mn, -140.f)), c1 = __builtin_amdgcn_exp2f(fmaxf(m1 - mn, -140.f));
+    li = li * c0 + mg[64] * c1;
+    if (P.sink) li += __builtin_amdgcn_exp2f(P.sink[h] * 1.44269504088896341f - mn);  // a term of the denominator without key or value
     const float inv = attn_head_gate(P, qrow, h) / li;
-    if (P.out32) {
-      float* out = P.out32 + (long long)qrow * P.ld_out32 + oh * DV;
+    float* out32 = P.out32 ? P.out32 + (long long)qrow * P.ld_out32 + oh * DV : nullptr;
+    bf16* out = P.out32 ? nullptr : (bf16*)P.out + (long long)qrow * P.ld_out + oh * DV;
+    const bool pairs = (P.ld_out & 3) == 0 && ((uintptr_t)P.out & 7) == 0;  // four values as one 8-byte store
 #pragma unroll
-      for (int j = 0; j < NV; ++j)
+    for (int j = 0; j < NV; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) out[32 * j + (r & 3) + 8 * (r >> 2) + 4 * hf] = o[j][r] * inv;
-    } else {
-      bf16* out = (bf16*)P.out + (long long)qrow * P.ld_out + oh * DV;
+      for (int k = 0; k < 4; ++k) {
+        float v[4];
 #pragma unroll
-      for (int j = 0; j < NV; ++j)
+        for (int i = 0; i < 4; ++i) v[i] = (o[j][4 * k + i] * c0 + mg[64 * (2 + 16 * j + 4 * k + i)] * c1) * inv;
+        const int d = 32 * j + 8 * k + 4 * hf;
+        if (out32) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) st(out + 32 * j + (r & 3) + 8 * (r >> 2) + 4 * hf, o[j][r] * inv);
-    }
+          for (int i = 0; i < 4; ++i) out32[d + i] = v[i];
+        } else if (pairs) {
+          *(unsigned long long*)(out + d) = (unsigned long long)pack_bf(v[0], v[1]) | ((unsigned long long)pack_bf(v[2], v[3]) << 32);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) st(out + d + i, v[i]);
+        }
+      }
   }
 }
 // (key size / 16, value size / 32) the kernel is built for: equal key and value sizes 64 / 96 / 128, and the rows of
@@ -1341,10 +1427,10 @@ void flash_prefill(const AttnParams& P, const StepRows& R, const int* tiles, int
   check(flash_prefill_supported(P) && tiles && ntiles > 0 && P.G > 0 && P.H % P.G == 0 && (P.out || P.out32) &&
             (P.vheads <= 1 || P.vheads == P.G),
         "flash prefill: operands");
-  dim3 grid(ntiles, P.H * (P.vheads > 1 ? P.vheads : 1));
-#define FLASH_LAUNCH(KD, NV)                  \
-  if (P.D == 16 * KD && P.Dv == 32 * NV)      \
-    hipLaunchKernelGGL((flash_prefill_kernel<KD, NV>), grid, dim3(64), 0, s, P, R, tiles);
+  const dim3 grid(ntiles * P.H * (P.vheads > 1 ? P.vheads : 1));
+#define FLASH_LAUNCH(KD, NV)             \
+  if (P.D == 16 * KD && P.Dv == 32 * NV) \
+    hipLaunchKernelGGL((flash_prefill_kernel<KD, NV>), grid, dim3(256), (FlashLds<KD, NV>::ALL), s, P, R, tiles, ntiles);
   FLASH_SHAPES(FLASH_LAUNCH)
 #undef FLASH_LAUNCH
   launched("flash_prefill");

@@ -99,10 +99,10 @@ void attn_prepare(const AttnParams& P, const StepRows& R, hipStream_t s);
 void attention(const AttnParams& P, const StepRows& R, hipStream_t s);
 
 // prompt portions on the matrix cores (bfloat16, head sizes 64 / 96 / 128 with dim == vdim): `tiles` is a device
-// table the host builds from the step's rows, per tile {first row, rows <= 32}, rows of one sequence in order
+// table the host builds from the step's rows, per tile {first row, rows <= 64}, rows of one sequence in order
 void flash_prefill(const AttnParams& P, const StepRows& R, const int* tiles, int ntiles, hipStream_t s);
 bool flash_prefill_supported(const AttnParams& P);
-constexpr int FLASH_TILE_ROWS = 32;
+constexpr int FLASH_TILE_ROWS = 64;
 
 // decode steps (M <= 8 rows that fit LDS): C = layer_norm(x) . W^T in one launch (nb null: the norm is an RMS norm with
 // weight nw, x / sqrt(mean(x^2) + eps) * nw); the normed rows also go to hout
