@@ -35,6 +35,45 @@ __device__ __forceinline__ float ld(const bf16* p) { return bf2f(p->v); }
 __device__ __forceinline__ void st(float* p, float v) { *p = v; }
 __device__ __forceinline__ void st(bf16* p, float v) { p->v = f2bf(v); }
 
+// ------------------------------------------------------------------------------------------------ epilogue
+struct Epi {
+  int mode;
+  float* C;
+  int ldc;
+  float mult;
+  const float* add;
+  float cap;
+};
+__device__ __forceinline__ void epi_store(const Epi& e, int m, int n, float acc) {
+  float* c = e.C + (long long)m * e.ldc + n;
+  if (e.mode == EPI_RESID) {
+    const float extra = e.add ? e.add[(long long)m * e.ldc + n] : 0.f;
+    *c = *c + e.mult * (acc + extra);
+  } else if (e.mode == EPI_SOFTCAP && e.cap != 0.f) {
+    *c = e.cap * tanhf(acc / e.cap);
+  } else if (e.mode == EPI_SCALE) {
+    *c = e.mult * acc;
+  } else {
+    *c = acc;
+  }
+}
+
+// Grouped form of a matrix product (routed experts): a device-side table of row tiles {expert, first row, rows} over rows
+// sorted by expert; a tile's weight matrix is W + expert * w_stride, row m of the tile reads activation row gather[m] / gdiv
+// (or m itself) and writes output row m.
+struct Group {
+  const int* tiles;   // null: a plain product
+  const int* ntiles;
+  const int* gather;
+  int gdiv;
+  long long w_stride;
+};
+// the bfloat16 products of more than 8 rows (stack_gemm.hip)
+void gemm_bf16(const bf16* A, int lda, const bf16* W, int M, int N, int K, const Epi& e, hipStream_t s);
+int gemm_group_tile(int rows, int groups);  // rows per tile of the grouped form
+void gemm_bf16_grouped(const bf16* A, int lda, const bf16* W, int rows, int groups, int max_tiles, int N, int K, const Epi& e, const Group& G,
+                       hipStream_t s);
+
 // butterfly reductions on DPP / permlane exchanges (wave_shuffle.h): no LDS round trip per dependent step
 __device__ __forceinline__ float wave_sum(float v) {
   v += xor_shfl<32>(v);

@@ -1,0 +1,489 @@
+// bfloat16 matrix products of prompt portions and of decode steps with more than 8 rows: C[M][N] = epi(A[M][K] . W[N][K]^T),
+// plain or grouped by expert (Group, stack_device.h). K % 8 == 0 and 16-byte aligned rows (checked by the callers).
+// float32 accumulation in all of them; only the order of the sums differs. Three kernels:
+//   gemm_pingpong_kernel  256 x 256 tiles, two groups of four waves in turns at the LDS and at the matrix cores
+//   gemm_ring_kernel      256 x 128 .. 64 x 64 tiles, loads several steps ahead in registers
+//   gemm_rows_kernel      up to 64 rows: weights straight from memory, K split over a block's waves
+#include <type_traits>
+
+#include "stack_device.h"
+
+namespace omx {
+namespace stack {
+
+namespace {
+
+constexpr int RG_BK = 64;  // K per step: 128-byte operand rows in LDS
+// LDS image of an operand: 16-byte chunk c of row r at chunk c ^ ((r >> 1) & 7) of its 128-byte row. The fragment reads of 16
+// consecutive rows at one chunk land in 16 distinct bank groups, and eight lanes write a whole row.
+
+template <int I, int N, typename F>
+__device__ __forceinline__ void each(const F& f) {  // f(I), .., f(N - 1) with constant arguments
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    each<I + 1, N>(f);
+  }
+}
+
+// the tile of block wg: bands of up to 8 tile rows, rows first: the blocks of an XCD (a contiguous range of wg) form a patch
+// about as wide as it is high, so its L2 fetches the fewest operand tiles
+__device__ __forceinline__ void tile_of(int wg, int mt, int ncol, int& mi, int& ni) {
+  const int band = wg / (8 * ncol), first = 8 * band, rows = min(8, mt - first), i = wg - first * ncol;
+  mi = first + i % rows;
+  ni = i / rows;
+}
+__device__ __forceinline__ int xcd_range(int orig, int nwg) {  // blocks go to the 8 XCDs in turn: give each a contiguous range
+  const int xcd = orig & 7, q8 = nwg >> 3, r8 = nwg & 7;
+  return (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (orig >> 3);
+}
+template <int BM, int BN>
+constexpr int ring_lds() { return 2 * (BM + BN) * RG_BK * 2; }  // two buffers of both operands
+
+// ---- 256 x 256 tiles. Eight waves of 128 x 64 in two groups; a SIMD holds one wave of each. Every step of 64 K is two phases
+// per wave: read 32 K of fragments from LDS, write a share of the next step's operands there and request the step after it;
+// then 16 products. The groups are one phase apart (an extra barrier for the second), so while one is at the LDS the other has
+// the matrix cores to itself: both units are needed for about the same time here (256 KiB through the LDS and 2,048 cycles of
+// products per step and CU), and waves in step use them one after the other. Reads are waited for before the barrier that ends
+// their phase, so no buffer is written while somebody still reads it.
+// Measured against 128 x 128 tiles of four waves with one step of look-ahead: 2,048 x 7,177 x 2,048 139 -> 74 us, 4,096^3
+// 1,139 TFLOP/s (the same tile with all waves in step: 847).
+__global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W, int M,
+                                                               int N, int K, Epi e) {
+  constexpr int BM = 256, BN = 256, WN = 4, TM = 4, TN = 2, L = 4;  // L: 16-byte pieces per thread, step and operand
+  constexpr int AB = BM * RG_BK * 2, BUF = (BM + BN) * RG_BK * 2;   // bytes
+  extern __shared__ __attribute__((aligned(16))) char gemm_smem[];
+  char* sm = gemm_smem;
+  const int ncol = (N + BN - 1) / BN;
+  int mi, ni;
+  tile_of(xcd_range(blockIdx.x, gridDim.x), (M + BM - 1) / BM, ncol, mi, ni);
+  const int m0 = mi * BM, n0 = ni * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = wave >> 2, wm = wave / WN, wn = wave % WN;
+  const int fr = lane & 31, fq = lane >> 5, xr = tid >> 3, xc = tid & 7;
+  unsigned oa[L], ow[L];  // byte offsets of this thread's pieces: row xr + 64 i (rows past the end repeat the last one), chunk xc
+#pragma unroll
+  for (int i = 0; i < L; ++i) {
+    oa[i] = 2u * ((unsigned)min(m0 + xr + 64 * i, M - 1) * (unsigned)lda + 8 * xc);
+    ow[i] = 2u * ((unsigned)min(n0 + xr + 64 * i, N - 1) * (unsigned)K + 8 * xc);
+  }
+  const int n = K / RG_BK;
+  u32x4 ra[L], rw[L];
+  auto load = [&](int step, auto c) {
+    constexpr int C = decltype(c)::value;
+    const int k0 = min(step, n - 1) * RG_BK;  // steps past the end: a repeated load that nobody multiplies
+    if constexpr (C < L) ra[C] = *(const u32x4*)((const char*)A + 2 * k0 + oa[C]);
+    else rw[C - L] = *(const u32x4*)((const char*)W + 2 * k0 + ow[C - L]);
+  };
+  const int wb = xr * 128 + 16 * (xc ^ ((xr >> 1) & 7));
+  auto write = [&](auto c, int buf) {
+    constexpr int C = decltype(c)::value;
+    char* d = sm + buf * BUF + wb;
+    if constexpr (C < L) *(u32x4*)(d + 8192 * C) = ra[C];
+    else *(u32x4*)(d + AB + 8192 * (C - L)) = rw[C - L];
+  };
+  f32x16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  const int sx = 16 * (fq ^ ((fr >> 1) & 7));  // chunk 2 kk + fq of a fragment row: this, with 32 kk flipped in
+  const int fa = (wm * 32 * TM + fr) * 128 + sx, fb = AB + (wn * 32 * TN + fr) * 128 + sx;
+  each<0, 2 * L>([&](auto c) { load(0, c); });
+  each<0, 2 * L>([&](auto c) { write(c, 0); });
+  each<0, 2 * L>([&](auto c) { load(1, c); });
+  __syncthreads();
+  auto bar = [] {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  if (grp) bar();
+  auto step = [&](int s, int buf) {
+    const char* d = sm + buf * BUF;
+    each<0, 2>([&](auto pc) {
+      constexpr int P = decltype(pc)::value;
+      bf16x8 a[2][TM], b[2][TN];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) b[k][j] = *(const bf16x8*)(d + (fb ^ (32 * (2 * P + k))) + 4096 * j);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) a[k][i] = *(const bf16x8*)(d + (fa ^ (32 * (2 * P + k))) + 4096 * i);
+      }
+      each<P * L, (P + 1) * L>([&](auto c) {
+        write(c, buf ^ 1);
+        load(s + 2, c);
+      });
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      bar();
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[k][i], b[k][j], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_sched_barrier(0);
+      bar();
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  int s = 0;
+  for (; s + 2 <= n; s += 2) {
+    step(s, 0);
+    step(s + 1, 1);
+  }
+  if (s < n) step(s, 0);
+  if (!grp) bar();
+  // C fragment: column (weight row) = lane & 31, row (activation row) = (r & 3) + 8 (r >> 2) + 4 (lane >> 5); one epilogue
+  // kind per unrolled body
+  auto out = [&](auto mode) {
+    Epi o = e;
+    o.mode = decltype(mode)::value;
+    each<0, TM * TN>([&](auto fc) {
+      constexpr int F = decltype(fc)::value;
+      const int nn = n0 + wn * 32 * TN + 32 * (F % TN) + fr, mb = m0 + wm * 32 * TM + 32 * (F / TN) + 4 * fq;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int m = mb + (r & 3) + 8 * (r >> 2);
+        if (m < M && nn < N) epi_store(o, m, nn, acc[F / TN][F % TN][r]);
+      }
+    });
+  };
+  switch (e.mode) {
+    case EPI_RESID: out(std::integral_constant<int, EPI_RESID>{}); break;
+    case EPI_SOFTCAP: out(std::integral_constant<int, EPI_SOFTCAP>{}); break;
+    case EPI_SCALE: out(std::integral_constant<int, EPI_SCALE>{}); break;
+    default: out(std::integral_constant<int, EPI_STORE>{}); break;
+  }
+}
+
+// ---- (BM x BN) tiles of WM x WN x KS waves; the KS sets of waves split every step's four 16-wide slices of K between them and
+// add up at the end. Both operands pass registers on their way to a double-buffered LDS image, RD steps deep: a load has RD - 1
+// steps to arrive, and the one barrier a step waits for none. What bounds it: on small grids the chain barrier, LDS write,
+// LDS read, products of a step (0.16 us at 64 x 64, 0.40 at 128 x 128, 0.76 at 256 x 128), on full ones the operands' way from
+// L2 and the Infinity Cache (0.45 / 0.62 / 1.09). Measured, 128 x 128 or 64 x 64 tiles without the ring
+// -> now: 2,048^3 47 -> 27 us, 4,096 x 2,048 x 2,048 61 -> 44, 500 x 2,048 x 2,048 26 -> 12, 128 x 7,177 x 2,048 34 -> 15. TAIL: K is no multiple of 64 (the predicate breaks the loop into pieces that
+// each wait for all loads, so the others go without it).
+template <int BM, int BN, int WM, int WN, int KS, int RD, bool TAIL>
+__global__ __launch_bounds__(64 * WM * WN * KS, BM * BN <= 64 * 64 ? 4 : 2) void gemm_ring_kernel(const bf16* __restrict__ A, int lda,
+                                                                                                 const bf16* __restrict__ W, int M,
+                                                                                                 int N, int K, Epi e, Group G,
+                                                                                                 int mtiles) {
+  constexpr int NT = 64 * WM * WN * KS, XR = NT / 8;
+  static_assert(RD % 2 == 0 && 4 % KS == 0, "LDS buffers alternate inside a trip");
+  constexpr int TM = BM / WM / 32, TN = BN / WN / 32, AL = BM / XR, WL = BN / XR, KK = 4 / KS, FR = TM * TN;
+  constexpr int AS = BM * RG_BK, BUF = (BM + BN) * RG_BK;
+  extern __shared__ __attribute__((aligned(16))) char gemm_smem[];
+  uint16_t* sm = (uint16_t*)gemm_smem;
+  const int ncol = (N + BN - 1) / BN, mt = G.tiles ? *G.ntiles : mtiles;
+  if ((int)blockIdx.x >= mt * ncol) return;
+  int mi, ni;
+  tile_of(xcd_range(blockIdx.x, mt * ncol), mt, ncol, mi, ni);
+  int m0 = mi * BM;
+  const int n0 = ni * BN;
+  if (G.tiles) {
+    const int* t = G.tiles + 3 * mi;
+    W += (long long)t[0] * G.w_stride;
+    m0 = t[1];
+    M = t[1] + t[2];
+  }
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int set = wave / (WM * WN), wm = wave / WN % WM, wn = wave % WN;
+  const int fr = lane & 31, fq = lane >> 5;
+  const int xr = tid >> 3, xc = tid & 7;  // staging: row xr + XR i, 16-byte chunk xc
+  unsigned oa[AL], ow[WL];                // byte offsets
+#pragma unroll
+  for (int i = 0; i < AL; ++i) {  // rows past the end repeat the last one (their results are not stored)
+    const int m = min(m0 + xr + XR * i, M - 1);
+    oa[i] = 2u * ((unsigned)(G.gather ? G.gather[m] / G.gdiv : m) * (unsigned)lda + 8 * xc);
+  }
+#pragma unroll
+  for (int i = 0; i < WL; ++i) ow[i] = 2u * ((unsigned)min(n0 + xr + XR * i, N - 1) * (unsigned)K + 8 * xc);
+  const int n = (K + RG_BK - 1) / RG_BK;
+  u32x4 ra[RD][AL], rw[RD][WL];
+  auto load = [&](int step, u32x4 (&a)[AL], u32x4 (&w)[WL]) {
+    const int k0 = min(step, n - 1) * RG_BK;  // steps past the end: a repeated load that nobody multiplies
+    const char* ca = (const char*)A + 2 * k0;
+    const char* cw = (const char*)W + 2 * k0;
+    const bool in = !TAIL || k0 + 8 * xc < K;
+#pragma unroll
+    for (int i = 0; i < AL; ++i) a[i] = in ? *(const u32x4*)(ca + oa[i]) : u32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < WL; ++i) w[i] = in ? *(const u32x4*)(cw + ow[i]) : u32x4{0, 0, 0, 0};
+  };
+  auto at = [](int r, int c) { return r * RG_BK + 8 * (c ^ ((r >> 1) & 7)); };
+  auto write = [&](const u32x4 (&a)[AL], const u32x4 (&w)[WL], int buf) {
+    uint16_t* d = sm + buf * BUF;
+#pragma unroll
+    for (int i = 0; i < AL; ++i) *(u32x4*)(d + at(xr + XR * i, xc)) = a[i];
+#pragma unroll
+    for (int i = 0; i < WL; ++i) *(u32x4*)(d + AS + at(xr + XR * i, xc)) = w[i];
+  };
+  f32x16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  auto compute = [&](int buf) {
+    const uint16_t* d = sm + buf * BUF;
+    bf16x8 a[2][TM], b[2][TN];
+    auto frags = [&](int k, bf16x8 (&fa)[TM], bf16x8 (&fb)[TN]) {
+      const int c = 2 * (set * KK + k) + fq;
+#pragma unroll
+      for (int j = 0; j < TN; ++j) fb[j] = *(const bf16x8*)(d + AS + at(wn * 32 * TN + 32 * j + fr, c));
+#pragma unroll
+      for (int i = 0; i < TM; ++i) fa[i] = *(const bf16x8*)(d + at(wm * 32 * TM + 32 * i + fr, c));
+    };
+    frags(0, a[0], b[0]);
+#pragma unroll
+    for (int k = 0; k < KK; ++k) {
+      if (k + 1 < KK) frags(k + 1, a[(k + 1) & 1], b[(k + 1) & 1]);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[k & 1][i], b[k & 1][j], acc[i][j], 0, 0, 0);
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < RD; ++u) load(u, ra[u], rw[u]);
+  write(ra[0], rw[0], 0);
+  load(RD, ra[0], rw[0]);
+  // at step s: LDS buffer s & 1 holds it, registers s + 1 .. s + RD the steps after it; behind the barrier the other buffer's
+  // readers are done, the next step goes in and its registers take the step RD later
+  int s = 0;
+  for (; s + RD <= n; s += RD) {
+#pragma unroll
+    for (int u = 0; u < RD; ++u) {
+      __syncthreads();
+      write(ra[(u + 1) % RD], rw[(u + 1) % RD], (u + 1) & 1);
+      load(s + u + 1 + RD, ra[(u + 1) % RD], rw[(u + 1) % RD]);
+      compute(u & 1);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < RD; ++u) {
+    if (s + u < n) {
+      __syncthreads();
+      if (s + u + 1 < n) write(ra[(u + 1) % RD], rw[(u + 1) % RD], (u + 1) & 1);
+      compute(u & 1);
+    }
+  }
+  // the sets' shares meet: set t keeps the fragments with index % KS == t and hands the others over through LDS
+  if constexpr (KS > 1) {
+    float* x = (float*)gemm_smem;
+#pragma unroll
+    for (int f = 0; f < FR; ++f) {
+      __syncthreads();  // the operand images (or the last fragment's shares) are read
+      if (set != f % KS) {
+        float* o = x + ((wave % (WM * WN)) * (KS - 1) + (set + KS - f % KS - 1) % KS) * 1024 + lane;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[64 * r] = acc[f / TN][f % TN][r];
+      }
+      __syncthreads();
+      if (set == f % KS) {
+#pragma unroll
+        for (int t = 0; t < KS - 1; ++t) {
+          const float* o = x + ((wave % (WM * WN)) * (KS - 1) + t) * 1024 + lane;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[f / TN][f % TN][r] += o[64 * r];
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int f = 0; f < FR; ++f) {
+    if (KS > 1 && set != f % KS) continue;
+    const int nn = n0 + wn * 32 * TN + 32 * (f % TN) + fr;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int m = m0 + wm * 32 * TM + 32 * (f / TN) + (r & 3) + 8 * (r >> 2) + 4 * fq;
+      if (m < M && nn < N) epi_store(e, m, nn, acc[f / TN][f % TN][r]);
+    }
+  }
+}
+
+// ---- few rows (up to 16 MT): 16 NT weight rows per block, its 8 waves split K (32 wide slices in turn) and add up through LDS.
+// Operands go from memory straight to the registers: a weight is read by one block only, the activations (up to 64 rows of K)
+// come from L2. What bounds it: the weights' way from memory (the products are idle most of the time), so the split is for as
+// many loads in flight as possible: N / (16 NT) blocks x 8 waves x 4 slices. A 64 x 64 tile walks K alone, a step per memory
+// round trip, on N / 64 blocks. Measured, 64 x 64 tiles -> this: 61 x 1,024 x 1,024 14.1 -> 7.6 us, 61 x 7,177 x 2,048
+// 34 -> 16, 12 x 32,000 x 1,024 22.7 -> 14.0 (four columns of blocks: 29 with one).
+template <int NT, int MT>
+__global__ __launch_bounds__(512) void gemm_rows_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W, int M, int N,
+                                                        int K, Epi e, Group G) {
+  __shared__ float red[8][NT * MT][256];
+  int m0 = 0;
+  if (G.tiles) {
+    if ((int)blockIdx.y >= *G.ntiles) return;
+    const int* t = G.tiles + 3 * blockIdx.y;
+    W += (long long)t[0] * G.w_stride;
+    m0 = t[1];
+    M = t[1] + t[2];
+  }
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n0 = blockIdx.x * 16 * NT, fr = lane & 15, fq = lane >> 4;
+  const int mt = (M - m0 + 15) >> 4;  // row tiles of 16
+  const bf16* pa[MT];
+  const bf16* pw[NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int m = min(m0 + 16 * i + fr, M - 1);
+    pa[i] = A + (long long)(G.gather ? G.gather[m] / G.gdiv : m) * lda + 8 * fq;
+  }
+#pragma unroll
+  for (int j = 0; j < NT; ++j) pw[j] = W + (long long)min(n0 + 16 * j + fr, N - 1) * K + 8 * fq;
+  f32x4 acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int steps = (K + 31) / 32;
+  constexpr int UN = 4;
+  for (int s = wave; s < steps; s += 8 * UN) {
+    u32x4 a[UN][MT], b[UN][NT];
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      const int k = 32 * (s + 8 * u);
+      const bool in = k + 8 * fq < K;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) b[u][j] = in ? *(const u32x4*)(pw[j] + k) : u32x4{0, 0, 0, 0};
+#pragma unroll
+      for (int i = 0; i < MT; ++i) a[u][i] = in && i < mt ? *(const u32x4*)(pa[i] + k) : u32x4{0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int u = 0; u < UN; ++u)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+        if (MT == 1 || i < mt) {
+#pragma unroll
+          for (int j = 0; j < NT; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[u][i]), __builtin_bit_cast(bf16x8, b[u][j]),
+                                                                acc[i][j], 0, 0, 0);
+        }
+  }
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+    if (i < mt) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[wave][i * NT + j][64 * r + lane] = acc[i][j][r];
+    }
+  __syncthreads();
+  for (int x = tid; x < min(mt, MT) * NT * 256; x += 512) {  // element r of lane l: row 4 (l >> 4) + r, column l & 15
+    const int f = x >> 8, r = (x >> 6) & 3, l = x & 63;
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) v += red[w][f][x & 255];
+    const int m = m0 + 16 * (f / NT) + 4 * (l >> 4) + r, nn = n0 + 16 * (f % NT) + (l & 15);
+    if (m < M && nn < N) epi_store(e, m, nn, v);
+  }
+}
+
+struct Operands {
+  const bf16* A;
+  int lda;
+  const bf16* W;
+  int M, N, K;
+};
+template <int BM, int BN, int WM, int WN, int KS, int RD, bool TAIL>
+void launch_ring(const Operands& o, const Epi& e, const Group& G, int mtiles, hipStream_t s) {
+  const unsigned grid = (unsigned)mtiles * ((o.N + BN - 1) / BN);
+  hipLaunchKernelGGL((gemm_ring_kernel<BM, BN, WM, WN, KS, RD, TAIL>), dim3(grid), dim3(64 * WM * WN * KS), (ring_lds<BM, BN>()), s, o.A,
+                     o.lda, o.W, o.M, o.N, o.K, e, G, mtiles);
+}
+template <int NT, int MT>
+void launch_rows(const Operands& o, const Epi& e, const Group& G, int mtiles, hipStream_t s) {
+  hipLaunchKernelGGL((gemm_rows_kernel<NT, MT>), dim3((o.N + 16 * NT - 1) / (16 * NT), mtiles), dim3(512), 0, s, o.A, o.lda, o.W, o.M, o.N,
+                     o.K, e, G);
+}
+void gemm_plain(const Operands& o, const Epi& e, hipStream_t s) {
+  const int M = o.M, N = o.N, n = (o.K + RG_BK - 1) / RG_BK;
+  if (M <= 64) {
+    if (M <= 16) {
+      if (N >= 4096) launch_rows<4, 1>(o, e, Group{}, 1, s);
+      else launch_rows<1, 1>(o, e, Group{}, 1, s);
+    } else if (N <= 4096) {
+      launch_rows<1, 4>(o, e, Group{}, 1, s);
+    } else {
+      launch_rows<2, 4>(o, e, Group{}, 1, s);
+    }
+    return;
+  }
+  if (o.K % RG_BK) {
+    if ((long long)((M + 127) / 128) * ((N + 127) / 128) >= 128) launch_ring<128, 128, 2, 2, 2, 4, true>(o, e, Group{}, (M + 127) / 128, s);
+    else launch_ring<64, 64, 2, 1, 4, 4, true>(o, e, Group{}, (M + 63) / 64, s);
+    return;
+  }
+  // the tile with the least time by a model of measured steps: a launch and its first and last step cost `fixed`, a step of 64
+  // K c0 while few blocks run and c1 on a full chip (us; 14 shapes of 128 .. 4096 rows, within 15 %)
+  struct Tile { int bm, bn, slots; double fixed, c0, c1; };
+  static const Tile tiles[6] = {{256, 256, 256, 12.0, 1.03, 1.95}, {256, 128, 256, 8.0, 0.76, 1.09}, {128, 128, 256, 7.0, 0.40, 0.62},
+                                {128, 128, 512, 7.0, 0.45, 1.25},  {128, 64, 256, 6.3, 0.275, 0.36}, {64, 64, 512, 5.5, 0.16, 0.45}};
+  int best = 0;
+  double least = 0.0;
+  for (int i = 0; i < 6; ++i) {
+    const Tile& t = tiles[i];
+    const double blocks = (double)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    const double waves = (double)(long long)((blocks + t.slots - 1) / t.slots), fill = blocks < t.slots ? blocks / t.slots : 1.0;
+    const double us = t.fixed + waves * n * (t.c0 + (t.c1 - t.c0) * fill);
+    if (i == 0 || us < least) best = i, least = us;
+  }
+  switch (best) {
+    case 0:
+      hipLaunchKernelGGL(gemm_pingpong_kernel, dim3((unsigned)((M + 255) / 256) * ((N + 255) / 256)), dim3(512), (ring_lds<256, 256>()), s,
+                         o.A, o.lda, o.W, M, N, o.K, e);
+      break;
+    case 1: launch_ring<256, 128, 4, 2, 1, 2, false>(o, e, Group{}, (M + 255) / 256, s); break;
+    case 2: launch_ring<128, 128, 2, 2, 2, 4, false>(o, e, Group{}, (M + 127) / 128, s); break;
+    case 3: launch_ring<128, 128, 2, 2, 2, 2, false>(o, e, Group{}, (M + 127) / 128, s); break;
+    case 4: launch_ring<128, 64, 2, 1, 4, 4, false>(o, e, Group{}, (M + 127) / 128, s); break;
+    default: launch_ring<64, 64, 2, 1, 4, 4, false>(o, e, Group{}, (M + 63) / 64, s); break;
+  }
+}
+
+}  // namespace
+
+void gemm_bf16(const bf16* A, int lda, const bf16* W, int M, int N, int K, const Epi& e, hipStream_t s) {
+  // the tile kernels address an operand with 32-bit byte offsets: larger ones go in parts
+  const long long most = (1LL << 31) - 1;  // elements
+  const int mp = (int)(most / lda < M ? most / lda / 256 * 256 : M), np = (int)(most / K < N ? most / K / 256 * 256 : N);
+  check(mp > 0 && np > 0, "gemm: rows of over 2^31 / 256 elements");
+  for (int m = 0; m < M; m += mp)
+    for (int c = 0; c < N; c += np) {
+      Epi p = e;
+      p.C += (long long)m * e.ldc + c;
+      if (p.add) p.add += (long long)m * e.ldc + c;
+      gemm_plain(Operands{A + (long long)m * lda, lda, W + (long long)c * K, M - m < mp ? M - m : mp, N - c < np ? N - c : np, K}, p, s);
+    }
+}
+
+// rows per tile of the grouped form: from the average number of rows per group (expert)
+int gemm_group_tile(int rows, int groups) { return rows / groups >= 192 ? 128 : 64; }
+
+void gemm_bf16_grouped(const bf16* A, int lda, const bf16* W, int rows, int groups, int max_tiles, int N, int K, const Epi& e, const Group& G,
+                       hipStream_t s) {
+  check((long long)rows * lda < (1LL << 31) && (long long)N * K < (1LL << 31), "grouped gemm: operands of over 2^31 elements");
+  const Operands o{A, lda, W, rows, N, K};
+  if (rows / groups < 48) {
+    launch_rows<1, 4>(o, e, G, max_tiles, s);
+  } else if (gemm_group_tile(rows, groups) == 64) {
+    if (K % RG_BK) launch_ring<64, 64, 2, 1, 4, 4, true>(o, e, G, max_tiles, s);
+    else launch_ring<64, 64, 2, 1, 4, 4, false>(o, e, G, max_tiles, s);
+  } else if (K % RG_BK) {
+    launch_ring<128, 128, 2, 2, 2, 4, true>(o, e, G, max_tiles, s);
+  } else {
+    launch_ring<128, 128, 2, 2, 2, 2, false>(o, e, G, max_tiles, s);
+  }
+}
+
+}  // namespace stack
+}  // namespace omx

@@ -14,29 +14,6 @@
 namespace omx {
 namespace stack {
 
-// ------------------------------------------------------------------------------------------------ epilogue
-struct Epi {
-  int mode;
-  float* C;
-  int ldc;
-  float mult;
-  const float* add;
-  float cap;
-};
-__device__ __forceinline__ void epi_store(const Epi& e, int m, int n, float acc) {
-  float* c = e.C + (long long)m * e.ldc + n;
-  if (e.mode == EPI_RESID) {
-    const float extra = e.add ? e.add[(long long)m * e.ldc + n] : 0.f;
-    *c = *c + e.mult * (acc + extra);
-  } else if (e.mode == EPI_SOFTCAP && e.cap != 0.f) {
-    *c = e.cap * tanhf(acc / e.cap);
-  } else if (e.mode == EPI_SCALE) {
-    *c = e.mult * acc;
-  } else {
-    *c = acc;
-  }
-}
-
 // ------------------------------------------------------------------------------------------------ GEMV (M <= 8)
 // one wave per weight row; the row is read once and meets every activation row
 template <typename T>
@@ -413,114 +390,6 @@ __global__ __launch_bounds__(256) void gemm_fma_kernel(const T* __restrict__ A, 
     }
 }
 
-// ------------------------------------------------------------------------------------------------ MFMA tile GEMM
-// bfloat16: (32 TM) x (32 TN) output tile per block of 4 waves (2 x 2), each wave TM x TN fragments of
-// v_mfma_f32_32x32x16_bf16; K in steps of 32 through LDS (rows padded to 40 elements so the 16-byte
-// fragment reads of 32 consecutive rows spread over the banks), the next step's global loads in flight
-// while the current one is multiplied. K % 8 == 0 and 16-byte aligned rows (host-checked).
-constexpr int MF_BK = 32, MF_LD = 40;
-// Grouped form (routed experts): blockIdx.y walks a device-side table of row tiles {expert, first row, rows} over
-// rows sorted by expert; the tile's weight matrix is W + expert * w_stride, row m of the tile reads activation
-// row gather[m] / gdiv (or m itself) and writes output row m.
-struct Group {
-  const int* tiles;   // null: a plain product
-  const int* ntiles;
-  const int* gather;
-  int gdiv;
-  long long w_stride;
-};
-template <int TM, int TN>
-__global__ __launch_bounds__(256) void gemm_mfma_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W,
-                                                        int M, int N, int K, Epi e, Group G) {
-  constexpr int BM = 64 * TM, BN = 64 * TN;
-  __shared__ __attribute__((aligned(16))) uint16_t As[2][BM * MF_LD];
-  __shared__ __attribute__((aligned(16))) uint16_t Ws[2][BN * MF_LD];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  int m0 = blockIdx.y * BM;
-  const int n0 = blockIdx.x * BN;
-  if (G.tiles) {
-    if ((int)blockIdx.y >= *G.ntiles) return;
-    const int* t = G.tiles + 3 * blockIdx.y;
-    W += (long long)t[0] * G.w_stride;
-    m0 = t[1];
-    M = t[1] + t[2];
-  }
-  const int fr = lane & 31, fq = lane >> 5;
-  // staging: 4 threads per row (8 elements each), 64 rows per pass
-  const int sr = tid >> 2, sk = (tid & 3) * 8;
-  long long arow[TM];
-#pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int m = m0 + sr + 64 * i;
-    arow[i] = (G.gather && m < M) ? G.gather[m] / G.gdiv : m;
-  }
-  u32x4 ra[TM], rw[TN];
-  auto fetch = [&](int k0) {
-    const int k = k0 + sk;
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int m = m0 + sr + 64 * i;
-      ra[i] = (m < M && k < K) ? *(const u32x4*)(A + arow[i] * lda + k) : u32x4{0, 0, 0, 0};
-    }
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int n = n0 + sr + 64 * j;
-      rw[j] = (n < N && k < K) ? *(const u32x4*)(W + (long long)n * K + k) : u32x4{0, 0, 0, 0};
-    }
-  };
-  auto stage = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i) *(u32x4*)(&As[buf][(sr + 64 * i) * MF_LD + sk]) = ra[i];
-#pragma unroll
-    for (int j = 0; j < TN; ++j) *(u32x4*)(&Ws[buf][(sr + 64 * j) * MF_LD + sk]) = rw[j];
-  };
-  f32x16 acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-  fetch(0);
-  stage(0);
-  __syncthreads();
-  int buf = 0;
-  for (int k0 = 0; k0 < K; k0 += MF_BK) {
-    const bool more = k0 + MF_BK < K;
-    if (more) fetch(k0 + MF_BK);
-#pragma unroll
-    for (int kk = 0; kk < MF_BK / 16; ++kk) {
-      bf16x8 a[TM], b[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-        a[i] = *(const bf16x8*)(&As[buf][(wm * 32 * TM + 32 * i + fr) * MF_LD + kk * 16 + fq * 8]);
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-        b[j] = *(const bf16x8*)(&Ws[buf][(wn * 32 * TN + 32 * j + fr) * MF_LD + kk * 16 + fq * 8]);
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
-    if (more) stage(buf ^ 1);  // the other buffer's readers finished before the previous barrier
-    __syncthreads();
-    buf ^= 1;
-  }
-  // C fragment: column (weight row) = lane & 31, row (activation row) = (r & 3) + 8 (r >> 2) + 4 (lane >> 5)
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int n = n0 + wn * 32 * TN + 32 * j + fr;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = m0 + wm * 32 * TM + 32 * i + (r & 3) + 8 * (r >> 2) + 4 * fq;
-        if (m < M && n < N) epi_store(e, m, n, acc[i][j][r]);
-      }
-    }
-}
-
 static int g_mfma = 1;
 void set_gemm_mfma(int on) { g_mfma = on; }
 
@@ -547,17 +416,7 @@ void gemm(const GemmParams& P, hipStream_t s) {
                          P.N, P.K, e, v);
     }
   } else if (path == 1) {
-    // 128 x 128 tiles once they still fill the chip, else 64 x 64
-    const long long big = (long long)((P.M + 127) / 128) * ((P.N + 127) / 128);
-    if (big >= 256) {
-      dim3 grid((P.N + 127) / 128, (P.M + 127) / 128);
-      hipLaunchKernelGGL((gemm_mfma_kernel<2, 2>), grid, dim3(256), 0, s, (const bf16*)P.A, P.lda, (const bf16*)P.W, P.M,
-                         P.N, P.K, e, Group{});
-    } else {
-      dim3 grid((P.N + 63) / 64, (P.M + 63) / 64);
-      hipLaunchKernelGGL((gemm_mfma_kernel<1, 1>), grid, dim3(256), 0, s, (const bf16*)P.A, P.lda, (const bf16*)P.W, P.M,
-                         P.N, P.K, e, Group{});
-    }
+    gemm_bf16((const bf16*)P.A, P.lda, (const bf16*)P.W, P.M, P.N, P.K, e, s);
   } else {
     dim3 grid((P.N + 63) / 64, (P.M + 63) / 64);
     if (P.f32)
@@ -1979,7 +1838,7 @@ void moe_grouped(const MoeParams& P, const MoeGroupWs& W, hipStream_t s) {
             (P.Fs == 0 || P.sgate || P.y_add),
         "grouped routed feed-forward: workspace or sizes");
   const int pairs = P.B * P.top, n1 = moe_rows(P.act) * P.F;
-  const int tile_m = pairs / P.X >= 192 ? 128 : 64;
+  const int tile_m = gemm_group_tile(pairs, P.X);
   const int max_tiles = (pairs + tile_m - 1) / tile_m + P.X;
   check(pairs <= W.max_pairs && max_tiles <= W.max_tiles, "grouped routed feed-forward: workspace too small");
   hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(256), 0, s, P.eids, P.ld_top, P.B, P.top, P.X, tile_m, W.rank, W.srow,
@@ -1989,15 +1848,7 @@ void moe_grouped(const MoeParams& P, const MoeGroupWs& W, hipStream_t s) {
   {
     Epi e{EPI_STORE, W.gu, n1, 0.f, nullptr, 0.f};
     Group G{W.tiles, W.ntiles, W.srow, P.top, (long long)n1 * P.E};
-    if (tile_m == 128) {
-      dim3 grid((n1 + 127) / 128, max_tiles);
-      hipLaunchKernelGGL((gemm_mfma_kernel<2, 2>), grid, dim3(256), 0, s, (const bf16*)P.h, P.E, (const bf16*)P.w_gu, pairs,
-                         n1, P.E, e, G);
-    } else {
-      dim3 grid((n1 + 63) / 64, max_tiles);
-      hipLaunchKernelGGL((gemm_mfma_kernel<1, 1>), grid, dim3(256), 0, s, (const bf16*)P.h, P.E, (const bf16*)P.w_gu, pairs,
-                         n1, P.E, e, G);
-    }
+    gemm_bf16_grouped((const bf16*)P.h, P.E, (const bf16*)P.w_gu, pairs, P.X, max_tiles, n1, P.E, e, G, s);
     launched("moe_gemm gate/up");
   }
   {
@@ -2009,15 +1860,7 @@ void moe_grouped(const MoeParams& P, const MoeGroupWs& W, hipStream_t s) {
   {
     Epi e{EPI_STORE, W.ds, P.E, 0.f, nullptr, 0.f};
     Group G{W.tiles, W.ntiles, nullptr, 1, (long long)P.E * P.F};
-    if (tile_m == 128) {
-      dim3 grid((P.E + 127) / 128, max_tiles);
-      hipLaunchKernelGGL((gemm_mfma_kernel<2, 2>), grid, dim3(256), 0, s, (const bf16*)W.hs, P.F, (const bf16*)P.w_down, pairs,
-                         P.E, P.F, e, G);
-    } else {
-      dim3 grid((P.E + 63) / 64, max_tiles);
-      hipLaunchKernelGGL((gemm_mfma_kernel<1, 1>), grid, dim3(256), 0, s, (const bf16*)W.hs, P.F, (const bf16*)P.w_down, pairs,
-                         P.E, P.F, e, G);
-    }
+    gemm_bf16_grouped((const bf16*)W.hs, P.F, (const bf16*)P.w_down, pairs, P.X, max_tiles, P.E, P.F, e, G, s);
     launched("moe_gemm down");
   }
   if (P.Fs > 0) {  // the shared expert's down projection over every row, into y (the stream: added to it)

@@ -2,8 +2,10 @@
 rows x 64 keys per tile) against the float64 implementation in `bizulix_oracle.py`."""
 import numpy as np
 import pytest
+import torch
 
 import bizulix_cases as bc
+from ollama_operator_amd.ops import stack_native
 
 pytestmark = pytest.mark.gpu
 
@@ -29,3 +31,44 @@ def test_flash_prefill_tile_edges(tmp_path, dim, heads, kv, cap):
     out = r.step_entries([(a, toks[40:140], list(range(100))), (b, toks[:70], list(range(70)))]).float().cpu().numpy()
     e = bc.rel_err(out, np.concatenate([want[40:140], want[:70]]))
     assert e.max() < 1e-2, f"two sequences in a step: row {int(e.argmax())} off by {e.max():.3g}"
+
+
+# rows x columns x K: up to 16 / 64 rows (one and several columns per block, K no multiple of 32 x 8 waves); the tiles from
+# 64 x 64 to 256 x 256 with ragged last rows and columns, one step of K, odd step counts, K no multiple of 64
+GEMMS = [(9, 1, 8), (16, 4100, 264), (16, 40, 72), (17, 33, 2048), (64, 4100, 1032), (64, 15, 96), (65, 64, 64), (65, 65, 72),
+         (100, 700, 192), (129, 1024, 704), (300, 3600, 1024), (500, 7177, 2048), (1000, 2048, 2048), (1030, 7177, 2048),
+         (2000, 7177, 2112), (2048, 1030, 200), (4096, 2048, 1088)]
+
+
+@pytest.mark.parametrize("M,N,K", GEMMS)
+def test_gemm_tiles(M, N, K):
+    """Every tile of the bfloat16 products against float64, three epilogues. The operands' products are exact in float32;
+    sums of K of them in any order stay within K 2^-24 of the sum of magnitudes (about K times the operands' mean square)."""
+    C, s = stack_native(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    lda = K + 24  # rows with other columns behind them
+    a = torch.randn(M, lda, device="cuda", generator=g).bfloat16()
+    w = torch.randn(N, K, device="cuda", generator=g).bfloat16()
+    add, res = (torch.randn(M, N, device="cuda", generator=g) for _ in range(2))
+    ref = a[:, :K].double() @ w.double().T
+    lim = 2.0 ** -24 * K * K ** 0.5 + 1e-5
+    p = dict(A=a.data_ptr(), lda=lda, W=w.data_ptr(), M=M, N=N, K=K, ldc=N, f32=0)
+    out = torch.full((M, N), 7.0, device="cuda")
+    C.gemm(dict(p, C=out.data_ptr(), epi=0), s)
+    assert float((out.double() - ref).abs().max()) < lim
+    want = res.double() + 0.5 * (ref + add.double())
+    C.gemm(dict(p, C=res.data_ptr(), epi=1, mult=0.5, add=add.data_ptr()), s)
+    assert float((res.double() - want).abs().max()) < lim
+    C.gemm(dict(p, C=out.data_ptr(), epi=2, cap=5.0), s)
+    assert float((out.double() - 5.0 * torch.tanh(ref / 5.0)).abs().max()) < lim + 1e-5
+
+
+@pytest.mark.parametrize("rows,experts,ff", [(40, 6, 24), (150, 4, 72), (500, 4, 64), (700, 3, 40)])
+def test_grouped_experts(tmp_path, rows, experts, ff):
+    """Routed feed-forwards with few, some and many rows per expert (16-row, 64-row and 128-row tiles; K = ff and K = 64 with
+    and without a remainder of 64) against the float64 implementation."""
+    m = bc.Model(tmp_path, bc.config([(bc.attn(dim=16, vdim=16), bc.moe(experts=experts, top=2, ff=ff, shared_ff=0))], cap=0.0))
+    r = m.runner("cuda", "bfloat16", max_batch=1024, kv_tokens=2048)
+    toks = bc.tokens(rows, 96, seed=rows)
+    want, _ = m.oracle(toks)
+    bc.check(bc.run_cuts(r, toks, [rows]), want, "bfloat16", f"{rows} rows, {experts} experts of {ff}")
