@@ -71,8 +71,8 @@ struct Group {
 // the bfloat16 products of more than 8 rows (stack_gemm.hip)
 void gemm_bf16(const bf16* A, int lda, const bf16* W, int M, int N, int K, const Epi& e, hipStream_t s);
 int gemm_group_tile(int rows, int groups);  // rows per tile of the grouped form
-void gemm_bf16_grouped(const bf16* A, int lda, const bf16* W, int rows, int groups, int max_tiles, int N, int K, const Epi& e, const Group& G,
-                       hipStream_t s);
+void gemm_bf16_grouped(const bf16* A, int lda, const bf16* W, int rows, int groups, int max_tiles, int N, int K, const Epi& e,
+                       const Group& G, hipStream_t s);
 
 // butterfly reductions on DPP / permlane exchanges (wave_shuffle.h): no LDS round trip per dependent step
 __device__ __forceinline__ float wave_sum(float v) {

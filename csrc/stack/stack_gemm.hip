@@ -168,8 +168,9 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(const bf16* __res
 // steps to arrive, and the one barrier a step waits for none. What bounds it: on small grids the chain barrier, LDS write,
 // LDS read, products of a step (0.16 us at 64 x 64, 0.40 at 128 x 128, 0.76 at 256 x 128), on full ones the operands' way from
 // L2 and the Infinity Cache (0.45 / 0.62 / 1.09). Measured, 128 x 128 or 64 x 64 tiles without the ring
-// -> now: 2,048^3 47 -> 27 us, 4,096 x 2,048 x 2,048 61 -> 44, 500 x 2,048 x 2,048 26 -> 12, 128 x 7,177 x 2,048 34 -> 15. TAIL: K is no multiple of 64 (the predicate breaks the loop into pieces that
-// each wait for all loads, so the others go without it).
+// -> now: 2,048^3 47 -> 27 us, 4,096 x 2,048 x 2,048 61 -> 44, 500 x 2,048 x 2,048 26 -> 12, 128 x 7,177 x 2,048 34 -> 15.
+// TAIL: K is no multiple of 64 (the predicate breaks the loop into pieces that each wait for all loads, so the others go
+// without it).
 template <int BM, int BN, int WM, int WN, int KS, int RD, bool TAIL>
 __global__ __launch_bounds__(64 * WM * WN * KS, BM * BN <= 64 * 64 ? 4 : 2) void gemm_ring_kernel(const bf16* __restrict__ A, int lda,
                                                                                                  const bf16* __restrict__ W, int M,
@@ -469,8 +470,8 @@ void gemm_bf16(const bf16* A, int lda, const bf16* W, int M, int N, int K, const
 // rows per tile of the grouped form: from the average number of rows per group (expert)
 int gemm_group_tile(int rows, int groups) { return rows / groups >= 192 ? 128 : 64; }
 
-void gemm_bf16_grouped(const bf16* A, int lda, const bf16* W, int rows, int groups, int max_tiles, int N, int K, const Epi& e, const Group& G,
-                       hipStream_t s) {
+void gemm_bf16_grouped(const bf16* A, int lda, const bf16* W, int rows, int groups, int max_tiles, int N, int K, const Epi& e,
+                       const Group& G, hipStream_t s) {
   check((long long)rows * lda < (1LL << 31) && (long long)N * K < (1LL << 31), "grouped gemm: operands of over 2^31 elements");
   const Operands o{A, lda, W, rows, N, K};
   if (rows / groups < 48) {
