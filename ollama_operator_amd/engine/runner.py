@@ -13,6 +13,7 @@ from __future__ import annotations
 
 import ctypes
 import gc
+import math
 import os
 import time
 import weakref
@@ -27,10 +28,12 @@ from ..ops import native, stream_handle
 from ..ops.reference import TorchExecutor
 from ..utils.trace import trace_range
 from .kv_cache import PagedKV
-from .sampling import SamplingOptions, sample_host
+from .sampling import MASK64, SamplingOptions, sample_host
 from .weights import DeviceWeights, DevQMat, StackWeights
 
 HIST_CAP = 256
+FLOAT_MAX = float(np.finfo(np.float32).max)
+SAMPLER_ROW_WORDS = 12 + HIST_CAP  # a row of sampler state as it is uploaded (csrc/kernels/sampling.hip)
 GEMM_SPLIT_WS_FLOATS = 32 << 20  # 128 MiB of fp32 split-K slabs (2-way split of a 2048 x 8192 output)
 
 
@@ -122,6 +125,32 @@ def kv_cache_type() -> str:
     Ollama's "q8_0", the 8-bit setting) or "f16" (default; "q4_0" falls back to it)."""
     v = (os.environ.get("OMX_KV_CACHE_TYPE") or os.environ.get("OLLAMA_KV_CACHE_TYPE") or "f16").strip().lower()
     return "fp8" if v in ("fp8", "e4m3", "q8_0") else "f16"
+
+
+class PinnedRing:
+    """Pinned host buffers that uploads pass through. `take(words)` hands out the next one (int32 words) once the
+    copies that read it last are done; `sent()` marks the copies issued since. Uploads then neither wait for the
+    stream (as copies from pageable memory do) nor overwrite what a copy still reads. Used by one thread at a time,
+    like the runner that owns it."""
+
+    def __init__(self, words: int, slots: int = 8):
+        self.bufs = [torch.zeros(words, dtype=torch.int32, pin_memory=True) for _ in range(slots)]
+        self.events: list = [None] * slots
+        self.i = 0
+
+    def take(self, words: int) -> torch.Tensor:
+        self.i = (self.i + 1) % len(self.bufs)
+        if self.events[self.i] is not None:
+            self.events[self.i].synchronize()
+            self.events[self.i] = None
+        if words > self.bufs[self.i].numel():
+            self.bufs[self.i] = torch.zeros(words, dtype=torch.int32, pin_memory=True)
+        return self.bufs[self.i]
+
+    def sent(self) -> None:
+        ev = torch.cuda.Event()
+        ev.record()
+        self.events[self.i] = ev
 
 
 @dataclass
@@ -379,10 +408,9 @@ class Runner:
         max_batch = self.max_batch
         self.graphs: dict[int, torch.cuda.CUDAGraph] = {}
         self._host_sampler: dict[int, tuple] = {}
-        self._pinned = None
+        self._ring = None
         if self.is_gpu:
-            self._pinned = [torch.zeros(5, max_batch, dtype=torch.int32).pin_memory() for _ in range(4)]
-            self._pin_i = 0
+            self._ring = PinnedRing(max(6 * max_batch, self.max_blocks, SAMPLER_ROW_WORDS))
             self._tok_host = torch.zeros(max_batch, dtype=torch.int32).pin_memory()
             # sampled tokens of the B == 1 steps, written by the feedback kernel straight into host-mapped
             # pinned memory (slot = input position % ring): no D2H copy command per step
@@ -495,22 +523,47 @@ class Runner:
         B = arr.shape[1]
         self._adv_next = None  # device step inputs no longer follow the last B == 1 decode
         if self.is_gpu:
-            buf = self._pinned[self._pin_i]
-            self._pin_i = (self._pin_i + 1) % len(self._pinned)
-            buf[:, :B] = torch.from_numpy(arr)
-            self.d_step[:5, :B].copy_(buf[:, :B], non_blocking=True)
-            if tokens is not None:
-                self.d_tokens[:len(tokens)].copy_(torch.from_numpy(tokens.astype(np.int32)), non_blocking=False)
+            # one copy: the packed rows up to what is needed of the last one (columns past B are not read)
+            nt, ld = 0 if tokens is None else len(tokens), self.d_step.shape[1]
+            if B:
+                n = 5 * ld + nt if nt else 4 * ld + B
+                buf = self._ring.take(n)
+                w = buf.numpy()
+                w[:n] = 0
+                for i in range(5):
+                    w[i * ld: i * ld + B] = arr[i]
+                w[5 * ld: 5 * ld + nt] = tokens if nt else 0
+                self.d_step.view(-1)[:n].copy_(buf[:n], non_blocking=True)
+                self._ring.sent()
+            elif nt:
+                self._put(self.d_tokens[:nt], tokens)
         else:
             self.d_step[:5, :B] = torch.from_numpy(arr)
             if tokens is not None:
                 self.d_tokens[:len(tokens)] = torch.from_numpy(tokens.astype(np.int32))
 
+    def _put(self, dst: torch.Tensor, src) -> None:
+        """int32 values -> a contiguous device tensor, in stream order and without waiting for the stream."""
+        n = dst.numel()
+        buf = self._ring.take(n)
+        buf.numpy()[:n] = np.asarray(src, np.int32).reshape(-1)
+        dst.view(-1).copy_(buf[:n], non_blocking=True)
+        self._ring.sent()
+
     def _sync_block_table(self, sid: int):
         self._adv_next = None
         s = self.kv.seqs[sid]
-        row = torch.tensor(s.blocks, dtype=torch.int32)
-        self.d_block_table[s.row, :len(s.blocks)].copy_(row.to(self.device))
+        dst = self.d_block_table[s.row, :len(s.blocks)]
+        if self.is_gpu:
+            if s.blocks:
+                self._put(dst, s.blocks)
+        else:
+            dst.copy_(torch.tensor(s.blocks, dtype=torch.int32))
+
+    def _slots(self, sid: int, pos: np.ndarray) -> np.ndarray:
+        """Cache slots of positions of one sequence."""
+        bs = self.block_size
+        return np.asarray(self.kv.seqs[sid].blocks, np.int64)[pos // bs] * bs + pos % bs
 
     # ------------------------------------------------------------------ sequences
     def new_sequence(self) -> int:
@@ -575,7 +628,7 @@ class Runner:
             chunk = tokens[c0:c0 + C]
             B = len(chunk)
             pos = np.arange(start + c0, start + c0 + B, dtype=np.int32)
-            slots = np.array([self.kv.slot(sid, int(p)) for p in pos], np.int32)
+            slots = self._slots(sid, pos)
             last = c0 + B >= n
             arr = np.stack([pos, slots, pos + 1, np.full(B, s.row, np.int32),
                             np.full(B, B - 1, np.int32)]).astype(np.int32)
@@ -608,23 +661,36 @@ class Runner:
 
     # ------------------------------------------------------------------ sampling
     def _set_sampler(self, row: int, o: SamplingOptions, history: list[int], seed: int, step: int = 0):
-        history = [t for t in history if t >= 0]  # external embedding rows (images) are not tokens
-        self.s_temp[row] = o.temperature
-        self.s_topk[row] = o.top_k
-        self.s_topp[row] = o.top_p
-        self.s_minp[row] = o.min_p
-        self.s_rpen[row] = o.repeat_penalty
-        self.s_ppen[row] = o.presence_penalty
-        self.s_fpen[row] = o.frequency_penalty
-        self.s_lastn[row] = o.repeat_last_n
-        self.s_seed[row] = seed - (1 << 64) if seed >= (1 << 63) else seed
-        self.s_step[row] = step  # RNG counter: draws already made for this request
-        h = history[-HIST_CAP:]
-        self.s_hist[row].zero_()
-        if h:
-            self.s_hist[row, :len(h)] = torch.tensor(h, dtype=torch.int32)
-        self.s_hcount[row] = len(h)
-        self._host_sampler[row] = (o, list(history), seed, step)
+        self._set_samplers([(o, history, seed, step)], row)
+
+    def _set_samplers(self, rows: list[tuple], first: int = 0) -> None:
+        """Sampler state of rows first ..: rows[i] = (options, history, seed, draws already made)."""
+        words = SAMPLER_ROW_WORDS
+        for at in range(0, len(rows), 64):
+            part = rows[at:at + 64]
+            n = len(part)
+            w = self._ring.take(n * words).numpy()[:n * words].reshape(n, words) if self.is_gpu else np.zeros((n, words), np.int32)
+            f = w.view(np.float32)
+            for i, (o, history, seed, step) in enumerate(part):
+                history = [t for t in history if t >= 0]  # external embedding rows (images) are not tokens
+                h = history[-HIST_CAP:]
+                reals = (o.temperature, o.top_p, o.min_p, o.repeat_penalty, o.presence_penalty, o.frequency_penalty)
+                if any(math.isfinite(v) and abs(v) > FLOAT_MAX for v in reals):
+                    raise RuntimeError("sampling option out of the range of float32")
+                f[i, 0] = reals[0]
+                f[i, 2:7] = reals[1:]
+                w[i, 1], w[i, 7], w[i, 8], w[i, 9] = o.top_k, o.repeat_last_n, step, len(h)
+                w[i, 10:12] = np.array([seed & MASK64], np.uint64).view(np.int32)
+                w[i, 12:12 + len(h)] = h
+                w[i, 12 + len(h):] = 0
+                self._host_sampler[first + at + i] = (o, list(history), seed, step)
+            if self.is_gpu:  # one launch reads the pinned rows and fills every array
+                self._sampler_module().sampler_rows(
+                    dict(rows=self._ring.bufs[self._ring.i].data_ptr(), n=n, first=first + at, cap=HIST_CAP,
+                         max_rows=self.max_batch, **{k: getattr(self, "s_" + k).data_ptr() for k in (
+                             "temp", "topk", "topp", "minp", "rpen", "ppen", "fpen", "lastn", "step", "hcount", "seed", "hist")}),
+                    stream_handle())
+                self._ring.sent()
 
     def _sample(self, B: int, feedback: bool = False):
         """feedback (GPU): the sampler's finishing lane of each row also feeds the token back and
@@ -904,17 +970,17 @@ class Runner:
                 raise ValueError(f"context overflow: {start + len(tokens)} > {self.ctx}")
             self.kv.reserve(sid, start + len(tokens))
             self._sync_block_table(sid)
-            for i in range(len(tokens)):
-                pos_l.append(start + i)
-                slot_l.append(self.kv.slot(sid, start + i))
-                row_l.append(s.row)
+            pos = np.arange(start, start + len(tokens))
+            pos_l.append(pos)
+            slot_l.append(self._slots(sid, pos))
+            row_l.append(np.full(len(tokens), s.row))
             toks += list(tokens)
             last.append(len(toks) - 1)
         B, n = len(toks), len(items)
-        pos = np.asarray(pos_l, np.int32)
+        pos = np.concatenate(pos_l)
         lidx = np.zeros(B, np.int32)
         lidx[:n] = last
-        arr = np.stack([pos, np.asarray(slot_l, np.int32), pos + 1, np.asarray(row_l, np.int32), lidx])
+        arr = np.stack([pos, np.concatenate(slot_l), pos + 1, np.concatenate(row_l), lidx])
         self._upload(arr.astype(np.int32), self._device_tokens(toks))
         # each admitted prompt is one sequence's contiguous positions: flash (MFMA) attention per segment
         segs, at = [], 0
@@ -931,9 +997,9 @@ class Runner:
                     seg_exe([])
             else:  # torch twin / CPU backend: their attention serves any row -> sequence mapping
                 self.forward(B, n, use_idx=True, prefill=False)
-        for i, (sid, _k, tokens, opts, history, seed, n_s) in enumerate(items):
+        for sid, _k, tokens, _o, _h, _sd, _n in items:
             self.kv.seqs[sid].tokens.extend(tokens)
-            self._set_sampler(i, opts, history, seed, n_s)
+        self._set_samplers([(opts, history, seed, n_s) for _sid, _k, _t, opts, history, seed, n_s in items])
         self._sample(n)
         return [int(t) for t in self.s_out[:n].tolist()]
 
@@ -997,8 +1063,7 @@ class Runner:
 
     def recompose(self, rows: list[tuple], tokens: list[int]) -> None:
         """New batch composition: rows[b] = (opts, history, seed, n_sampled) and the rows' next inputs."""
-        for b, (o, hist, seed, n) in enumerate(rows):
-            self._set_sampler(b, o, hist, seed, n)
+        self._set_samplers(rows)
         self.set_tokens(tokens)
 
     def evict(self, sid: int) -> None:

@@ -24,6 +24,7 @@ from __future__ import annotations
 import os
 import time
 
+import numpy as np
 import torch
 
 from ..models.config import (ACT_CLAMPED_GLU, ACT_GELU_UP, ACT_SILU, BLOCK_POSTNORM, BLOCK_PRENORM, BLOCK_SANDWICH, FF_DENSE,
@@ -178,20 +179,17 @@ class StackExec:
         if rows is None or len(rows[0]) <= 16:
             return
         _pos, qseq = rows
-        B, segs, a = len(qseq), [], 0
-        for i in range(1, B + 1):
-            if i == B or qseq[i] != qseq[a]:
-                segs.append((a, i))
-                a = i
+        cuts = [0, *(np.flatnonzero(np.diff(qseq)) + 1).tolist(), len(qseq)]
+        segs = list(zip(cuts[:-1], cuts[1:]))
         C, T = self.chunk_rows, self.tile_rows
         chunks = [(c0, min(C, i - c0), int(qseq[a]), (1 if c0 == a else 0) | (2 if c0 + C >= i else 0))
                   for a, i in segs for c0 in range(a, i, C)] if r.cfg.has_state else []
         tiles = [(t0, min(T, i - t0)) for a, i in segs for t0 in range(a, i, T)]
         if chunks and len(chunks) <= r.d_chunks.shape[0]:
-            r.d_chunks[:len(chunks)].copy_(torch.tensor(chunks, dtype=torch.int32))
+            r._put(r.d_chunks[:len(chunks)], chunks)
             self.exe.set_chunks(len(chunks))
         if len(tiles) <= r.d_tiles.shape[0]:
-            r.d_tiles[:len(tiles)].copy_(torch.tensor(tiles, dtype=torch.int32))
+            r._put(r.d_tiles[:len(tiles)], tiles)
             self.exe.set_tiles(len(tiles))
 
     def run(self, stage: str, layer: int, B: int, n_logits: int = 0, use_idx: bool = False, prefill: bool = False):
@@ -201,7 +199,7 @@ class StackExec:
             self.bind_chunks(rows)
             # decode attention: blocks per (row, head) by the longest context of the step. A batch-1 step says
             # it itself (`_decode_S`, part of its graph's key); other steps by the rows the host uploaded
-            S = self.r._decode_S or (self.r.decode_splits(max(rows[0]) + 1) if rows is not None else 1)
+            S = self.r._decode_S or (self.r.decode_splits(int(rows[0].max()) + 1) if rows is not None else 1)
             self.exe.set_splits(max(1, S))
         self.exe.step(self.stages[stage], layer, B, n_logits, use_idx, torch.cuda.current_stream().cuda_stream)
 
@@ -378,7 +376,7 @@ class StackRunner(Runner):
     def _upload(self, arr, tokens):
         super()._upload(arr, tokens)
         if arr.shape[1]:
-            self._step_rows = (arr[0].tolist(), arr[3].tolist())
+            self._step_rows = (arr[0].copy(), arr[3].copy())
 
     def split_plan(self, B: int) -> tuple[int, int]:
         return 1, 0
