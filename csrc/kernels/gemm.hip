@@ -599,8 +599,8 @@ static bool gemm_lib(const GemvParams& P, const f16* x16, hipStream_t s) {
 void gemm(const GemvParams& P, hipStream_t s) {
   f16* x16 = (f16*)P.xws;
   // hipBLASLt from gemm_lib_min_m() rows (the GLU matrices unless OMX_GEMM_LIB_GLU=0; always when the
-  // threshold is forced below 128: the test oracle); from 128 rows the stream-order kernel
-  // (gemm_dq.hip), below that the 128 x 128 tile here
+  // threshold is forced below 128: the test oracle); from 65 rows the stream-order kernel
+  // (gemm_dq.hip), below that gemm_rows.hip; the 128 x 128 tile here where they are switched off or short of workspace
   const int lm = lib_min_for(P.w);
   const bool glu = P.epi == EPI_GLU || P.epi == EPI_GEGLU;
   const bool lib = lm > 0 && P.B >= lm && (!glu || lib_glu() || lm < 128);
@@ -613,6 +613,7 @@ void gemm(const GemvParams& P, hipStream_t s) {
   }
   if (dq_gemm(P, s)) return;
   count_launch(LC_GEMM_TILE);
+  if (dq_rows(P, s)) return;
   if (!lib) hipLaunchKernelGGL(prep_x16_kernel, dim3(P.B), dim3(256), 0, s, P, x16);
   switch (P.w.qtype) {
     case QT_Q4_K: launch_gemm<QT_Q4_K>(P, x16, s); break;

@@ -50,8 +50,9 @@ void set_dq_tuning(int cfg, int sk) {
 }
 
 bool dq_gemm(const GemvParams& P, hipStream_t s) {
-  if (!dq_gemm_enabled() || P.B < 128 || !P.xws || P.expert_ids || P.moe_tiles) return false;
+  if (!dq_gemm_enabled() || P.B <= 64 || !P.xws || P.expert_ids || P.moe_tiles) return false;
   const int qt = P.w.qtype;
+  if (qt == QT_F16 && P.B < 128) return false;
   if (qt != QT_Q4_K && qt != QT_Q5_K && qt != QT_Q6_K && qt != QT_Q4_0 && qt != QT_Q8_0 && qt != QT_F16) return false;
   const int Kp = ((P.w.K + 255) >> 8) * 256;
   const long long cap = P.xws_elems ? P.xws_elems : (long long)P.B * P.w.K;

@@ -87,7 +87,8 @@ __host__ __device__ __forceinline__ int piece_off(int t, int sb, int g) {
 // activations: x fp32 [B][ldx] -> (norm) -> fp16 [B][Kp] in storage order; one block per row.
 // Stream position kp: piece P = kp / 32 (t = P / SB, sb = P % SB), slot p = kp % 32: half g = p / 16,
 // byte i = 4 ((p & 15) / 4) + (0, 2, 1, 3)[p & 3] -> natural k = piece_off(t, sb, g) + i
-template <int QT>
+// ROWS (gemm_rows.hip): [16-row tile][32-K piece][8-K run][row], so that a wave reads a run of 16 rows as one block
+template <int QT, bool ROWS = false>
 __global__ __launch_bounds__(256) void prep_xp_kernel(GemvParams P, f16* out, int Kp) {
   // K-quant / Q4_0 / Q8_0 rows: the normalised row is staged in LDS in natural order (coalesced global
   // reads of x and the norm weights), then every thread gathers its 8 stream positions from LDS and
@@ -124,7 +125,7 @@ __global__ __launch_bounds__(256) void prep_xp_kernel(GemvParams P, f16* out, in
       }
     }
   }
-  f16* o = out + (long long)b * Kp;
+  f16* o = ROWS ? out + (long long)(b & ~15) * Kp + 8 * (b & 15) : out + (long long)b * Kp;
   if constexpr (QT == QT_F16) {  // natural order: the weight rows are plain fp16
     for (int c = threadIdx.x; c < Kp / 8; c += 256) {
       f16x8 v;
@@ -180,7 +181,7 @@ __global__ __launch_bounds__(256) void prep_xp_kernel(GemvParams P, f16* out, in
           v[j] = (f16)e;
         }
       }
-      *(f16x8*)(o + kp) = v;
+      *(f16x8*)(o + (ROWS ? 16 * kp : kp)) = v;
     }
   }
 }

@@ -1,0 +1,155 @@
+// Prompt portions of fewer rows than a tile of the prefill GEMM (gemm_dq_impl.h): Y[M][N] = epi(X[M][K] . W[N][K]^T) for
+// M <= 64, W in the resident layout v2, X in storage order (prep_xp_kernel, as for the larger GEMMs).
+//
+// What bounds it: the weights' way from memory; the products need a fifth of that time. So a block takes 16 NT weight rows
+// over all of K, its 8 waves split K, and a weight goes from memory straight to the registers of the one lane that
+// dequantises it: the four lane groups of a wave own one super-block each, lane (n, group) holds a 32-weight piece of row n,
+// and the piece's four runs of 8 weights are the B operands of four v_mfma_f32_16x16x32_f16 per row tile (K runs in an order
+// of its own, the same for the activations, which lane (m, group) finds in 256-byte runs of 16 rows). The next pieces are in
+// flight while one is multiplied. No LDS until the waves' partial sums meet at the end; the epilogue follows in the same launch.
+// (64 x 128 tiles through LDS left two thirds of the chip idle at N = 4096, and split K into slabs with a second launch.)
+// The activations come from L2 once per block, in an order that makes a wave's reads of them whole lines (row by row they cost
+// 16 lines a request and more time than the weights).
+// Measured, Llama-2-7B Q4_K_M at 33 rows, tile kernel + finalize -> this: gate_up 82 -> 43 us, q k v (Q4_K) 49 -> 23, o 34 ->
+// 15, down (Q6_K) 48 -> 23; with 65 rows and more the 128-row tiles of the larger GEMM are ahead (gate_up 93 -> 65 us).
+#include "gemm_dq_impl.h"
+
+namespace omx {
+
+namespace {
+
+template <int QT, int MT, int NT>
+__global__ __launch_bounds__(512, 2) void dq_rows_kernel(GemvParams P, const f16* __restrict__ X, int Kp) {
+  extern __shared__ float red[];  // [8][mt * NT][256]
+  const QMat& w = P.w;
+  const int M = P.B, N = w.N, SB = Kp >> 8;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int fr = lane & 15, g = lane >> 4, n0 = blockIdx.x * 16 * NT;
+  const int mt = (M + 15) >> 4;  // row tiles of 16
+  int row[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) row[j] = min(n0 + 16 * j + fr, N - 1);  // rows past the end repeat the last (not stored)
+  f32x4 acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  // a unit: four super-blocks (one per lane group) x four of their eight pieces; units go to the waves in turn
+  const int units = 2 * ((SB + 3) >> 2), steps = 4 * ((units - wave + 7) >> 3);
+  auto where = [&](int q, int& t, int& sb) {
+    const int u = wave + 8 * (q >> 2);
+    t = 4 * (u & 1) + (q & 3);
+    sb = 4 * (u >> 1) + g;
+  };
+  Piece<QT> pa[NT], pb[NT];
+  u32x4 xa[MT][4], xb[MT][4];
+  auto load = [&](int q, Piece<QT> (&p)[NT], u32x4 (&a)[MT][4]) {
+    int t, sb;
+    where(q, t, sb);
+    const int pc = t * SB + min(sb, SB - 1);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) load_piece<QT>(w, row[j], SB, pc, p[j]);
+    const f16* x = X + 512 * pc + 8 * fr;  // (rows past the end hold anything: not stored)
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+      if (i < mt) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) a[i][k] = *(const u32x4*)(x + i * 16 * Kp + 128 * k);
+      }
+  };
+  auto multiply = [&](int q, const Piece<QT> (&p)[NT], const u32x4 (&a)[MT][4]) {
+    int t, sb;
+    where(q, t, sb);
+    const bool in = sb < SB;  // a lane group past the last super-block multiplies zeros
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      unsigned o[16];
+      dq_piece<QT>(p[j], t, o);
+#pragma unroll
+      for (int k = 0; k < 16; ++k) o[k] = in ? o[k] : 0u;
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+        if (i < mt) {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const u32x4 b = (u32x4){o[4 * k], o[4 * k + 1], o[4 * k + 2], o[4 * k + 3]};
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a[i][k]), __builtin_bit_cast(f16x8, b),
+                                                               acc[i][j], 0, 0, 0);
+          }
+        }
+    }
+  };
+  if (steps > 0) {
+    load(0, pa, xa);
+    for (int q = 0; q < steps; q += 2) {  // steps is a multiple of 4
+      load(q + 1, pb, xb);
+      multiply(q, pa, xa);
+      load(min(q + 2, steps - 1), pa, xa);  // the last one: a repeated load that nobody multiplies
+      multiply(q + 1, pb, xb);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+    if (i < mt) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[(wave * mt * NT + i * NT + j) * 256 + 64 * r + lane] = acc[i][j][r];
+    }
+  __syncthreads();
+  for (int e = tid; e < mt * NT * 256; e += 512) {  // element r of lane l: row 4 (l >> 4) + r, column l & 15
+    const int f = e >> 8, r = (e >> 6) & 3, l = e & 63;
+    float v = 0.f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v += red[k * mt * NT * 256 + e];
+    const float pv = __shfl_xor(v, 1);  // the row pair's partner: the next lane
+    const int m = 16 * (f / NT) + 4 * (l >> 4) + r, n = n0 + 16 * (f % NT) + (l & 15);
+    if (m < M && n < N) epi_apply(P, m, n + P.row_offset, v, pv, 0);
+  }
+}
+
+template <int QT, int MT, int NT>
+void launch_rows(const GemvParams& P, const f16* xp, int Kp, hipStream_t s) {
+  const int mt = (P.B + 15) / 16;
+  hipLaunchKernelGGL((dq_rows_kernel<QT, MT, NT>), dim3((P.w.N + 16 * NT - 1) / (16 * NT)), dim3(512), (size_t)8 * mt * NT * 1024, s, P, xp,
+                     Kp);
+}
+
+template <int QT>
+void run_rows(const GemvParams& P, f16* xp, int Kp, hipStream_t s) {
+  hipLaunchKernelGGL((prep_xp_kernel<QT, true>), dim3(P.B), dim3(256), (size_t)P.w.K * sizeof(float), s, P, xp, Kp);
+  const int N = P.w.N;
+  // columns per block by what still leaves a block for most CUs (Q4_K, 48 rows: N = 22016 43 us at 48 columns, 49 at 64, 47
+  // at 32; 6144 17.9 at 32, 21.5 at 48, 22.8 at 16; 4096 14.7 at 16, 16.9 at 32); at 64 rows three column tiles do not fit
+  // the registers
+  const bool wide = N >= 48 * 208, middle = N >= 32 * 160;
+  if (P.B <= 48) {
+    if (wide) launch_rows<QT, 3, 3>(P, xp, Kp, s);
+    else if (middle) launch_rows<QT, 3, 2>(P, xp, Kp, s);
+    else launch_rows<QT, 3, 1>(P, xp, Kp, s);
+  } else {
+    if (middle) launch_rows<QT, 4, 2>(P, xp, Kp, s);
+    else launch_rows<QT, 4, 1>(P, xp, Kp, s);
+  }
+}
+
+}  // namespace
+
+bool dq_rows(const GemvParams& P, hipStream_t s) {
+  if (!dq_gemm_enabled() || P.B < 2 || P.B > 64 || !P.xws || P.expert_ids || P.moe_tiles || P.w.K % 8) return false;
+  const int Kp = ((P.w.K + 255) >> 8) * 256;
+  const long long cap = P.xws_elems ? P.xws_elems : (long long)P.B * P.w.K;
+  if ((long long)((P.B + 15) & ~15) * Kp > cap) return false;  // whole 16-row tiles
+  f16* xp = (f16*)P.xws;
+  switch (P.w.qtype) {
+    case QT_Q4_K: run_rows<QT_Q4_K>(P, xp, Kp, s); break;
+    case QT_Q5_K: run_rows<QT_Q5_K>(P, xp, Kp, s); break;
+    case QT_Q6_K: run_rows<QT_Q6_K>(P, xp, Kp, s); break;
+    case QT_Q4_0: run_rows<QT_Q4_0>(P, xp, Kp, s); break;
+    case QT_Q8_0: run_rows<QT_Q8_0>(P, xp, Kp, s); break;
+    default: return false;
+  }
+  return true;
+}
+
+}  // namespace omx

@@ -185,8 +185,10 @@ size_t mfma_layout_bytes(int qtype, int N, int K);  // 0 = no layout M for this 
 void repack_m(const QMat& w, void* out, hipStream_t s);
 bool gemm_eligible(const GemvParams& P);
 void gemm(const GemvParams& P, hipStream_t s);
-// stream-order dequant MFMA GEMM (gemm_dq.hip): M >= 128, dense v2 matrices; false = not covered
+// stream-order dequant MFMA GEMM (gemm_dq.hip): M > 64 (fp16 weights: M >= 128), dense v2 matrices; false = not covered
 bool dq_gemm(const GemvParams& P, hipStream_t s);
+// the same for fewer rows (gemm_rows.hip): M <= 64; false = not covered
+bool dq_rows(const GemvParams& P, hipStream_t s);
 bool dq_gemm_enabled();
 void set_dq_gemm(int on);
 void set_dq_ring(int on);  // 1: the register-ring dq kernel (gemm_dq_impl.h), 0: the glds kernel
