@@ -18,6 +18,11 @@ void run_dq_q5k(const GemvParams& P, f16* xp, int Kp, hipStream_t s);  // gemm_d
 void run_dq_q6k(const GemvParams& P, f16* xp, int Kp, hipStream_t s);  // gemm_dq_q6k.hip
 void run_dq_q40(const GemvParams& P, f16* xp, int Kp, hipStream_t s);  // gemm_dq_q40.hip
 void run_dq_q80(const GemvParams& P, f16* xp, int Kp, hipStream_t s);  // gemm_dq_q80.hip
+void run_dq_moe_q4k(const GemvParams& P, f16* xp, int Kp, hipStream_t s);
+void run_dq_moe_q5k(const GemvParams& P, f16* xp, int Kp, hipStream_t s);
+void run_dq_moe_q6k(const GemvParams& P, f16* xp, int Kp, hipStream_t s);
+void run_dq_moe_q40(const GemvParams& P, f16* xp, int Kp, hipStream_t s);
+void run_dq_moe_q80(const GemvParams& P, f16* xp, int Kp, hipStream_t s);
 void run_dq_f16(const GemvParams& P, f16* xp, int Kp, hipStream_t s);  // gemm_dq_f16.hip
 
 bool dq_gemm_enabled() {
@@ -68,6 +73,27 @@ bool dq_gemm(const GemvParams& P, hipStream_t s) {
     default: run_dq_q80(P, xp, Kp, s); break;
   }
   return true;
+}
+
+// Routed experts: gate / up of every (token, expert) pair, then down with the pairs' own output rows in P.y. From a block per
+// CU on: below that (tiny experts) too few of the chip's CUs walk K, and the callers keep the per-expert path.
+bool dq_moe_covered(const GemvParams& P) {
+  const int qt = P.w.qtype, Kp = ((P.w.K + 255) >> 8) * 256;
+  return dq_gemm_enabled() && P.xws && P.moe_tiles && P.moe_rows && (long long)P.B * Kp <= P.xws_elems && P.w.K % 4 == 0 &&
+         (qt == QT_Q4_K || qt == QT_Q5_K || qt == QT_Q6_K || qt == QT_Q4_0 || qt == QT_Q8_0) &&
+         (P.epi == EPI_GLU || P.epi == EPI_GEGLU || P.epi == EPI_STORE);
+}
+void dq_moe(const GemvParams& P, hipStream_t s) {
+  const int Kp = ((P.w.K + 255) >> 8) * 256;
+  f16* xp = (f16*)P.xws;
+  count_launch(LC_DQ_GEMM);
+  switch (P.w.qtype) {
+    case QT_Q4_K: run_dq_moe_q4k(P, xp, Kp, s); break;
+    case QT_Q5_K: run_dq_moe_q5k(P, xp, Kp, s); break;
+    case QT_Q6_K: run_dq_moe_q6k(P, xp, Kp, s); break;
+    case QT_Q4_0: run_dq_moe_q40(P, xp, Kp, s); break;
+    default: run_dq_moe_q80(P, xp, Kp, s); break;
+  }
 }
 
 }  // namespace omx

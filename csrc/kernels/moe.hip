@@ -280,4 +280,20 @@ void moe_sort(const int* eids, int n_pairs, int X, int* rows, int* tiles, int* n
                      tile_m);
 }
 
+// A token's routed pairs, weighted and summed in routing order (the sum does not depend on which expert finished first).
+// E % 4 == 0 (dq_moe_covered). Bound by its bytes: k + 2 rows of E floats per token.
+__global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restrict__ ds, const float* __restrict__ ew, int k, int E,
+                                                          float* __restrict__ y, int ldy) {
+  const int t = blockIdx.y, n = 4 * (blockIdx.x * 256 + threadIdx.x);
+  if (n >= E) return;
+  f32x4* out = (f32x4*)(y + (long long)t * ldy + n);
+  f32x4 v = *out;
+  for (int j = 0; j < k; ++j) v += ew[t * k + j] * *(const f32x4*)(ds + ((long long)t * k + j) * E + n);
+  *out = v;
+}
+void moe_combine(const float* ds, const float* ew, int B, int k, int E, float* y, int ldy, hipStream_t s) {
+  if (B <= 0) return;
+  hipLaunchKernelGGL(moe_combine_kernel, dim3((E + 1023) / 1024, B), dim3(256), 0, s, ds, ew, k, E, y, ldy);
+}
+
 }  // namespace omx

@@ -189,6 +189,9 @@ void gemm(const GemvParams& P, hipStream_t s);
 bool dq_gemm(const GemvParams& P, hipStream_t s);
 // the same for fewer rows (gemm_rows.hip): M <= 64; false = not covered
 bool dq_rows(const GemvParams& P, hipStream_t s);
+// routed experts in one launch per matrix (P.moe_* set; gemm_dq.hip); dq_moe only where dq_moe_covered
+bool dq_moe_covered(const GemvParams& P);
+void dq_moe(const GemvParams& P, hipStream_t s);
 bool dq_gemm_enabled();
 void set_dq_gemm(int on);
 void set_dq_ring(int on);  // 1: the register-ring dq kernel (gemm_dq_impl.h), 0: the glds kernel
@@ -302,6 +305,8 @@ void moe_route(const float* logits, int B, int X, int k, int* ids, float* w, hip
 // fused RMSNorm + router logits + top-k softmax (P.w = router [X <= 64][K], P.x = resid, P.norm_w)
 bool moe_router(const GemvParams& P, int k, int* ids, float* w, hipStream_t s);  // false: shape not covered
 void gather_rows(const float* x, int ld, const int* idx, int rows, int n, float* out, hipStream_t s);
+// y[t][n] += sum_j ew[t k + j] * ds[t k + j][n], in routing order (moe.hip)
+void moe_combine(const float* ds, const float* ew, int B, int k, int E, float* y, int ldy, hipStream_t s);
 void moe_sort(const int* eids, int n_pairs, int X, int* rows, int* tiles, int* n_tiles, int tile_m, hipStream_t s);
 // grouped dequant GEMM over expert-homogeneous row tiles (P.moe_* set; P.B = number of pairs)
 void moe_gemm(const GemvParams& P, hipStream_t s);

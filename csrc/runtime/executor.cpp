@@ -423,6 +423,22 @@ void Executor::ffn_block(int i, const StepInputs& in, hipStream_t s) {
       G.ldy = F;
       grouped(G);
       G.moe_gather = 1;
+      GemvParams Dn = base_params(L.down_exps, pairs, ws.hbuf, F, ws);
+      Dn.ldy = E;
+      grouped(Dn);
+      Dn.moe_scatter = 1;
+      // all experts in one launch per matrix (gemm_dq.hip) where their tiles fill the chip; outputs of the down projection
+      // per pair, summed per token afterwards
+      Dn.epi = EPI_STORE;
+      Dn.y = ws.yws;
+      const long long blocks = (long long)((pairs + MOE_TILE_M - 1) / MOE_TILE_M) * ((G.w.N + 255) / 256);
+      if (blocks >= 256 && ws.yws && (long long)pairs * E <= ws.yws_elems && dq_moe_covered(G) && dq_moe_covered(Dn)) {
+        dq_moe(G, s);
+        dq_moe(Dn, s);
+        if (cfg.tp > 1) hipMemsetAsync(dst, 0, sizeof(float) * (size_t)B * E, s);
+        moe_combine(ws.yws, ws.ew, B, k, E, dst, E, s);
+        return;
+      }
       // long prompts: per-expert hipBLASLt GEMMs (gemm.hip moe_gemm_lib) need the routed counts on the
       // host -- one small D2H copy + sync per layer (prefill is never graph-captured)
       std::vector<int> counts;
@@ -441,14 +457,10 @@ void Executor::ffn_block(int i, const StepInputs& in, hipStream_t s) {
       const bool lib = !counts.empty() && moe_gemm_lib(G, counts.data(), X, s);
       if (!lib) moe_gemm(G, s);
       if (cfg.tp > 1) hipMemsetAsync(dst, 0, sizeof(float) * (size_t)B * E, s);
-      GemvParams Dn = base_params(L.down_exps, pairs, ws.hbuf, F, ws);
       Dn.epi = EPI_ADD;  // routing-weighted, atomically accumulated per token
       Dn.y = dst;
-      Dn.ldy = E;
       Dn.expert_ids = ws.eids;
       Dn.expert_w = ws.ew;
-      grouped(Dn);
-      Dn.moe_scatter = 1;
       if (!(lib && moe_gemm_lib(Dn, counts.data(), X, s))) moe_gemm(Dn, s);
       return;
     }

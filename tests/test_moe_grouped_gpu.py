@@ -1,0 +1,48 @@
+"""Routed experts of a prompt in one launch per matrix (csrc/kernels/gemm_dq_impl.h, grouped): every weight type, both tile
+widths, tiles that end inside an expert's rows."""
+import numpy as np
+import pytest
+import torch
+
+from ollama_operator_amd.engine.runner import Runner
+from ollama_operator_amd.gguf.constants import FileType
+from ollama_operator_amd.models.config import preset
+from ollama_operator_amd.models.random_init import write_random_gguf
+from ollama_operator_amd.ops import native
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("ft,n_ff,rows,arch", [
+    (FileType.MOSTLY_Q4_K_M, 8192, 260, "llama"), (FileType.MOSTLY_Q4_K_M, 3840, 577, "llama"), (FileType.MOSTLY_Q5_K_S, 8192, 257, "llama"),
+    (FileType.MOSTLY_Q4_0, 8192, 321, "llama"), (FileType.MOSTLY_Q8_0, 3840, 640, "llama"), (FileType.MOSTLY_Q6_K, 8192, 300, "llama")])
+def test_grouped_experts(tmp_path, ft, n_ff, rows, arch):
+    """Against float32 on the CPU, beside the path that is taken with these kernels switched off: both round the same two
+    operands to fp16 and add in float32, so neither may be further from float32 than the other by more than the order of sums
+    and the atomics' order explain (a fifth)."""
+    path = str(tmp_path / "m.gguf")
+    write_random_gguf(path, preset("tiny-mixtral", n_embd=512, n_ff=n_ff, n_layer=1, n_head=8, ctx_len=768), ft, seed=int(ft))
+    rng = np.random.default_rng(rows)
+    toks = [1] + [int(x) for x in rng.integers(3, 500, rows - 1)]
+    C = native()
+
+    def logits(device):
+        r = Runner(path, device=device, max_batch=640, max_seqs=2, ctx=704)
+        C.reset_launch_counts()
+        r.prefill(r.new_sequence(), toks)
+        out = r.logits[0, :r.cfg.n_vocab].double().cpu()
+        n = C.launch_counts() if device == "cuda" else None
+        r.close()
+        return out, n
+
+    want, _ = logits("cpu")
+    on = C.dq_gemm_enabled()
+    C.set_dq_gemm(1)
+    got, n = logits("cuda")
+    C.set_dq_gemm(0)
+    old, m = logits("cuda")
+    C.set_dq_gemm(int(on))
+    assert n["dq_gemm"] >= 4 and n["gemm_tile"] == 0 and m["dq_gemm"] == 0, (n, m)  # q|k|v, o, gate|up, down
+    err = lambda v: float((v - want).norm() / want.norm())  # noqa: E731
+    print(err(got), err(old))
+    assert err(got) < 1.2 * err(old) + 1e-4
