@@ -464,10 +464,17 @@ __global__ __launch_bounds__(ATT_NT) void attn_decode_kernel(AttnParams P) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Causal prefill attention on the matrix cores: one sequence, NQ >= 16
-// contiguous query positions (a prefill chunk), K/V already in the paged cache (the QKV epilogue
-// wrote them). Block = 4 waves x 32 queries of one head; key tiles of 32 staged in LDS and shared
-// by the waves. Per tile and wave:
+// Causal prefill attention on the matrix cores: one sequence, NQ >= 16 contiguous query positions (a
+// prefill chunk), K/V already in the paged cache (the QKV epilogue wrote them). A block of 4 waves
+// takes 64 queries of one head and walks the keys in tiles of 64, double-buffered in LDS with the next
+// tile on its way in registers; waves 0 and 1 take the first 32 keys of a tile for the lower and the
+// upper 32 queries, waves 2 and 3 the other 32, and the two halves meet through LDS at the end. So a
+// block's chain is half as many tiles as with 128 queries (one wave per 32, all keys), there are twice
+// as many blocks (577 rows x 16 heads: 160 instead of 80 on 256 CUs), and a tile costs one barrier.
+// What bounds it: the softmax VALU work beside the products, two waves per SIMD sharing the two units.
+// Measured against blocks of 128 queries, a wave per 32 and single-buffered tiles of 32 keys: 2,048 rows x 32
+// heads of 128 107.7 -> 79.1 us, 509 rows 30.9 -> 18.9, 577 rows x 16 heads of 64, every key visible, 22.8 -> 13.8.
+// Per tile and wave:
 //   S^T = K . Q^T   (v_mfma_f32_32x32x16_f16; keys on the accumulator rows, one query per lane, so
 //                    the online softmax is lane-local + one exchange with lane ^ 32)
 //   O^T += V^T . P^T (P^T used straight from the accumulator registers as the B operand in the
@@ -477,7 +484,7 @@ __global__ __launch_bounds__(ATT_NT) void attn_decode_kernel(AttnParams P) {
 //                    reads are bank-conflict-free)
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16a __attribute__((ext_vector_type(16)));
-constexpr int PF_BQ = 128, PF_BK = 32;
+constexpr int PF_BQ = 64, PF_BK = 64;  // queries of a block, keys of a tile
 
 // T10 (b): byte offset of 16-B chunk ch of V row `row`; rows of VROW bytes (256, or 512 for D = 256:
 // each 256-B half swizzled on its own)
@@ -486,37 +493,48 @@ __device__ __forceinline__ int vswz(int row, int ch) {
   return VROW * row + 256 * (ch >> 4) + 16 * ((ch & 15) ^ (((row & 3) << 2) | ((row >> 2) & 3)));
 }
 
+template <int D>
+struct PfLds {
+  static constexpr int NDT = (D + 31) / 32;                   // 32-row d tiles of O^T
+  static constexpr int LDK = D + 8;                           // K tile row stride (f16): 16-B rows offset by 4 banks
+  static constexpr int VROW = D > 128 ? 2 * D : 256;
+  static constexpr int KB = PF_BK * LDK * 2, BUF = KB + PF_BK * VROW;
+  static constexpr int MERGE = 2 * (16 * NDT + 2) * 64 * 4;   // the second key halves' outputs, maxima and sums
+  static constexpr int TILES = 2 * BUF > MERGE ? 2 * BUF : MERGE;
+  static constexpr int ALL = TILES + 2 * PF_BK * 4;           // + the cache rows of two tiles' keys
+};
+
 template <int D, bool KV8 = false>
-__global__ __launch_bounds__(256) void attn_prefill_kernel(AttnParams P) {
+__global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void attn_prefill_kernel(AttnParams P) {
+  typedef PfLds<D> L;
   constexpr int NKS = D / 16;             // k-steps of S^T over the head dim
-  constexpr int NDT = (D + 31) / 32;      // 32-row d tiles of O^T
-  constexpr int LDK = D + 8;              // K tile row stride (f16): 16-B rows offset by 4 banks
+  constexpr int NDT = L::NDT, LDK = L::LDK, VROW = L::VROW;
   constexpr int KCH = D / 8;              // 16-B chunks per K/V row
-  constexpr int VROW = D > 128 ? 2 * D : 256;
-  __shared__ __attribute__((aligned(16))) f16 Ks[PF_BK * LDK];
-  __shared__ __attribute__((aligned(16))) char Vs[PF_BK * VROW];  // [key][VROW B] swizzled, zero-padded
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, h2 = lane >> 5, qc = lane & 31;
-  const int head = blockIdx.y, G = P.H / P.n_kv, kvh = head / G;
-  // causal load balance: block b and b + 256 share a CU in the first dispatch wave (2 blocks per CU), and
-  // consecutive heads hold the same query-block index, so the CUs that drew the last query blocks got twice
-  // the heaviest work. The upper half of the heads walks the query blocks in reverse: every CU pairs a
-  // heavy block with a light one.
-  const int qb = blockIdx.y >= gridDim.y / 2 ? (int)(gridDim.x - 1 - blockIdx.x) : (int)blockIdx.x;
-  const int q0 = qb * PF_BQ;
+  extern __shared__ __attribute__((aligned(16))) char pf_smem[];  // 2 x { K tile, V tile [key][VROW B] swizzled, zero-padded }, rows
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, h2 = lane >> 5, qc = lane & 31;
+  const int qw = wave & 1, set = wave >> 1;
+  // late queries see the most keys: tiles go from the last to the first; where all blocks run at once (two per CU, 256
+  // apart), the second half from the first up, so that a CU has a long block beside a short one
+  const int ntiles = (P.NQ + PF_BQ - 1) / PF_BQ, rank = blockIdx.x / P.H, half = (ntiles + 1) / 2;
+  const int tile = rank < half || ntiles * P.H > 512 ? ntiles - 1 - rank : rank - half;
+  const int head = blockIdx.x % P.H, G = P.H / P.n_kv, kvh = head / G;
+  const int q0 = tile * PF_BQ;
   const int NQ = P.NQ;
-  const int qi = min(q0 + wave * 32 + qc, NQ - 1);  // this lane's query (clamped; stores masked)
-  const int len_q = P.q_len[qi];                    // visible keys = pos + 1
+  const int qo = q0 + 32 * qw + qc, qi = min(qo, NQ - 1);  // this lane's query (clamped; stores masked)
+  const int len_q = P.q_len[qi];                           // visible keys = pos + 1
   const int kstart_q = P.window > 0 ? max(0, len_q - P.window) : 0;
   const int seq = P.q_seq ? P.q_seq[0] : 0;
   const int* bt = P.block_table + (long long)seq * P.max_blocks;
   const f16* kc = (const f16*)P.kc;
   const f16* vc = (const f16*)P.vc;
   const int bs = P.bs;
-  // key range of the block: contiguous positions -> first query has the smallest window start,
-  // the last query the largest length
-  const int q_last = min(q0 + PF_BQ, NQ) - 1;
-  const int len_max = P.q_len[q_last];
-  const int k_lo = P.window > 0 ? max(0, P.q_len[q0] - P.window) / PF_BK * PF_BK : 0;
+  // key ranges of the block and of this wave (none: a wave past the last query): contiguous positions -> the
+  // first query has the smallest window start, the last query the largest length
+  const int len_max = P.q_len[min(q0 + PF_BQ, NQ) - 1];
+  const int k_lo = P.window > 0 ? max(0, P.q_len[q0] - P.window) / 32 * 32 : 0;
+  const int wq = q0 + 32 * qw;
+  const int w_max = wq < NQ ? P.q_len[min(wq + 32, NQ) - 1] : 0;
+  const int w_lo = P.window > 0 && wq < NQ ? max(0, P.q_len[wq] - P.window) : 0;
 
   // Q^T fragments (B operand of S^T): lane = query, 8 consecutive d per k-step, scaled by scale * log2(e):
   // the scores come out in the log2 domain, so the softmax takes v_exp_f32 directly (no multiply per score)
@@ -544,21 +562,27 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnParams P) {
 
   // zero the V padding columns once (d in [D, 128)): they feed the last O^T tile when D % 32 != 0
   if (D < 128) {
-    for (int i = tid; i < PF_BK * 16; i += 256) {
-      const int row = i >> 4, ch = i & 15;
-      if (ch >= KCH) *(u32x4*)(Vs + vswz<VROW>(row, ch)) = (u32x4){0u, 0u, 0u, 0u};
+    for (int i = tid; i < 2 * PF_BK * 16; i += 256) {
+      const int row = (i >> 4) & (PF_BK - 1), ch = i & 15;
+      if (ch >= KCH) *(u32x4*)(pf_smem + (i / (PF_BK * 16)) * L::BUF + L::KB + vswz<VROW>(row, ch)) = (u32x4){0u, 0u, 0u, 0u};
     }
   }
-  // staging: each thread moves chunks of the K and V tiles (global paged cache -> registers -> LDS)
+  // staging: each thread moves chunks of the K and V tiles (global paged cache -> registers -> LDS). One thread
+  // per key looks its cache row up two tiles ahead; keys past the end repeat the last one (masked)
   constexpr int NCH = (PF_BK * KCH + 255) / 256;
   u32x4 kr[NCH], vr[NCH];
-  auto issue = [&](int kt0) {
+  int* rows = (int*)(pf_smem + L::TILES);
+  int nkey = 0, nblk = 0;
+  auto find = [&](int kt0) {
+    nkey = min(kt0 + lane, len_max - 1);
+    nblk = bt[nkey / bs];
+  };
+  auto note = [&](int b) { rows[PF_BK * b + lane] = (nblk * P.n_kv + kvh) * bs + nkey % bs; };
+  auto issue = [&](int b) {
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
-      const int i = tid + 256 * c;
-      const int row = min(i / KCH, PF_BK - 1), ch = i % KCH;
-      const int t = min(kt0 + row, len_max - 1);
-      const long long base = (((long long)bt[t / bs] * P.n_kv + kvh) * bs + (t % bs)) * D + 8 * ch;
+      const int i = min(tid + 256 * c, PF_BK * KCH - 1);
+      const long long base = (long long)rows[PF_BK * b + i / KCH] * D + 8 * (i % KCH);
       if constexpr (KV8) {  // 8 fp8 bytes in .x / .y, widened at the LDS write
         const u32x2 k8 = *(const u32x2*)((const uint8_t*)P.kc + base), v8 = *(const u32x2*)((const uint8_t*)P.vc + base);
         kr[c] = (u32x4){k8.x, k8.y, 0u, 0u};
@@ -579,27 +603,40 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnParams P) {
     for (int j = 0; j < 8; ++j) h[j] = t[j];
     return __builtin_bit_cast(u32x4, h);
   };
-  issue(k_lo);
-  for (int kt0 = k_lo; kt0 < len_max; kt0 += PF_BK) {
-    __syncthreads();  // previous tile's LDS reads done
+  if (wave == 0) {
+    find(k_lo);
+    note(0);
+    find(k_lo + PF_BK);
+  }
+  __syncthreads();
+  issue(0);
+  int buf = 0;
+  for (int t0 = k_lo; t0 < len_max; t0 += PF_BK, buf ^= 1) {
+    f16* Ks = (f16*)(pf_smem + buf * L::BUF);
+    char* Vs = pf_smem + buf * L::BUF + L::KB;
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
       const int i = tid + 256 * c;
-      if (i < PF_BK * KCH) {
+      if (PF_BK * KCH % 256 == 0 || i < PF_BK * KCH) {
         const int row = i / KCH, ch = i % KCH;
         *(u32x4*)(Ks + row * LDK + 8 * ch) = widen(kr[c]);
         *(u32x4*)(Vs + vswz<VROW>(row, ch)) = widen(vr[c]);
       }
     }
+    if (wave == 0) note(buf ^ 1);
+    // one barrier a tile: this buffer's readers of two tiles ago passed the last barrier after they were done
     __syncthreads();
-    if (kt0 + PF_BK < len_max) issue(kt0 + PF_BK);  // next tile in flight during the MFMAs
+    if (wave == 0) find(t0 + 2 * PF_BK);
+    if (t0 + PF_BK < len_max) issue(buf ^ 1);  // next tile in flight during the MFMAs
+    const int kt0 = t0 + 32 * set;             // this wave's half
+    if (kt0 >= w_max || kt0 + 32 <= w_lo) continue;
     // S^T = K . Q^T : rows = keys kt0 + (r&3) + 8(r>>2) + 4*h2, column = this lane's query
     f32x16a sacc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) sacc[r] = 0.f;
 #pragma unroll
     for (int kk = 0; kk < NKS; ++kk) {
-      const f16x8 kf = *(const f16x8*)(Ks + qc * LDK + 16 * kk + 8 * h2);
+      const f16x8 kf = *(const f16x8*)(Ks + (32 * set + qc) * LDK + 16 * kk + 8 * h2);
       sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[kk], sacc, 0, 0, 0);
     }
     // causal / window / length mask + online softmax (per lane = per query; halves exchange). The VALU
@@ -607,7 +644,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnParams P) {
     // inside every query's window of this wave skip the mask, and the accumulator rescale is skipped
     // when no query's running max moved
     float tmax = -INFINITY;
-    if (__all(kt0 + PF_BK <= len_q && kt0 >= kstart_q)) {
+    if (__all(kt0 + 32 <= len_q && kt0 >= kstart_q)) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, sacc[r]);
     } else {
@@ -647,7 +684,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnParams P) {
 #pragma unroll
       for (int i = 0; i < NDT; ++i) {
         const int c0 = (32 * i + 16 * (g & 1)) / 8;  // first 16-B chunk of this group's 16 d columns
-        const int r0 = 16 * s2 + 4 * h2;             // element j < 4: keys r0 + 0..3; j >= 4: + 8
+        const int r0 = 32 * set + 16 * s2 + 4 * h2;  // element j < 4: keys r0 + 0..3; j >= 4: + 8
         const int a0 = vswz<VROW>(r0 + qq, c0 + (pp >> 1)) + 8 * (pp & 1);
         const int a1 = vswz<VROW>(r0 + 8 + qq, c0 + (pp >> 1)) + 8 * (pp & 1);
         typedef __attribute__((address_space(3))) s16x4 lds_s4;
@@ -660,9 +697,23 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnParams P) {
       }
     }
   }
+  // the second key halves' share joins the first's (the tiles' buffers are free once everybody is here)
+  __syncthreads();
+  float* mg = (float*)pf_smem + qw * (16 * NDT + 2) * 64 + lane;
+  if (set == 1) {
+    mg[0] = m;
+    mg[64] = l;
+#pragma unroll
+    for (int i = 0; i < NDT; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mg[64 * (2 + 16 * i + r)] = o[i][r];
+  }
+  __syncthreads();
   // O = O^T / l : lane = query, rows = d (r&3) + 8(r>>2) + 4*h2 of d tile i
-  const int qo = q0 + wave * 32 + qc;
-  if (qo < NQ) {
+  if (set == 0 && qo < NQ) {
+    const float m1 = mg[0], mn = fmaxf(m, m1);
+    const float c0 = mn == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn), c1 = mn == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - mn);
+    l = l * c0 + mg[64] * c1;
     const float inv = l > 0.f ? 1.f / l : 0.f;
     float* out = P.out + (long long)qo * P.ldo + head * Dv;
 #pragma unroll
@@ -670,9 +721,10 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnParams P) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const int d = 32 * i + 8 * k + 4 * h2;
-        if (d < Dv)
-          *(f32x4*)(out + d) = (f32x4){o[i][4 * k] * inv, o[i][4 * k + 1] * inv, o[i][4 * k + 2] * inv,
-                                       o[i][4 * k + 3] * inv};
+        f32x4 v;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = (o[i][4 * k + j] * c0 + mg[64 * (2 + 16 * i + 4 * k + j)] * c1) * inv;
+        if (d < Dv) *(f32x4*)(out + d) = v;
       }
   }
 }
@@ -714,8 +766,8 @@ static void launch_d(const AttnParams& P, hipStream_t s) {
 }
 template <int D>
 static void launch_pf(const AttnParams& P, dim3 grid, hipStream_t s) {
-  if (P.kv8) hipLaunchKernelGGL((attn_prefill_kernel<D, true>), grid, dim3(256), 0, s, P);
-  else hipLaunchKernelGGL((attn_prefill_kernel<D, false>), grid, dim3(256), 0, s, P);
+  if (P.kv8) hipLaunchKernelGGL((attn_prefill_kernel<D, true>), grid, dim3(256), (PfLds<D>::ALL), s, P);
+  else hipLaunchKernelGGL((attn_prefill_kernel<D, false>), grid, dim3(256), (PfLds<D>::ALL), s, P);
 }
 
 void attention_decode(const AttnParams& P0, hipStream_t s) {
@@ -723,7 +775,7 @@ void attention_decode(const AttnParams& P0, hipStream_t s) {
   AttnParams P = P0;
   if (P.kps <= 0) P.kps = g_attn_kps;
   if (P.prefill && P.NQ >= 16 && P.D % 16 == 0) {  // one sequence, contiguous positions: MFMA flash
-    dim3 grid((P.NQ + PF_BQ - 1) / PF_BQ, P.H);
+    dim3 grid((P.NQ + PF_BQ - 1) / PF_BQ * P.H);
     count_launch(LC_ATTN_PREFILL);
     switch (P.D) {
       case 64: launch_pf<64>(P, grid, s); return;
