@@ -23,7 +23,7 @@ void run_dq_moe_q5k(const GemvParams& P, f16* xp, int Kp, hipStream_t s);
 void run_dq_moe_q6k(const GemvParams& P, f16* xp, int Kp, hipStream_t s);
 void run_dq_moe_q40(const GemvParams& P, f16* xp, int Kp, hipStream_t s);
 void run_dq_moe_q80(const GemvParams& P, f16* xp, int Kp, hipStream_t s);
-void run_dq_f16(const GemvParams& P, f16* xp, int Kp, hipStream_t s);  // gemm_dq_f16.hip
+void run_dq_f16(const GemvParams& P, f16* xp, int Kp, hipStream_t s);  // gemm_f16.hip: tiles of its own
 
 bool dq_gemm_enabled() {
   if (g_dq_enable < 0) {

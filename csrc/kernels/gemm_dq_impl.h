@@ -77,7 +77,6 @@ __device__ __forceinline__ unsigned dsel(const u32x4& v, int i) { return i == 0 
 // weight offsets (natural K) of the lo / hi 16-weight halves of piece t of super-block sb
 template <int QT>
 __host__ __device__ __forceinline__ int piece_off(int t, int sb, int g) {
-  static_assert(QT != QT_F16, "F16 rows are in natural order (prep_xp copies them straight)");
   if constexpr (QT == QT_Q4_K || QT == QT_Q5_K) return 256 * sb + 64 * (t >> 1) + 16 * (t & 1) + 32 * g;
   else if constexpr (QT == QT_Q6_K) return 256 * sb + 128 * (t >> 2) + 16 * (t & 3) + 64 * g;
   else return 256 * sb + 32 * t + 16 * g;  // Q4_0 / Q8_0
@@ -94,95 +93,72 @@ __global__ __launch_bounds__(256) void prep_xp_kernel(GemvParams P, f16* out, in
   // reads of x and the norm weights), then every thread gathers its 8 stream positions from LDS and
   // writes them as one 16-B store. Gathering straight from global memory made every x read a scattered
   // 4-B load: 36 us per call at 2048 rows, 10 % of the 2048-token TTFT (profiles/r5_gemm prefill trace)
-  extern __shared__ float xs[];  // [Kp] (quantized rows; F16 rows do not use it)
+  extern __shared__ float xs[];  // [Kp]
   __shared__ float red[4];
   const int b = blockIdx.x, K = P.w.K, SB = Kp >> 8;
   const float* x = P.x + (long long)(P.moe_gather ? P.moe_rows[b] / P.n_sel : b) * P.ldx;  // routed pairs: their token's row
   float mean = 0.f, rstd = 1.f;
-  constexpr bool STAGE = QT != QT_F16;
-  if (P.norm != NORM_NONE || STAGE) {
-    float s = 0.f, ss = 0.f;
-    for (int i = threadIdx.x; i < K / 4; i += 256) {
-      const f32x4 v = *(const f32x4*)(x + 4 * i);
-      if constexpr (STAGE) *(f32x4*)(xs + 4 * i) = v;
-      s += v.x + v.y + v.z + v.w;
-      ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
-    }
-    for (int k = (K & ~3) + threadIdx.x; k < K; k += 256) {  // K % 4 tail
-      const float v = x[k];
-      if constexpr (STAGE) xs[k] = v;
-      s += v;
-      ss += v * v;
-    }
-    if (P.norm != NORM_NONE) {
-      ss = block_sum<256>(ss, red);
-      if (P.norm == NORM_LAYER) {
-        s = block_sum<256>(s, red);
-        mean = s / K;
-        rstd = rsqrtf(fmaxf(ss / K - mean * mean, 0.f) + P.eps);
-      } else {
-        rstd = rsqrtf(ss / K + P.eps);
-      }
+  float s = 0.f, ss = 0.f;
+  for (int i = threadIdx.x; i < K / 4; i += 256) {
+    const f32x4 v = *(const f32x4*)(x + 4 * i);
+    *(f32x4*)(xs + 4 * i) = v;
+    s += v.x + v.y + v.z + v.w;
+    ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+  }
+  for (int k = (K & ~3) + threadIdx.x; k < K; k += 256) {  // K % 4 tail
+    const float v = x[k];
+    xs[k] = v;
+    s += v;
+    ss += v * v;
+  }
+  if (P.norm != NORM_NONE) {
+    ss = block_sum<256>(ss, red);
+    if (P.norm == NORM_LAYER) {
+      s = block_sum<256>(s, red);
+      mean = s / K;
+      rstd = rsqrtf(fmaxf(ss / K - mean * mean, 0.f) + P.eps);
+    } else {
+      rstd = rsqrtf(ss / K + P.eps);
     }
   }
   f16* o = ROWS ? out + (long long)(b & ~15) * Kp + 8 * (b & 15) : out + (long long)b * Kp;
-  if constexpr (QT == QT_F16) {  // natural order: the weight rows are plain fp16
-    for (int c = threadIdx.x; c < Kp / 8; c += 256) {
-      f16x8 v;
+  // a 16-B output chunk is 8 CONSECUTIVE natural positions base .. base + 7 in the order
+  // 0 2 1 3 4 6 5 7: two 16-B LDS reads (+ two of the norm weights), permuted in registers
+  __syncthreads();  // the staged row (and block_sum's broadcast) are visible
+  const bool nrm = P.norm != NORM_NONE, lnb = P.norm == NORM_LAYER && P.norm_b;
+  for (int c = threadIdx.x; c < Kp / 8; c += 256) {
+    const int kp = 8 * c, pc = kp >> 5, p0 = kp & 31;
+    const int t = pc / SB, sb = pc - t * SB;
+    const int base = piece_off<QT>(t, sb, p0 >> 4) + 4 * ((p0 & 15) >> 2);
+    f16x8 v;
+    if (base + 8 <= K) {
+      f32x4 a = *(const f32x4*)(xs + base), b = *(const f32x4*)(xs + base + 4);
+      if (nrm) {
+        const f32x4 wa = *(const f32x4*)(P.norm_w + base), wb = *(const f32x4*)(P.norm_w + base + 4);
+        a = (a - mean) * rstd * wa;
+        b = (b - mean) * rstd * wb;
+        if (lnb) {
+          a += *(const f32x4*)(P.norm_b + base);
+          b += *(const f32x4*)(P.norm_b + base + 4);
+        }
+      }
+      v = (f16x8){(f16)a.x, (f16)a.z, (f16)a.y, (f16)a.w, (f16)b.x, (f16)b.z, (f16)b.y, (f16)b.w};
+    } else {  // the row's K padding (Q4_0 / Q8_0 with K % 256 != 0)
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const int k = 8 * c + j;
+        const int r = j & 3, k = base + 4 * (j >> 2) + (r == 1 ? 2 : r == 2 ? 1 : r);
         float e = 0.f;
         if (k < K) {
-          e = x[k];
-          if (P.norm != NORM_NONE) {
+          e = xs[k];
+          if (nrm) {
             e = (e - mean) * rstd * P.norm_w[k];
-            if (P.norm == NORM_LAYER && P.norm_b) e += P.norm_b[k];
+            if (lnb) e += P.norm_b[k];
           }
         }
         v[j] = (f16)e;
       }
-      *(f16x8*)(o + 8 * c) = v;
     }
-  } else {
-    // a 16-B output chunk is 8 CONSECUTIVE natural positions base .. base + 7 in the order
-    // 0 2 1 3 4 6 5 7: two 16-B LDS reads (+ two of the norm weights), permuted in registers
-    __syncthreads();  // the staged row (and block_sum's broadcast) are visible
-    const bool nrm = P.norm != NORM_NONE, lnb = P.norm == NORM_LAYER && P.norm_b;
-    for (int c = threadIdx.x; c < Kp / 8; c += 256) {
-      const int kp = 8 * c, pc = kp >> 5, p0 = kp & 31;
-      const int t = pc / SB, sb = pc - t * SB;
-      const int base = piece_off<QT>(t, sb, p0 >> 4) + 4 * ((p0 & 15) >> 2);
-      f16x8 v;
-      if (base + 8 <= K) {
-        f32x4 a = *(const f32x4*)(xs + base), b = *(const f32x4*)(xs + base + 4);
-        if (nrm) {
-          const f32x4 wa = *(const f32x4*)(P.norm_w + base), wb = *(const f32x4*)(P.norm_w + base + 4);
-          a = (a - mean) * rstd * wa;
-          b = (b - mean) * rstd * wb;
-          if (lnb) {
-            a += *(const f32x4*)(P.norm_b + base);
-            b += *(const f32x4*)(P.norm_b + base + 4);
-          }
-        }
-        v = (f16x8){(f16)a.x, (f16)a.z, (f16)a.y, (f16)a.w, (f16)b.x, (f16)b.z, (f16)b.y, (f16)b.w};
-      } else {  // the row's K padding (Q4_0 / Q8_0 with K % 256 != 0)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int r = j & 3, k = base + 4 * (j >> 2) + (r == 1 ? 2 : r == 2 ? 1 : r);
-          float e = 0.f;
-          if (k < K) {
-            e = xs[k];
-            if (nrm) {
-              e = (e - mean) * rstd * P.norm_w[k];
-              if (lnb) e += P.norm_b[k];
-            }
-          }
-          v[j] = (f16)e;
-        }
-      }
-      *(f16x8*)(o + (ROWS ? 16 * kp : kp)) = v;
-    }
+    *(f16x8*)(o + (ROWS ? 16 * kp : kp)) = v;
   }
 }
 
@@ -195,19 +171,10 @@ struct Piece {
   u32x4 m;                                   // Q4_K / Q5_K meta (d, dmin, scales12); Q6_K int8 scales
   u32x2 h;                                   // Q6_K high-bit pairs
   unsigned e;                                // Q5_K 5th bits; Q6_K / Q4_0 / Q8_0: fp16 d (low half)
-  u32x4 f[QT == QT_F16 ? 2 : 1];             // F16: halves 16..31 of the piece
 };
 
 template <int QT>
 __device__ __forceinline__ void load_piece(const QMat& w, long long row, int SB, int pc, Piece<QT>& R) {
-  if constexpr (QT == QT_F16) {  // natural order: piece pc = halves 32 pc .. + 31 of the row
-    const uint8_t* q = w.s0 + row * SB * 512 + 64LL * pc;
-    R.a = *(const u32x4*)q;
-    R.b = *(const u32x4*)(q + 16);
-    R.f[0] = *(const u32x4*)(q + 32);
-    R.f[1] = *(const u32x4*)(q + 48);
-    return;
-  }
   const int t = pc / SB, sb = pc - t * SB;
   if constexpr (QT == QT_Q8_0) {
     const uint8_t* q = w.s0 + row * SB * 256 + 32LL * pc;
@@ -241,11 +208,7 @@ __device__ __forceinline__ void k_scale(const u32x4& m, int j, float& sc, float&
 // dequantise a piece to 32 fp16 in stream order: o[0..7] = lo half pairs, o[8..15] = hi half pairs
 template <int QT>
 __device__ __forceinline__ void dq_piece(const Piece<QT>& R, int t, unsigned (&o)[16]) {
-  if constexpr (QT == QT_F16) {
-    const u32x4 v[4] = {R.a, R.b, R.f[0], R.f[1]};
-#pragma unroll
-    for (int i = 0; i < 16; ++i) o[i] = dsel(v[i >> 2], i & 3);
-  } else if constexpr (QT == QT_Q4_K || QT == QT_Q5_K) {
+  if constexpr (QT == QT_Q4_K || QT == QT_Q5_K) {
     const int c = t >> 1;
     float s0, c0, s1, c1;
     k_scale(R.m, 2 * c, s0, c0);
@@ -700,8 +663,7 @@ void launch_dq(const GemvParams& P, const f16* xp, int Kp, int sk, hipStream_t s
 
 template <int QT>
 void run_dq(const GemvParams& P, f16* xp, int Kp, hipStream_t s) {
-  hipLaunchKernelGGL(prep_xp_kernel<QT>, dim3(P.B), dim3(256), QT == QT_F16 ? 0 : (size_t)P.w.K * sizeof(float), s, P, xp,
-                     Kp);
+  hipLaunchKernelGGL(prep_xp_kernel<QT>, dim3(P.B), dim3(256), (size_t)P.w.K * sizeof(float), s, P, xp, Kp);
   const int M = P.B, N = P.w.N, nks = Kp / DQ_BK;
   // tile x split-K from a wave model calibrated on MI355X (scripts/bench_dq_sweep.py, profiles/r4_gemm):
   // time = waves * (K steps per split) * c[cfg] + split-K slab traffic, waves = ceil(units / slots);

@@ -8,6 +8,7 @@
 #include <stdexcept>
 #include <string>
 
+#include "../kernels/gemm_ring.h"
 #include "../kernels/wave_shuffle.h"
 #include "stack_ops.h"
 
@@ -58,16 +59,7 @@ __device__ __forceinline__ void epi_store(const Epi& e, int m, int n, float acc)
   }
 }
 
-// Grouped form of a matrix product (routed experts): a device-side table of row tiles {expert, first row, rows} over rows
-// sorted by expert; a tile's weight matrix is W + expert * w_stride, row m of the tile reads activation row gather[m] / gdiv
-// (or m itself) and writes output row m.
-struct Group {
-  const int* tiles;   // null: a plain product
-  const int* ntiles;
-  const int* gather;
-  int gdiv;
-  long long w_stride;
-};
+using ring::Group;  // grouped form of a matrix product (routed experts)
 // the bfloat16 products of more than 8 rows (stack_gemm.hip)
 void gemm_bf16(const bf16* A, int lda, const bf16* W, int M, int N, int K, const Epi& e, hipStream_t s);
 int gemm_group_tile(int rows, int groups);  // rows per tile of the grouped form
