@@ -72,3 +72,19 @@ def test_grouped_experts(tmp_path, rows, experts, ff):
     toks = bc.tokens(rows, 96, seed=rows)
     want, _ = m.oracle(toks)
     bc.check(bc.run_cuts(r, toks, [rows]), want, "bfloat16", f"{rows} rows, {experts} experts of {ff}")
+
+
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (72, 44), (96, 96), (128, 128), (40, 120), (64, 200), (24, 30)])
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+def test_decode_attention(tmp_path, dim, vdim, dtype):
+    """Single rows over 1 .. 300 keys, where the groups of 64 keys and the rounds of four waves end: values requested ahead of
+    the scores (16-bit, up to 128 dims), value rows no multiple of a piece, wide ones. Limits as for the prompts; in
+    float32 the oracle's (2^-24 per operation, some hundred of them in a row)."""
+    m = bc.Model(tmp_path, bc.config([(bc.attn(heads=2, kv_heads=1, dim=dim, vdim=vdim, scale=dim ** -0.5), None)], cap=0.0))
+    r = m.runner("cuda", dtype, max_batch=512, kv_tokens=2048)
+    toks = bc.tokens(300, 96, seed=dim + vdim)
+    want, _ = m.oracle(toks)
+    for n in (1, 2, 63, 64, 65, 128, 129, 255, 256, 257, 300):
+        got = bc.run_cuts(r, toks[:n], [n] if n == 1 else [n - 1, n])
+        e = bc.rel_err(got[-1:], want[n - 1:n])
+        assert e.max() < (1e-2 if dtype == "bfloat16" else 1e-4), f"{n} keys: off by {e.max():.3g}"
