@@ -82,6 +82,17 @@ __host__ __device__ __forceinline__ int piece_off(int t, int sb, int g) {
   else return 256 * sb + 32 * t + 16 * g;  // Q4_0 / Q8_0
 }
 
+// LDS place of element k of a staged row: the 16-B slot index xor bits of the super-block (and, where a piece's
+// halves are 64 apart, of that bit), so that the four chunks of four neighbouring pieces, slots {0, 2, 8, 10}
+// (Q4_K / Q5_K, Q6_K) or {0, 2, 4, 6} (Q4_0 / Q8_0) of as many super-blocks, cover all 16 slots of the banks
+template <int QT>
+__host__ __device__ __forceinline__ int prep_at(int k) {
+  const int sb = k >> 8, hi = QT == QT_Q4_0 || QT == QT_Q8_0 ? 8 : 4;
+  int m = (sb & 1) | ((sb & 2) ? hi : 0);
+  if (QT == QT_Q6_K) m ^= (k >> 3) & 8;
+  return k ^ (4 * m);
+}
+
 // ------------------------------------------------------------------------------------------------
 // activations: x fp32 [B][ldx] -> (norm) -> fp16 [B][Kp] in storage order; one block per row.
 // Stream position kp: piece P = kp / 32 (t = P / SB, sb = P % SB), slot p = kp % 32: half g = p / 16,
@@ -89,29 +100,33 @@ __host__ __device__ __forceinline__ int piece_off(int t, int sb, int g) {
 // ROWS (gemm_rows.hip): [16-row tile][32-K piece][8-K run][row], so that a wave reads a run of 16 rows as one block
 template <int QT, bool ROWS = false>
 __global__ __launch_bounds__(256) void prep_xp_kernel(GemvParams P, f16* out, int Kp) {
-  // K-quant / Q4_0 / Q8_0 rows: the normalised row is staged in LDS in natural order (coalesced global
-  // reads of x and the norm weights), then every thread gathers its 8 stream positions from LDS and
-  // writes them as one 16-B store. Gathering straight from global memory made every x read a scattered
-  // 4-B load: 36 us per call at 2048 rows, 10 % of the 2048-token TTFT (profiles/r5_gemm prefill trace)
+  // The row is staged in LDS in natural order (coalesced reads of x), normed there in place (coalesced reads of the
+  // weights), then every thread gathers its 8 stream positions and writes them as one 16-B store. Neighbouring
+  // chunks of the stream are whole super-blocks apart, the same banks: prep_at() swaps 16-B slots inside each
+  // super-block so that the gathers of 16 lanes take 16 different ones. What bounds it: its bytes, 6 per element.
+  // Measured against gathers that met in the banks (four or eight at a time) and applied the norm's weights from
+  // memory in stream order: 2,048 rows of 4,096 20.6 -> 15.1 us, of 11,008 31.4 -> 23.2; 500 tokens' 1,000 pairs of
+  // 14,336 66 -> 48.
   extern __shared__ float xs[];  // [Kp]
   __shared__ float red[4];
   const int b = blockIdx.x, K = P.w.K, SB = Kp >> 8;
   const float* x = P.x + (long long)(P.moe_gather ? P.moe_rows[b] / P.n_sel : b) * P.ldx;  // routed pairs: their token's row
-  float mean = 0.f, rstd = 1.f;
+  const bool nrm = P.norm != NORM_NONE, lnb = P.norm == NORM_LAYER && P.norm_b;
   float s = 0.f, ss = 0.f;
   for (int i = threadIdx.x; i < K / 4; i += 256) {
     const f32x4 v = *(const f32x4*)(x + 4 * i);
-    *(f32x4*)(xs + 4 * i) = v;
+    *(f32x4*)(xs + prep_at<QT>(4 * i)) = v;
     s += v.x + v.y + v.z + v.w;
     ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
   }
   for (int k = (K & ~3) + threadIdx.x; k < K; k += 256) {  // K % 4 tail
     const float v = x[k];
-    xs[k] = v;
+    xs[prep_at<QT>(k)] = v;
     s += v;
     ss += v * v;
   }
-  if (P.norm != NORM_NONE) {
+  if (nrm) {
+    float mean = 0.f, rstd;
     ss = block_sum<256>(ss, red);
     if (P.norm == NORM_LAYER) {
       s = block_sum<256>(s, red);
@@ -120,42 +135,35 @@ __global__ __launch_bounds__(256) void prep_xp_kernel(GemvParams P, f16* out, in
     } else {
       rstd = rsqrtf(ss / K + P.eps);
     }
+    for (int i = threadIdx.x; i < K / 4; i += 256) {  // each thread its own elements
+      f32x4* p = (f32x4*)(xs + prep_at<QT>(4 * i));
+      f32x4 v = (*p - mean) * rstd * *(const f32x4*)(P.norm_w + 4 * i);
+      if (lnb) v += *(const f32x4*)(P.norm_b + 4 * i);
+      *p = v;
+    }
+    for (int k = (K & ~3) + threadIdx.x; k < K; k += 256) {
+      float v = (xs[prep_at<QT>(k)] - mean) * rstd * P.norm_w[k];
+      if (lnb) v += P.norm_b[k];
+      xs[prep_at<QT>(k)] = v;
+    }
   }
   f16* o = ROWS ? out + (long long)(b & ~15) * Kp + 8 * (b & 15) : out + (long long)b * Kp;
+  __syncthreads();
   // a 16-B output chunk is 8 CONSECUTIVE natural positions base .. base + 7 in the order
-  // 0 2 1 3 4 6 5 7: two 16-B LDS reads (+ two of the norm weights), permuted in registers
-  __syncthreads();  // the staged row (and block_sum's broadcast) are visible
-  const bool nrm = P.norm != NORM_NONE, lnb = P.norm == NORM_LAYER && P.norm_b;
+  // 0 2 1 3 4 6 5 7: two 16-B LDS reads, permuted in registers
   for (int c = threadIdx.x; c < Kp / 8; c += 256) {
     const int kp = 8 * c, pc = kp >> 5, p0 = kp & 31;
     const int t = pc / SB, sb = pc - t * SB;
     const int base = piece_off<QT>(t, sb, p0 >> 4) + 4 * ((p0 & 15) >> 2);
     f16x8 v;
     if (base + 8 <= K) {
-      f32x4 a = *(const f32x4*)(xs + base), b = *(const f32x4*)(xs + base + 4);
-      if (nrm) {
-        const f32x4 wa = *(const f32x4*)(P.norm_w + base), wb = *(const f32x4*)(P.norm_w + base + 4);
-        a = (a - mean) * rstd * wa;
-        b = (b - mean) * rstd * wb;
-        if (lnb) {
-          a += *(const f32x4*)(P.norm_b + base);
-          b += *(const f32x4*)(P.norm_b + base + 4);
-        }
-      }
+      const f32x4 a = *(const f32x4*)(xs + prep_at<QT>(base)), b = *(const f32x4*)(xs + prep_at<QT>(base + 4));
       v = (f16x8){(f16)a.x, (f16)a.z, (f16)a.y, (f16)a.w, (f16)b.x, (f16)b.z, (f16)b.y, (f16)b.w};
     } else {  // the row's K padding (Q4_0 / Q8_0 with K % 256 != 0)
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         const int r = j & 3, k = base + 4 * (j >> 2) + (r == 1 ? 2 : r == 2 ? 1 : r);
-        float e = 0.f;
-        if (k < K) {
-          e = xs[k];
-          if (nrm) {
-            e = (e - mean) * rstd * P.norm_w[k];
-            if (lnb) e += P.norm_b[k];
-          }
-        }
-        v[j] = (f16)e;
+        v[j] = (f16)(k < K ? xs[prep_at<QT>(k)] : 0.f);
       }
     }
     *(f16x8*)(o + (ROWS ? 16 * kp : kp)) = v;
@@ -663,7 +671,7 @@ void launch_dq(const GemvParams& P, const f16* xp, int Kp, int sk, hipStream_t s
 
 template <int QT>
 void run_dq(const GemvParams& P, f16* xp, int Kp, hipStream_t s) {
-  hipLaunchKernelGGL(prep_xp_kernel<QT>, dim3(P.B), dim3(256), (size_t)P.w.K * sizeof(float), s, P, xp, Kp);
+  hipLaunchKernelGGL(prep_xp_kernel<QT>, dim3(P.B), dim3(256), (size_t)Kp * sizeof(float), s, P, xp, Kp);
   const int M = P.B, N = P.w.N, nks = Kp / DQ_BK;
   // tile x split-K from a wave model calibrated on MI355X (scripts/bench_dq_sweep.py, profiles/r4_gemm):
   // time = waves * (K steps per split) * c[cfg] + split-K slab traffic, waves = ceil(units / slots);
@@ -703,7 +711,7 @@ void launch_dq_moe(const GemvParams& P, const f16* xp, int Kp, hipStream_t s) {
 }
 template <int QT>
 void run_dq_moe(const GemvParams& P, f16* xp, int Kp, hipStream_t s) {
-  hipLaunchKernelGGL(prep_xp_kernel<QT>, dim3(P.B), dim3(256), (size_t)P.w.K * sizeof(float), s, P, xp, Kp);
+  hipLaunchKernelGGL(prep_xp_kernel<QT>, dim3(P.B), dim3(256), (size_t)Kp * sizeof(float), s, P, xp, Kp);
   // wide matrices in 256 columns a tile; narrow ones in 128, two blocks per CU, which leave a shorter last wave
   if (P.w.N >= 8192) launch_dq_moe<QT, 256>(P, xp, Kp, s);
   else launch_dq_moe<QT, 128>(P, xp, Kp, s);

@@ -117,7 +117,7 @@ void launch_rows(const GemvParams& P, const f16* xp, int Kp, hipStream_t s) {
 
 template <int QT>
 void run_rows(const GemvParams& P, f16* xp, int Kp, hipStream_t s) {
-  hipLaunchKernelGGL((prep_xp_kernel<QT, true>), dim3(P.B), dim3(256), (size_t)P.w.K * sizeof(float), s, P, xp, Kp);
+  hipLaunchKernelGGL((prep_xp_kernel<QT, true>), dim3(P.B), dim3(256), (size_t)Kp * sizeof(float), s, P, xp, Kp);
   const int N = P.w.N;
   // columns per block by what still leaves a block for most CUs (Q4_K, 48 rows: N = 22016 43 us at 48 columns, 49 at 64, 47
   // at 32; 6144 17.9 at 32, 21.5 at 48, 22.8 at 16; 4096 14.7 at 16, 16.9 at 32); at 64 rows three column tiles do not fit

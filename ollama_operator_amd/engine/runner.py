@@ -200,7 +200,8 @@ class Runner:
         # weight copy exists -- OMX_GEMM_LIB_MIN_M=<rows> is the A/B knob)
         self.lib_min = native().gemm_lib_min_m() if self.is_gpu else 0
         # MoE prefill: (token, expert) pairs from which each expert's GEMM runs on hipBLASLt over its
-        # per-call dequantised weights (gemm.hip moe_gemm_lib; default 256, OMX_MOE_LIB_MIN_M)
+        # per-call dequantised weights (gemm.hip moe_gemm_lib; default 256, OMX_MOE_LIB_MIN_M) where the grouped
+        # launches' tiles do not fill the chip (gemm_dq.hip dq_moe)
         self.moe_lib = native().moe_lib_min_m() if self.is_gpu and self.w.cfg.n_expert else 0
         cfg = self.cfg = self.w.cfg
         loc = self.w.local

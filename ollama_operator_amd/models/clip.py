@@ -222,9 +222,9 @@ def unpad_grid(t: torch.Tensor, size: tuple[int, int]) -> torch.Tensor:
 
 
 class _NativeTower:
-    """The CLIP tower on the engine's own kernels (GPU): every projection is the stream-order MFMA GEMM
-    (csrc/kernels/gemm_dq.hip) on fp16 weight rows (QT_F16, K zero-padded to 256) with the LayerNorm
-    fused into its activation prologue and bias / quick-GELU / erf-GELU / residual add in its epilogue;
+    """The CLIP tower on the engine's own kernels (GPU): every projection is a register-ring MFMA product
+    (csrc/kernels/gemm_f16.hip) on fp16 weight rows (QT_F16, K zero-padded to 256) with the LayerNorm
+    fused into its activation preparation and bias / quick-GELU / erf-GELU / residual add in its epilogue;
     QKV goes through the same RoPE-less QKV epilogue as the LLM and scatters K/V into a private paged
     cache that the MFMA flash-attention kernel (attention.hip) reads with every key visible to every
     query (q_len = n: bidirectional). Only the patch im2col, the class/position add and the stand-alone
@@ -275,11 +275,10 @@ class _NativeTower:
         self.mm2, self.mb2 = M(w2), f(b2)
         self.F = enc.blocks[0]["ffn_up.weight"].shape[0] if enc.blocks else E
         self.P = w0.shape[0]
-        # workspaces: fp16 activations (largest K), split-K slabs, the attention cache and step inputs
+        # workspaces: fp16 activations (largest K), the attention cache and step inputs
         kmax = max((w.shape[1] + 255) // 256 * 256 for w in [enc.patch_w.reshape(E, -1), w0, w2] +
                    [b["ffn_down.weight"] for b in enc.blocks] + [b["attn_q.weight"] for b in enc.blocks])
         self.xws = torch.empty(n * kmax, **h16)
-        self.gws = torch.empty(8 << 20, **f32)
         self.H, self.D = c.n_head, E // c.n_head
         self.bs = 16
         nblk = (n + self.bs - 1) // self.bs
@@ -297,8 +296,7 @@ class _NativeTower:
 
     def _gemm(self, w, B, x, ldx, y, ldy, epi, bias=None, norm=None, extra=None):
         d = dict(extra or {})
-        d.update(xws=self.xws.data_ptr(), xws_elems=self.xws.numel(), gws=self.gws.data_ptr(),
-                 gws_elems=self.gws.numel())
+        d.update(xws=self.xws.data_ptr(), xws_elems=self.xws.numel())
         nw, nb = norm if norm is not None else (None, None)
         p = lambda t: t.data_ptr() if t is not None else 0  # noqa: E731
         self.C.gemv(w, B, x.data_ptr(), ldx, self.NORM_LAYER if norm is not None else 0, p(nw), p(nb),
