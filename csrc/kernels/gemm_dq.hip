@@ -18,11 +18,7 @@ void run_dq_q5k(const GemvParams& P, f16* xp, int Kp, hipStream_t s);  // gemm_d
 void run_dq_q6k(const GemvParams& P, f16* xp, int Kp, hipStream_t s);  // gemm_dq_q6k.hip
 void run_dq_q40(const GemvParams& P, f16* xp, int Kp, hipStream_t s);  // gemm_dq_q40.hip
 void run_dq_q80(const GemvParams& P, f16* xp, int Kp, hipStream_t s);  // gemm_dq_q80.hip
-void run_dq_moe_q4k(const GemvParams& P, f16* xp, int Kp, hipStream_t s);
-void run_dq_moe_q5k(const GemvParams& P, f16* xp, int Kp, hipStream_t s);
-void run_dq_moe_q6k(const GemvParams& P, f16* xp, int Kp, hipStream_t s);
-void run_dq_moe_q40(const GemvParams& P, f16* xp, int Kp, hipStream_t s);
-void run_dq_moe_q80(const GemvParams& P, f16* xp, int Kp, hipStream_t s);
+void run_dq_moe(const GemvParams& P, f16* xp, int Kp, hipStream_t s);  // gemm_dq_moe.hip
 void run_dq_f16(const GemvParams& P, f16* xp, int Kp, hipStream_t s);  // gemm_f16.hip: tiles of its own
 
 bool dq_gemm_enabled() {
@@ -75,8 +71,7 @@ bool dq_gemm(const GemvParams& P, hipStream_t s) {
   return true;
 }
 
-// Routed experts: gate / up of every (token, expert) pair, then down with the pairs' own output rows in P.y. From a block per
-// CU on: below that (tiny experts) too few of the chip's CUs walk K, and the callers keep the per-expert path.
+// Routed experts: gate / up of every (token, expert) pair, then down with the pairs' own output rows in P.y
 bool dq_moe_covered(const GemvParams& P) {
   const int qt = P.w.qtype, Kp = ((P.w.K + 255) >> 8) * 256;
   return dq_gemm_enabled() && P.xws && P.moe_tiles && P.moe_rows && (long long)P.B * Kp <= P.xws_elems && P.w.K % 4 == 0 &&
@@ -87,13 +82,7 @@ void dq_moe(const GemvParams& P, hipStream_t s) {
   const int Kp = ((P.w.K + 255) >> 8) * 256;
   f16* xp = (f16*)P.xws;
   count_launch(LC_DQ_GEMM);
-  switch (P.w.qtype) {
-    case QT_Q4_K: run_dq_moe_q4k(P, xp, Kp, s); break;
-    case QT_Q5_K: run_dq_moe_q5k(P, xp, Kp, s); break;
-    case QT_Q6_K: run_dq_moe_q6k(P, xp, Kp, s); break;
-    case QT_Q4_0: run_dq_moe_q40(P, xp, Kp, s); break;
-    default: run_dq_moe_q80(P, xp, Kp, s); break;
-  }
+  run_dq_moe(P, xp, Kp, s);
 }
 
 }  // namespace omx

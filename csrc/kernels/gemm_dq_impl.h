@@ -479,8 +479,9 @@ __global__ __launch_bounds__(DQ_NT, 1) void dq_gemm_kernel(GemvParams P, const f
 // moe_scatter, to the pair's own row, unweighted (moe_combine sums a token's pairs). One launch for all experts, and the
 // routed counts stay on the device. What bounds it: the weights' way in (a tile of an expert's matrix serves one or two M
 // tiles, so little comes from L2) and dequantising them for 128 rows at a time. Measured, 500 rows through the top 2 of 8
-// experts of 14336 x 4096: gate / up 0.98 ms, down 0.52 (Q4_K) and 0.71 (Q6_K); two layers with everything else 3.87 ms, where
-// dequantising each expert to fp16 for a library product, with the counts on the host, made them 5.60.
+// experts of 14336 x 4096: gate / up 0.87 ms, down 0.51 (Q4_K) and 0.71 (Q6_K); two layers with everything else 3.80 ms, where
+// dequantising each expert to fp16 for a library product, with the counts on the host, made them 5.60. Tiles of 128 columns,
+// two blocks per CU: with 256 columns gate / up took 0.98, four K steps deep 0.92, down 0.62 and 0.82.
 template <int QT, int BM, int BN, int WM, int WN, bool GROUPED = false>
 __global__ __launch_bounds__(DQ_NT, 1) void dq_gemm_ring_kernel(GemvParams P, const f16* __restrict__ X, int Kp, int sk) {
   static_assert(WM * WN == 8, "8 waves");
@@ -701,20 +702,6 @@ void run_dq(const GemvParams& P, f16* xp, int Kp, hipStream_t s) {
     default: launch_dq<QT, 128, 128, 2, 4>(P, xp, Kp, sk, s); break;
   }
   if (sk > 1) gemm_finalize(P, sk, s);
-}
-
-template <int QT, int BN>
-void launch_dq_moe(const GemvParams& P, const f16* xp, int Kp, hipStream_t s) {
-  const int nt = (P.w.N + BN - 1) / BN;
-  hipLaunchKernelGGL((dq_gemm_ring_kernel<QT, 128, BN, 2, 4, true>), dim3(P.moe_max_tiles * nt), dim3(DQ_NT), (dq_lds<128, BN>()), s, P, xp,
-                     Kp, 1);
-}
-template <int QT>
-void run_dq_moe(const GemvParams& P, f16* xp, int Kp, hipStream_t s) {
-  hipLaunchKernelGGL(prep_xp_kernel<QT>, dim3(P.B), dim3(256), (size_t)Kp * sizeof(float), s, P, xp, Kp);
-  // wide matrices in 256 columns a tile; narrow ones in 128, two blocks per CU, which leave a shorter last wave
-  if (P.w.N >= 8192) launch_dq_moe<QT, 256>(P, xp, Kp, s);
-  else launch_dq_moe<QT, 128>(P, xp, Kp, s);
 }
 
 }  // namespace

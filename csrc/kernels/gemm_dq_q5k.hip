@@ -4,6 +4,5 @@
 namespace omx {
 
 void run_dq_q5k(const GemvParams& P, f16* xp, int Kp, hipStream_t s) { run_dq<QT_Q5_K>(P, xp, Kp, s); }
-void run_dq_moe_q5k(const GemvParams& P, f16* xp, int Kp, hipStream_t s) { run_dq_moe<QT_Q5_K>(P, xp, Kp, s); }
 
 }  // namespace omx

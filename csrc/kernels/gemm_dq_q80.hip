@@ -4,6 +4,5 @@
 namespace omx {
 
 void run_dq_q80(const GemvParams& P, f16* xp, int Kp, hipStream_t s) { run_dq<QT_Q8_0>(P, xp, Kp, s); }
-void run_dq_moe_q80(const GemvParams& P, f16* xp, int Kp, hipStream_t s) { run_dq_moe<QT_Q8_0>(P, xp, Kp, s); }
 
 }  // namespace omx

@@ -201,7 +201,7 @@ class Runner:
         self.lib_min = native().gemm_lib_min_m() if self.is_gpu else 0
         # MoE prefill: (token, expert) pairs from which each expert's GEMM runs on hipBLASLt over its
         # per-call dequantised weights (gemm.hip moe_gemm_lib; default 256, OMX_MOE_LIB_MIN_M) where the grouped
-        # launches' tiles do not fill the chip (gemm_dq.hip dq_moe)
+        # launches do not take them (executor.cpp ffn_block: gate and up of under 2,048 rows)
         self.moe_lib = native().moe_lib_min_m() if self.is_gpu and self.w.cfg.n_expert else 0
         cfg = self.cfg = self.w.cfg
         loc = self.w.local
