@@ -79,7 +79,7 @@ __global__ __launch_bounds__(256) void prep_f16_kernel(GemvParams P, f16* out, i
 template <int E>
 struct Out {
   GemvParams P;
-  __device__ __forceinline__ void operator()(int m, int n, float v, float pv) const { epi_apply_t<E>(P, m, n, v, pv, 0); }
+  __device__ __forceinline__ void operator()(int m, int n, float v, float pv) const { epi_apply_t<E>(P, m, n + P.row_offset, v, pv, 0); }
 };
 
 template <int E>

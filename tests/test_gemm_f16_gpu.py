@@ -9,11 +9,11 @@ pytestmark = pytest.mark.gpu
 p = lambda t: t.data_ptr() if t is not None else 0  # noqa: E731
 
 
-def run(w, K, x, y, epi=0, norm=0, nw=None, nb=None, bias=None):
+def run(w, K, x, y, epi=0, norm=0, nw=None, nb=None, bias=None, row_offset=0):
     B = x.shape[0]
     xws = torch.empty(B * w.shape[1], device="cuda", dtype=torch.float16)
     C().reset_launch_counts()
-    C().gemv((p(w), 0, 0, 0, w.shape[0], K, 1), B, p(x), x.shape[1], norm, p(nw), p(nb), 1e-5, epi, p(y), y.shape[1], p(bias), 0,
+    C().gemv((p(w), 0, 0, 0, w.shape[0], K, 1), B, p(x), x.shape[1], norm, p(nw), p(nb), 1e-5, epi, p(y), y.shape[1], p(bias), row_offset,
              dict(xws=p(xws), xws_elems=xws.numel()), S())
     torch.cuda.synchronize()
     assert C().launch_counts()["dq_gemm"] == 1
@@ -52,3 +52,18 @@ def test_gemm_f16(B, N, K):
         run(w, K, x, y, epi=2)
         g = z - bias.double()
         assert rel(y, (torch.nn.functional.silu(g[:, 0::2]) * g[:, 1::2]).float()) < 4e-5
+
+
+@pytest.mark.parametrize("B,N,K,at", [(128, 70, 588, 5), (577, 1024, 1024, 2048), (300, 130, 4360, 1)])
+def test_rows_of_a_concatenated_matrix(B, N, K, at):
+    """The matrix is rows at .. at + N - 1 of a concatenated one: outputs and biases sit there, the columns beside them stay.
+    Tolerance as above."""
+    torch.manual_seed(at)
+    w = torch.zeros(N, (K + 255) // 256 * 256, device="cuda", dtype=torch.float16)
+    w[:, :K] = torch.randn(N, K, device="cuda") / K ** 0.5
+    x, bias = torch.randn(B, K, device="cuda"), torch.randn(at + N, device="cuda")
+    y = torch.full((B, at + N + 3), 9.0, device="cuda")
+    run(w, K, x, y, bias=bias, row_offset=at)
+    z = x.half().double() @ w[:, :K].double().T + bias[at:].double()
+    assert rel(y[:, at:at + N], z.float()) < 2e-5
+    assert bool((y[:, :at] == 9.0).all()) and bool((y[:, at + N:] == 9.0).all())
