@@ -57,10 +57,20 @@ __global__ __launch_bounds__(512, 2) void dq_rows_kernel(GemvParams P, const f16
         for (int k = 0; k < 4; ++k) a[i][k] = *(const u32x4*)(x + i * 16 * Kp + 128 * k);
       }
   };
-  auto multiply = [&](int q, const Piece<QT> (&p)[NT], const u32x4 (&a)[MT][4]) {
+  auto multiply = [&](int q, const Piece<QT> (&p)[NT], u32x4 (&a)[MT][4]) {
     int t, sb;
     where(q, t, sb);
-    const bool in = sb < SB;  // a lane group past the last super-block multiplies zeros
+    const bool in = sb < SB;
+    // a lane group past the last super-block multiplies zeros with zeros: what it loaded is another group's, and an
+    // activation that is infinite in fp16 would make 0 times it no number
+    if (!in) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+        if (i < mt) {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) a[i][k] = (u32x4){0u, 0u, 0u, 0u};
+        }
+    }
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       unsigned o[16];

@@ -77,3 +77,23 @@ def test_rows_epilogues(B):
     seen = lambda c: c.permute(0, 2, 1, 3).reshape(blocks * bs, kv, D)[:B].float()  # noqa: E731
     assert rel(seen(kc), turn(zk.view(B, kv, D))) < 3e-3 and rel(seen(vc), zv.view(B, kv, D)) < 3e-3
     assert math.isfinite(float(kc.float().abs().max()))
+
+
+@pytest.mark.parametrize("qt", QTYPES)
+@pytest.mark.parametrize("K", [256, 768, 1280, 2304])
+def test_activations_past_fp16(qt, K):
+    """An activation that overflows fp16 (its rows' products are infinite, or no number where the weight is 0) in the last
+    super-block, which the lane groups past a count that is no multiple of four load too: the same infinities as the product
+    of the rounded operands gives, and rows without one stay finite."""
+    m = QM(qt, 96, K, seed=K)
+    for B in (16, 33, 64):
+        x = torch.randn(B, K, device="cuda")
+        x[B // 2, K - 7] = 1e6
+        y = torch.zeros(B, 96, device="cuda")
+        run(m, x, y)
+        want = x.half().double() @ m.w.double().T
+        assert bool((torch.isnan(y) == torch.isnan(want)).all()) and bool((torch.isinf(y) == torch.isinf(want)).all())
+        inf = torch.isinf(want)
+        assert bool((y[inf].double() == want[inf]).all())
+        rows = torch.arange(B, device="cuda") != B // 2
+        assert rel(y[rows], want[rows].float()) < 2e-3
