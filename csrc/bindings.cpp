@@ -322,7 +322,7 @@ PYBIND11_MODULE(_C, m) {
   // launch counters (ops.h LC_*): tests assert which kernel family a call enqueued
   m.def("launch_counts", []() {
     static const char* names[LC_N] = {"dq_gemm", "gemm_tile", "gemm_lib", "gemv8_row1", "gemv8_rows", "gemv8_dual",
-                                      "gemv_mb", "gemv_flight", "attn_decode", "attn_prefill", "gemv8_pair"};
+                                      "gemv_mb", "gemv_flight", "attn_decode", "attn_prefill", "gemv8_pair", "gemm_rows"};
     py::dict d;
     for (int i = 0; i < LC_N; ++i) d[names[i]] = launch_count(i);
     return d;

@@ -612,8 +612,8 @@ void gemm(const GemvParams& P, hipStream_t s) {
     }
   }
   if (dq_gemm(P, s)) return;
-  count_launch(LC_GEMM_TILE);
   if (dq_rows(P, s)) return;
+  count_launch(LC_GEMM_TILE);
   if (!lib) hipLaunchKernelGGL(prep_x16_kernel, dim3(P.B), dim3(256), 0, s, P, x16);
   switch (P.w.qtype) {
     case QT_Q4_K: launch_gemm<QT_Q4_K>(P, x16, s); break;

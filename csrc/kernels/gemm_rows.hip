@@ -159,6 +159,7 @@ bool dq_rows(const GemvParams& P, hipStream_t s) {
     case QT_Q8_0: run_rows<QT_Q8_0>(P, xp, Kp, s); break;
     default: return false;
   }
+  count_launch(LC_GEMM_ROWS);
   return true;
 }
 

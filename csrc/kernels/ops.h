@@ -345,7 +345,7 @@ void ar_allgather(const ARParams& P, int slab, float* out, int rows, int n_local
 // the host per enqueue (a captured graph counts at capture); tests reset, run, and assert.
 enum {
   LC_DQ_GEMM = 0,    // gemm_dq.hip stream-order MFMA prefill GEMM
-  LC_GEMM_TILE,      // gemm.hip 128 x 128 tile GEMM (< 128 rows, or a declined dq shape)
+  LC_GEMM_TILE,      // gemm.hip 128 x 128 tile GEMM (what gemm_dq.hip and gemm_rows.hip decline)
   LC_GEMM_LIB,       // hipBLASLt path (OMX_GEMM_LIB_MIN_M)
   LC_GEMV8_ROW1,     // gemv8.hip int8 chain, one row
   LC_GEMV8_ROWS,     // gemv8.hip int8 chain, 2..4 batched rows
@@ -355,6 +355,7 @@ enum {
   LC_ATTN_DECODE,    // attention.hip split flash-decode kernel
   LC_ATTN_PREFILL,   // attention.hip MFMA flash prefill
   LC_GEMV8_PAIR,     // gemv8_pair.hip Phi-2 O + ffn_down in one launch
+  LC_GEMM_ROWS,      // gemm_rows.hip products of 16..64 rows
   LC_N
 };
 void count_launch(int which);

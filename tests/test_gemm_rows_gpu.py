@@ -1,6 +1,6 @@
 """Prompt portions of 16 .. 64 rows (csrc/kernels/gemm_rows.hip) and of 65 .. 127 (the 128-row tiles of gemm_dq.hip): every quant
-type against a float32 product on the
-dequantised weights, where rows, columns, super-blocks and the waves' shares of K end, and the epilogues that pair rows."""
+type against a float32 product on the dequantised weights, where rows, columns, super-blocks and the waves' shares of K end, the
+epilogues that pair rows, and what the kernels leave to others. Launch counters say which kernel ran."""
 import math
 
 import pytest
@@ -13,9 +13,10 @@ pytestmark = pytest.mark.gpu
 p = lambda t: t.data_ptr() if t is not None else 0  # noqa: E731
 
 
-def run(m, x, y, epi=0, norm=0, nw=None, bias=None, extra=None):
+def run(m, x, y, epi=0, norm=0, nw=None, bias=None, extra=None, rows=0, kernel=""):
+    """rows: rows that the fp16 workspace holds (0: whole row tiles); kernel: the launch counter that moves, and no other."""
     B, K = x.shape
-    xws = torch.empty((B + 15) // 16 * 16 * ((K + 255) // 256 * 256), device="cuda", dtype=torch.float16)
+    xws = torch.empty((rows or (B + 15) // 16 * 16) * ((K + 255) // 256 * 256), device="cuda", dtype=torch.float16)
     d = dict(extra or {}, xws=xws.data_ptr(), xws_elems=xws.numel())
     on = C().dq_gemm_enabled()
     C().set_dq_gemm(1)
@@ -24,7 +25,8 @@ def run(m, x, y, epi=0, norm=0, nw=None, bias=None, extra=None):
     torch.cuda.synchronize()
     C().set_dq_gemm(int(on))
     n = C().launch_counts()
-    assert n["gemm_tile"] == int(B <= 64) and n["dq_gemm"] == int(B > 64), n
+    kernel = kernel or ("gemm_rows" if B <= 64 else "dq_gemm")
+    assert {k: v for k, v in n.items() if v} == {kernel: 1}, n
 
 
 @pytest.mark.parametrize("qt", QTYPES)
@@ -97,3 +99,12 @@ def test_activations_past_fp16(qt, K):
         assert bool((y[inf].double() == want[inf]).all())
         rows = torch.arange(B, device="cuda") != B // 2
         assert rel(y[rows], want[rows].float()) < 2e-3
+
+
+@pytest.mark.parametrize("B", [17, 33, 63])
+def test_short_workspace(B):
+    """A workspace without room for the last row tile (the caller's rows only): the 128 x 128 tile kernel takes the call."""
+    m = QM(GGMLType.Q4_K, 200, 1024, seed=B)
+    x, y = torch.randn(B, 1024, device="cuda"), torch.zeros(B, 200, device="cuda")
+    run(m, x, y, rows=B, kernel="gemm_tile")
+    assert rel(y, x @ m.w.T) < 2e-3
