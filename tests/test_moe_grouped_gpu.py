@@ -43,7 +43,8 @@ def test_grouped_experts(tmp_path, ft, n_ff, rows):
     old, m = logits("cuda")
     C.set_dq_gemm(int(on))
     # gate|up and down: dq_gemm; q|k|v (one launch, or v apart) and o: the same tiles from 65 rows, gemm_rows.hip below
-    assert n["gemm_tile"] == 0 and (n["dq_gemm"] >= 4 and n["gemm_rows"] == 0 if rows > 64 else n["dq_gemm"] == 2 and n["gemm_rows"] >= 2), n
+    assert n["gemm_tile"] == 0, n
+    assert n["dq_gemm"] >= 4 and n["gemm_rows"] == 0 if rows > 64 else n["dq_gemm"] == 2 and n["gemm_rows"] >= 2, n
     assert m["dq_gemm"] == m["gemm_rows"] == 0, m
     err = lambda v: float((v - want).norm() / want.norm())  # noqa: E731
     print(err(got), err(old))
