@@ -57,7 +57,7 @@ bool dq_gemm(const GemvParams& P, hipStream_t s) {
   if (qt != QT_Q4_K && qt != QT_Q5_K && qt != QT_Q6_K && qt != QT_Q4_0 && qt != QT_Q8_0 && qt != QT_F16) return false;
   const int Kp = ((P.w.K + 255) >> 8) * 256;
   const long long cap = P.xws_elems ? P.xws_elems : (long long)P.B * P.w.K;
-  if ((long long)P.B * Kp > cap) return false;
+  if ((long long)P.B * Kp > cap || (qt != QT_F16 && Kp > PREP_MAX_KP)) return false;
   f16* xp = (f16*)P.xws;
   count_launch(LC_DQ_GEMM);
   switch (qt) {
@@ -75,6 +75,7 @@ bool dq_gemm(const GemvParams& P, hipStream_t s) {
 bool dq_moe_covered(const GemvParams& P) {
   const int qt = P.w.qtype, Kp = ((P.w.K + 255) >> 8) * 256;
   return dq_gemm_enabled() && P.xws && P.moe_tiles && P.moe_rows && (long long)P.B * Kp <= P.xws_elems && P.w.K % 4 == 0 &&
+         Kp <= PREP_MAX_KP &&
          (qt == QT_Q4_K || qt == QT_Q5_K || qt == QT_Q6_K || qt == QT_Q4_0 || qt == QT_Q8_0) &&
          (P.epi == EPI_GLU || P.epi == EPI_GEGLU || P.epi == EPI_STORE);
 }

@@ -98,6 +98,7 @@ __host__ __device__ __forceinline__ int prep_at(int k) {
 // Stream position kp: piece P = kp / 32 (t = P / SB, sb = P % SB), slot p = kp % 32: half g = p / 16,
 // byte i = 4 ((p & 15) / 4) + (0, 2, 1, 3)[p & 3] -> natural k = piece_off(t, sb, g) + i
 // ROWS (gemm_rows.hip): [16-row tile][32-K piece][8-K run][row], so that a wave reads a run of 16 rows as one block
+// (PREP_MAX_KP: the longest row that fits)
 template <int QT, bool ROWS = false>
 __global__ __launch_bounds__(256) void prep_xp_kernel(GemvParams P, f16* out, int Kp) {
   // The row is staged in LDS in natural order (coalesced reads of x), normed there in place (coalesced reads of the

@@ -149,7 +149,7 @@ bool dq_rows(const GemvParams& P, hipStream_t s) {
   if (!dq_gemm_enabled() || P.B < 2 || P.B > 64 || !P.xws || P.expert_ids || P.moe_tiles || P.w.K % 8) return false;
   const int Kp = ((P.w.K + 255) >> 8) * 256;
   const long long cap = P.xws_elems ? P.xws_elems : (long long)P.B * P.w.K;
-  if ((long long)((P.B + 15) & ~15) * Kp > cap) return false;  // whole 16-row tiles
+  if ((long long)((P.B + 15) & ~15) * Kp > cap || Kp > PREP_MAX_KP) return false;  // whole 16-row tiles
   f16* xp = (f16*)P.xws;
   switch (P.w.qtype) {
     case QT_Q4_K: run_rows<QT_Q4_K>(P, xp, Kp, s); break;

@@ -185,6 +185,9 @@ size_t mfma_layout_bytes(int qtype, int N, int K);  // 0 = no layout M for this 
 void repack_m(const QMat& w, void* out, hipStream_t s);
 bool gemm_eligible(const GemvParams& P);
 void gemm(const GemvParams& P, hipStream_t s);
+// Their preparation keeps a row of activations in LDS (prep_xp_kernel), which bounds the padded K of the three kernels below:
+// 4 bytes per element of the 160 KB, less the 16 of its sums. A wider matrix is not covered.
+constexpr int PREP_MAX_KP = (160 * 1024 - 16) / 1024 * 256;
 // stream-order dequant MFMA GEMM (gemm_dq.hip): M > 64 (fp16 weights: M >= 128), dense v2 matrices; false = not covered
 bool dq_gemm(const GemvParams& P, hipStream_t s);
 // the same for fewer rows (gemm_rows.hip): M <= 64; false = not covered

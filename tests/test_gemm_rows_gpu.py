@@ -108,3 +108,15 @@ def test_short_workspace(B):
     x, y = torch.randn(B, 1024, device="cuda"), torch.zeros(B, 200, device="cuda")
     run(m, x, y, rows=B, kernel="gemm_tile")
     assert rel(y, x @ m.w.T) < 2e-3
+
+
+@pytest.mark.parametrize("qt", [GGMLType.Q4_0, GGMLType.Q6_K])
+@pytest.mark.parametrize("B", [16, 64, 65, 130])
+def test_wide_rows(qt, B):
+    """The preparation keeps a row of activations in LDS, 160 KB: K = 40,704 is the last that fits, a wider matrix goes to the
+    tile kernel. (32-wide blocks: K need not be whole super-blocks.)"""
+    for K, kernel in ((40704, ""), (40736 if qt == GGMLType.Q4_0 else 40960, "gemm_tile"), (45056, "gemm_tile")):
+        m = QM(qt, 40, K, seed=B)
+        x, y = torch.randn(B, K, device="cuda"), torch.zeros(B, 40, device="cuda")
+        run(m, x, y, kernel=kernel)
+        assert rel(y, x @ m.w.T) < 2e-3, K
