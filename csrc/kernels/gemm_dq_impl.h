@@ -682,15 +682,21 @@ void run_dq(const GemvParams& P, f16* xp, int Kp, hipStream_t s) {
   const int bm[4] = {256, 256, 128, 128}, bn[4] = {256, 128, 256, 128};
   const double cst[4] = {2.19, 1.32, 1.44, 1.34};
   const int slots[4] = {256, 256, 256, 512};
+  // One M tile leaves a narrow matrix a handful of tiles, so under 128 rows K splits in up to 16 while all blocks run at once
+  // (in up to 4, the 128 x 128 tile kernel of gemm.hip, which splits finer, was ahead there). 4-bit types, 65 rows, tile
+  // kernel / 4 / 16: 1,024 x 4,096 25.0 / 31.5 / 25.7 us, 4,096 x 4,096 28.7 / 32.5 / 29.1, 4,096 x 11,008 58.8 / 66.6 / 43.4;
+  // 96 rows of 4,096 x 4,096 30.9 / 33.1 / 30.0
+  const int max_sk = M < 128 ? 16 : 4, min_steps = M < 128 ? 4 : 8;
   auto ntl = [&](int c) { return (long long)((M + bm[c] - 1) / bm[c]) * ((N + bn[c] - 1) / bn[c]); };
   int cfg = 3, sk = 1;
   double best = -1.0;
   for (int c = 0; c < 4; ++c) {
     if (g_dq_cfg >= 0 && g_dq_cfg <= 3 && c != g_dq_cfg) continue;  // microbenchmark override (OMX_DQ_CFG)
-    for (int k = 1; k <= 4; ++k) {
-      if (k > 1 && (!P.gws || (long long)k * M * N > P.gws_elems || nks / k < 8)) break;
+    for (int k = 1; k <= max_sk; ++k) {
+      if (k > 1 && (!P.gws || (long long)k * M * N > P.gws_elems || nks / k < min_steps)) break;
       if (g_dq_sk > 0 && k != g_dq_sk) continue;  // microbenchmark override (set_dq_tuning)
       const long long units = ntl(c) * k;
+      if (k > 4 && units > slots[c]) break;
       const double waves = (double)((units + slots[c] - 1) / slots[c]);
       const double t = waves * ((double)nks / k) * cst[c] + (k > 1 ? 2.0 * k * M * N * 4 / 5e6 : 0.0);
       if (best < 0.0 || t < best) best = t, cfg = c, sk = k;

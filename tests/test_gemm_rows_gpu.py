@@ -120,3 +120,17 @@ def test_wide_rows(qt, B):
         x, y = torch.randn(B, K, device="cuda"), torch.zeros(B, 40, device="cuda")
         run(m, x, y, kernel=kernel)
         assert rel(y, x @ m.w.T) < 2e-3, K
+
+
+@pytest.mark.parametrize("qt", QTYPES)
+@pytest.mark.parametrize("N,K", [(130, 1024), (256, 2304), (1024, 4096), (4096, 4096), (512, 11008), (2048, 11008), (22016, 512)])
+def test_split_k(qt, N, K):
+    """65 .. 127 rows with room for partial sums: narrow matrices split K up to 16 ways, shares of unequal length among them, and
+    add the shares up in a second launch. Limits as above."""
+    m = QM(qt, N, K, seed=N)
+    gws = torch.full((16 * 127 * N,), float("nan"), device="cuda")
+    for B in (65, 96, 127):
+        x, y = torch.randn(B, K, device="cuda"), torch.full((B, N + 3), 9.0, device="cuda")
+        run(m, x, y, extra=dict(gws=p(gws), gws_elems=gws.numel()))
+        assert rel(y[:, :N], x @ m.w.T) < 2e-3, B
+        assert bool((y[:, N:] == 9.0).all())
