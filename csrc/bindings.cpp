@@ -312,6 +312,8 @@ PYBIND11_MODULE(_C, m) {
   m.def("gemm_lib_min_m", &gemm_lib_min_m);
   m.def("set_moe_lib_min_m", &set_moe_lib_min_m, "MoE prefill pairs from which experts run on hipBLASLt (0 = off)");
   m.def("moe_lib_min_m", &moe_lib_min_m);
+  m.def("moe_grouped", [](py::object gu, py::object down) { return moe_grouped(qmat(gu), qmat(down)); },
+        "whether a layer's routed experts take the grouped launches (gemm_dq_moe.hip) for prompts");
   m.def("set_dq_gemm", &set_dq_gemm, "1: prefill GEMMs from 128 rows on the stream-order dequant kernel (gemm_dq.hip)");
   m.def("set_dq_tuning", &set_dq_tuning, "microbenchmarks: force the dq GEMM tile config (0..3, -1 auto) and split-K factor (0 auto)");
   m.def("dq_gemm_enabled", &dq_gemm_enabled);
@@ -471,6 +473,8 @@ PYBIND11_MODULE(_C, m) {
         w.moe_rows = Pp<int>(ptr("moe_rows"));
         w.moe_tiles = Pp<int>(ptr("moe_tiles"));
         w.moe_ntiles = Pp<int>(ptr("moe_ntiles"));
+        w.moe_y = Pp<float>(ptr("moe_y"));
+        w.moe_y_elems = d.contains("moe_y_elems") ? d["moe_y_elems"].cast<long long>() : 0;
         w.mb_ok = (d.contains("mb_ok") ? d["mb_ok"].cast<int>() : 0) && e.chain_capable() ? 1 : 0;
         w.xa16 = Pp<void>(ptr("xa16"));
         w.h16 = Pp<void>(ptr("h16"));

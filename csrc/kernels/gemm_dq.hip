@@ -71,12 +71,22 @@ bool dq_gemm(const GemvParams& P, hipStream_t s) {
   return true;
 }
 
-// Routed experts: gate / up of every (token, expert) pair, then down with the pairs' own output rows in P.y
+// Routed experts: gate / up of every (token, expert) pair, then down with the pairs' own output rows in P.y.
+// Four layers of 8 experts, top 2, this path against the others (executor.cpp ffn_block): 1024 x 1024 (2,048 rows of gate and
+// up) 17 rows 454 / 514 us, 130 rows 649 / 1,715; 4096 x 2048 17 rows 770 / 1,085, 1,000 rows 1,722 / 3,451; 14336 x 4096 64 rows
+// 2,668 / 4,838. Two layers of 64 experts of 1,024 x 2,048, top 8: 17 rows 617 / 842, 1,000 rows 1,902 / 7,230. Smaller experts
+// (not measured) stay with the others.
+static bool moe_matrix(const QMat& w) {
+  const int qt = w.qtype;
+  return w.K % 4 == 0 && ((w.K + 255) >> 8) * 256 <= PREP_MAX_KP &&
+         (qt == QT_Q4_K || qt == QT_Q5_K || qt == QT_Q6_K || qt == QT_Q4_0 || qt == QT_Q8_0);
+}
+bool moe_grouped(const QMat& gu, const QMat& down) {
+  return dq_gemm_enabled() && gu.N >= 2048 && moe_matrix(gu) && moe_matrix(down);
+}
 bool dq_moe_covered(const GemvParams& P) {
-  const int qt = P.w.qtype, Kp = ((P.w.K + 255) >> 8) * 256;
-  return dq_gemm_enabled() && P.xws && P.moe_tiles && P.moe_rows && (long long)P.B * Kp <= P.xws_elems && P.w.K % 4 == 0 &&
-         Kp <= PREP_MAX_KP &&
-         (qt == QT_Q4_K || qt == QT_Q5_K || qt == QT_Q6_K || qt == QT_Q4_0 || qt == QT_Q8_0) &&
+  const int Kp = ((P.w.K + 255) >> 8) * 256;
+  return dq_gemm_enabled() && moe_matrix(P.w) && P.xws && P.moe_tiles && P.moe_rows && (long long)P.B * Kp <= P.xws_elems &&
          (P.epi == EPI_GLU || P.epi == EPI_GEGLU || P.epi == EPI_STORE);
 }
 void dq_moe(const GemvParams& P, hipStream_t s) {

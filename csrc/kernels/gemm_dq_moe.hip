@@ -6,7 +6,7 @@ namespace {
 
 template <int QT>
 void run_moe(const GemvParams& P, f16* xp, int Kp, hipStream_t s) {
-  constexpr int BM = 128, BN = 128;  // BM: the tiles of P.moe_tiles
+  constexpr int BM = MOE_TILE_M, BN = 128;  // BM: the tiles of P.moe_tiles
   hipLaunchKernelGGL(prep_xp_kernel<QT>, dim3(P.B), dim3(256), (size_t)Kp * sizeof(float), s, P, xp, Kp);
   hipLaunchKernelGGL((dq_gemm_ring_kernel<QT, BM, BN, 2, 4, true>), dim3(P.moe_max_tiles * ((P.w.N + BN - 1) / BN)), dim3(DQ_NT),
                      (dq_lds<BM, BN>()), s, P, xp, Kp, 1);

@@ -192,7 +192,9 @@ constexpr int PREP_MAX_KP = (160 * 1024 - 16) / 1024 * 256;
 bool dq_gemm(const GemvParams& P, hipStream_t s);
 // the same for fewer rows (gemm_rows.hip): M <= 64; false = not covered
 bool dq_rows(const GemvParams& P, hipStream_t s);
-// routed experts in one launch per matrix (P.moe_* set; gemm_dq.hip); dq_moe only where dq_moe_covered
+// routed experts in one launch per matrix (P.moe_* set; gemm_dq.hip). moe_grouped: whether a layer's experts take it, given the
+// workspaces (the runner sizes them by the same rule); dq_moe only where dq_moe_covered
+bool moe_grouped(const QMat& gu, const QMat& down);
 bool dq_moe_covered(const GemvParams& P);
 void dq_moe(const GemvParams& P, hipStream_t s);
 bool dq_gemm_enabled();

@@ -427,17 +427,16 @@ void Executor::ffn_block(int i, const StepInputs& in, hipStream_t s) {
       Dn.ldy = E;
       grouped(Dn);
       Dn.moe_scatter = 1;
-      // all experts in one launch per matrix (gemm_dq_moe.hip), outputs of the down projection per pair, summed per token
-      // afterwards. Four layers of 8 experts, top 2, this path against the ones below: 1024 x 1024 (2,048 rows of
-      // gate and up) 17 rows 454 / 514 us, 130 rows 649 / 1,715; 4096 x 2048 17 rows 770 / 1,085, 1,000 rows 1,722 / 3,451;
-      // 14336 x 4096 64 rows 2,668 / 4,838. Smaller experts (not measured) stay below, as does what is short of workspace
+      // all experts in one launch per matrix (gemm_dq_moe.hip; the rule is moe_grouped's), outputs of the down projection per
+      // pair, summed per token afterwards
       Dn.epi = EPI_STORE;
-      Dn.y = ws.yws;
-      if (G.w.N >= 2048 && ws.yws && (long long)pairs * E <= ws.yws_elems && dq_moe_covered(G) && dq_moe_covered(Dn)) {
+      Dn.y = ws.moe_y;
+      if (moe_grouped(L.gu_exps, L.down_exps) && ws.moe_y && (long long)pairs * E <= ws.moe_y_elems && dq_moe_covered(G) &&
+          dq_moe_covered(Dn)) {
         dq_moe(G, s);
         dq_moe(Dn, s);
         if (cfg.tp > 1) hipMemsetAsync(dst, 0, sizeof(float) * (size_t)B * E, s);
-        moe_combine(ws.yws, ws.ew, B, k, E, dst, E, s);
+        moe_combine(ws.moe_y, ws.ew, B, k, E, dst, E, s);
         return;
       }
       // long prompts: per-expert hipBLASLt GEMMs (gemm.hip moe_gemm_lib) need the routed counts on the

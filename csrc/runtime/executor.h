@@ -70,6 +70,8 @@ struct Workspace {
   int* moe_rows = nullptr;   // [maxB*k] MoE prefill: pairs sorted by expert
   int* moe_tiles = nullptr;  // [(maxB*k/128 + X + 1)*3] expert row tiles
   int* moe_ntiles = nullptr; // [1]
+  float* moe_y = nullptr;    // [maxB*k][E] grouped experts: the down projection's outputs per pair
+  long long moe_y_elems = 0;
   long long gws_elems = 0;
   const float* ext = nullptr;  // [*][E] external embedding rows (negative token ids), e.g. image patches
   void* w16 = nullptr;       // large-M prefill library GEMM: fp16 dequantised weight [N][K] scratch

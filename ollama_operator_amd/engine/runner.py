@@ -71,7 +71,7 @@ class NativeExec:
                              attn_ws=p(r.attn_ws), attn_cnt=p(r.attn_cnt), x16=p(r.x16), x16_elems=r.x16.numel(),
                              gws=p(r.gws),
                              moe_rows=p(r.moe_rows) if cfg.n_expert else 0, moe_tiles=p(r.moe_tiles),
-                             moe_ntiles=p(r.moe_ntiles),
+                             moe_ntiles=p(r.moe_ntiles), moe_y=p(r.moe_y), moe_y_elems=r.moe_y.numel() if r.moe_y is not None else 0,
                              gws_elems=r.gws.numel(), max_B=r.max_batch, ld_logits=r.logits.shape[1],
                              ext=p(r.ext), w16=p(r.w16), w16_elems=r.w16.numel() if r.w16 is not None else 0,
                              yws=p(r.yws), yws_elems=r.yws.numel() if r.yws is not None else 0,
@@ -199,9 +199,9 @@ class Runner:
         # prefill GEMM runs the hand-written dequant kernel over the resident quantised weights, and no fp16
         # weight copy exists -- OMX_GEMM_LIB_MIN_M=<rows> is the A/B knob)
         self.lib_min = native().gemm_lib_min_m() if self.is_gpu else 0
-        # MoE prefill: (token, expert) pairs from which each expert's GEMM runs on hipBLASLt over its
-        # per-call dequantised weights (gemm.hip moe_gemm_lib; default 256, OMX_MOE_LIB_MIN_M) where the grouped
-        # launches do not take them (executor.cpp ffn_block: gate and up of under 2,048 rows)
+        # MoE prefill, experts that the grouped launches leave (gemm_dq.hip moe_grouped: gate and up of under 2,048
+        # rows): (token, expert) pairs from which each expert's GEMM runs on hipBLASLt over its per-call
+        # dequantised weights (gemm.hip moe_gemm_lib; default 256, OMX_MOE_LIB_MIN_M)
         self.moe_lib = native().moe_lib_min_m() if self.is_gpu and self.w.cfg.n_expert else 0
         cfg = self.cfg = self.w.cfg
         loc = self.w.local
@@ -241,13 +241,15 @@ class Runner:
         self.rlogits = torch.zeros(max_batch, max(1, cfg.n_expert), **f32)
         self.eids = torch.zeros(max_batch, ksel, **i32)
         self.ew = torch.zeros(max_batch, ksel, **f32)
-        # fp16 activations for the prefill MFMA GEMM (any GEMM input: E, H*D, F, k*F wide)
-        self.x16 = torch.zeros(max_batch * max(E, Eq, ksel * Fl, ksel * E), device=dev, dtype=torch.float16)
+        # fp16 activations for the prefill MFMA GEMM (any GEMM input: E, H*D, F, k*F wide), whole 16-row tiles of whole
+        # super-blocks as the dequantising kernels lay them out
+        r256 = lambda n: (n + 255) // 256 * 256  # noqa: E731
+        self.x16 = torch.zeros((max_batch + 15) // 16 * 16 * max(r256(Eq), ksel * r256(Fl), ksel * r256(E)), device=dev,
+                               dtype=torch.float16)
         # batched decode chain on the matrix cores (executor.cpp chain(): 2 <= B <= 16): fp16 activation
         # rows [17][ld] (row 16 stays zero) + RMS sum-of-squares partial slabs
         self.mb_bufs = None
         if self.mfma_bytes:
-            r256 = lambda n: (n + 255) // 256 * 256  # noqa: E731
             h16 = dict(device=dev, dtype=torch.float16)
             self.mb_bufs = dict(xa16=torch.zeros(17, r256(E), **h16), h16=torch.zeros(17, r256(Fl), **h16),
                                 a16=torch.zeros(17, r256(Eq), **h16), st0=torch.zeros((E + 15) // 16 * 16 + 32, **f32),
@@ -275,19 +277,25 @@ class Runner:
         self._ext_next = 0
         # split-K partial slabs of small-M prefill GEMMs (the kernel picks splits that fit)
         self.gws = torch.zeros(GEMM_SPLIT_WS_FLOATS if str(dev).startswith("cuda") else 1, **f32)
-        # hipBLASLt prefill (gemm.hip gemm_lib) for chunks of >= gemm_lib_min_m() rows (default 2048;
-        # OMX_GEMM_LIB_MIN_M, 0 = never): fp16 dequantised-weight scratch sized for the largest dense
-        # layer matrix and its fp32 output slab at max_batch rows
+        # MoE prompts: layers whose experts take the grouped launches need an output row per (token, expert) pair; the
+        # others' experts may take hipBLASLt
+        experts = [(L["gu_exps"], L["down_exps"]) for L in self.w.layers if L.get("gu_exps") is not None] if self.is_gpu else []
+        grouped = [native().moe_grouped(gu.tup, dn.tup) for gu, dn in experts]
+        self.moe_y = torch.empty(n_pairs * E, **f32) if any(grouped) else None
+        # hipBLASLt prefill (gemm.hip gemm_lib, moe_gemm_lib) for chunks of >= gemm_lib_min_m() rows (default 0 = never)
+        # and the experts above: fp16 dequantised-weight scratch sized for the largest such matrix (expert stacks count
+        # per expert: DevQMat.N = rows of one expert) and its fp32 output slab at max_batch rows
         self.w16 = self.yws = None
         dense_lib = self.lib_min > 0 and max_batch >= max(16, self.lib_min)
-        moe_lib = self.moe_lib > 0 and max_batch * ksel >= self.moe_lib
-        if self.is_gpu and (dense_lib or moe_lib):
-            # expert stacks count per expert (DevQMat.N = rows of one expert): moe_gemm_lib
-            mats = [v for L in self.w.layers for k, v in L.items() if isinstance(v, DevQMat) and k != "router"
-                    and (dense_lib or k in ("gu_exps", "down_exps"))]
-            if mats:
-                self.w16 = torch.empty(max(m.N * m.K for m in mats), device=dev, dtype=torch.float16)
-                self.yws = torch.empty(max_batch * (ksel if moe_lib else 1) * max(m.N for m in mats), **f32)
+        mats = [m for pair, g in zip(experts, grouped) if not g for m in pair] if self.moe_lib > 0 and n_pairs >= self.moe_lib else []
+        slab = max_batch * ksel if mats else max_batch
+        if self.is_gpu and dense_lib:
+            mats += [v for L in self.w.layers for k, v in L.items()
+                     if isinstance(v, DevQMat) and k not in ("router", "gu_exps", "down_exps")]
+        self._lib_shapes = sorted({(m.N, m.K) for m in mats})
+        if mats:
+            self.w16 = torch.empty(max(N * K for N, K in self._lib_shapes), device=dev, dtype=torch.float16)
+            self.yws = torch.empty(slab * max(N for N, _K in self._lib_shapes), **f32)
         ws = max(self._ws_floats(B) for B in range(1, max_batch + 1))
         self.attn_ws = torch.zeros(max(ws, 1), **f32)
         self.attn_cnt = torch.zeros(max_batch * loc["H"], **i32)  # self re-arming tickets
@@ -765,14 +773,8 @@ class Runner:
         if not self.is_gpu:
             return
         if self.w16 is not None:  # hipBLASLt plans for the long-prefill path (gemm.hip gemm_lib)
-            C = native()
-            lm = self.lib_min
-            if (lm > 0 and self.max_batch >= lm) or self.moe_lib > 0:
-                shapes = {(v.N, v.K) for L in self.w.layers for k, v in L.items()
-                          if isinstance(v, DevQMat) and k != "router" and (lm > 0 or k in ("gu_exps", "down_exps"))}
-                for N, K in sorted(shapes):
-                    if N * K <= self.w16.numel():  # from 128: MoE experts see any row count
-                        C.gemm_lib_prepare(N, K, 128, self.max_batch, self.gws.numel() * 4)
+            for N, K in self._lib_shapes:  # from 128: MoE experts see any row count
+                native().gemm_lib_prepare(N, K, 128, self.max_batch, self.gws.numel() * 4)
         # short prompts through the prefill path (GEMM + prep/finalize kernels resolved once); one per
         # hipBLASLt M bucket too -- a bucket's first GEMM also loads its kernel's code object (~0.1 s),
         # which must not land in a request's TTFT

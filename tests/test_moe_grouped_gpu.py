@@ -12,16 +12,20 @@ from ollama_operator_amd.ops import native
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("ft,n_ff,rows", [
-    (FileType.MOSTLY_Q4_K_M, 8192, 260), (FileType.MOSTLY_Q4_K_M, 3840, 577), (FileType.MOSTLY_Q5_K_S, 8192, 257),
-    (FileType.MOSTLY_Q4_0, 8192, 321), (FileType.MOSTLY_Q8_0, 3840, 640), (FileType.MOSTLY_Q6_K, 8192, 300),
-    (FileType.MOSTLY_Q4_K_M, 1024, 17), (FileType.MOSTLY_Q4_0, 1280, 129)])
-def test_grouped_experts(tmp_path, ft, n_ff, rows):
+@pytest.mark.parametrize("ft,n_ff,rows,n_embd", [
+    (FileType.MOSTLY_Q4_K_M, 8192, 260, 512), (FileType.MOSTLY_Q4_K_M, 3840, 577, 512), (FileType.MOSTLY_Q5_K_S, 8192, 257, 512),
+    (FileType.MOSTLY_Q4_0, 8192, 321, 512), (FileType.MOSTLY_Q8_0, 3840, 640, 512), (FileType.MOSTLY_Q6_K, 8192, 300, 512),
+    (FileType.MOSTLY_Q4_K_M, 1024, 17, 512), (FileType.MOSTLY_Q4_0, 1280, 129, 512),
+    # widths that are no multiple of 256 (padded K) nor of 128 (the last columns of an expert's tile), a full portion among them
+    (FileType.MOSTLY_Q4_0, 1056, 640, 576), (FileType.MOSTLY_Q8_0, 1056, 101, 576), (FileType.MOSTLY_Q4_0, 2144, 40, 1088),
+    (FileType.MOSTLY_Q8_0, 1120, 640, 1088)])
+def test_grouped_experts(tmp_path, ft, n_ff, rows, n_embd):
     """Against float32 on the CPU, beside the path that is taken with these kernels switched off: both round the same two
     operands to fp16 and add in float32, so neither may be further from float32 than the other by more than the order of sums
     and the atomics' order explain (a fifth)."""
     path = str(tmp_path / "m.gguf")
-    write_random_gguf(path, preset("tiny-mixtral", n_embd=512, n_ff=n_ff, n_layer=1, n_head=8, ctx_len=768), ft, seed=int(ft))
+    heads = dict(n_head=8) if n_embd == 512 else dict(n_head=n_embd // 64, n_head_kv=1)
+    write_random_gguf(path, preset("tiny-mixtral", n_embd=n_embd, n_ff=n_ff, n_layer=1, ctx_len=768, **heads), ft, seed=int(ft))
     rng = np.random.default_rng(rows)
     toks = [1] + [int(x) for x in rng.integers(3, 500, rows - 1)]
     C = native()
@@ -49,3 +53,28 @@ def test_grouped_experts(tmp_path, ft, n_ff, rows):
     err = lambda v: float((v - want).norm() / want.norm())  # noqa: E731
     print(err(got), err(old))
     assert err(got) < 1.2 * err(old) + 1e-4
+
+
+def test_grouped_experts_need_no_library(tmp_path, monkeypatch):
+    """The grouped launches run for a runner of a few rows, with the library path switched off or on, and bring no workspace of
+    the library's along; experts they leave (gate and up of under 2,048 rows) keep theirs."""
+    C = native()
+
+    def load(n_ff, max_batch, lib):
+        path = str(tmp_path / f"m{n_ff}.gguf")
+        write_random_gguf(path, preset("tiny-mixtral", n_embd=512, n_ff=n_ff, n_layer=1, n_head=8, ctx_len=512), FileType.MOSTLY_Q4_0,
+                          seed=1)
+        old = C.moe_lib_min_m()
+        C.set_moe_lib_min_m(lib)
+        try:
+            r = Runner(path, device="cuda", max_batch=max_batch, max_seqs=2, ctx=512)
+            C.reset_launch_counts()
+            r.prefill(r.new_sequence(), list(range(3, 43)))
+            return C.launch_counts()["dq_gemm"], r.w16 is not None, r.yws is not None, r.moe_y.numel() if r.moe_y is not None else 0
+        finally:
+            C.set_moe_lib_min_m(old)
+
+    for max_batch, lib in ((64, 256), (512, 256), (64, 0)):
+        assert load(1024, max_batch, lib) == (2, False, False, max_batch * 2 * 512)
+    assert load(512, 512, 256) == (0, True, True, 0)
+    assert load(512, 512, 0) == (0, False, False, 0)
