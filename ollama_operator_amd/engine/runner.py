@@ -686,11 +686,16 @@ class Runner:
                 reals = (o.temperature, o.top_p, o.min_p, o.repeat_penalty, o.presence_penalty, o.frequency_penalty)
                 if any(math.isfinite(v) and abs(v) > FLOAT_MAX for v in reals):
                     raise RuntimeError("sampling option out of the range of float32")
+                if not -(1 << 63) <= seed <= MASK64:
+                    raise RuntimeError("seed out of the range of 64 bits")
                 f[i, 0] = reals[0]
                 f[i, 2:7] = reals[1:]
-                w[i, 1], w[i, 7], w[i, 8], w[i, 9] = o.top_k, o.repeat_last_n, step, len(h)
+                try:
+                    w[i, 1], w[i, 7], w[i, 8], w[i, 9] = o.top_k, o.repeat_last_n, step, len(h)
+                    w[i, 12:12 + len(h)] = h
+                except OverflowError as e:
+                    raise RuntimeError(f"sampling option or token out of the range of int32: {e}") from e
                 w[i, 10:12] = np.array([seed & MASK64], np.uint64).view(np.int32)
-                w[i, 12:12 + len(h)] = h
                 w[i, 12 + len(h):] = 0
                 self._host_sampler[first + at + i] = (o, list(history), seed, step)
             if self.is_gpu:  # one launch reads the pinned rows and fills every array
@@ -700,6 +705,13 @@ class Runner:
                              "temp", "topk", "topp", "minp", "rpen", "ppen", "fpen", "lastn", "step", "hcount", "seed", "hist")}),
                     stream_handle())
                 self._ring.sent()
+            else:
+                b = slice(first + at, first + at + n)
+                for k, src, c in (("temp", f, 0), ("topk", w, 1), ("topp", f, 2), ("minp", f, 3), ("rpen", f, 4), ("ppen", f, 5),
+                                  ("fpen", f, 6), ("lastn", w, 7), ("step", w, 8), ("hcount", w, 9)):
+                    getattr(self, "s_" + k)[b] = torch.from_numpy(src[:, c])
+                self.s_seed[b] = torch.from_numpy(w[:, 10:12].copy().view(np.int64)[:, 0])
+                self.s_hist[b] = torch.from_numpy(w[:, 12:])
 
     def _sample(self, B: int, feedback: bool = False):
         """feedback (GPU): the sampler's finishing lane of each row also feeds the token back and

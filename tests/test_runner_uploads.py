@@ -9,21 +9,40 @@ from ollama_operator_amd.gguf.constants import FileType
 from ollama_operator_amd.models.config import preset
 from ollama_operator_amd.models.random_init import write_random_gguf
 
-pytestmark = pytest.mark.gpu
-
-
-@pytest.fixture(scope="module")
-def runner(tmp_path_factory):
+def make(tmp_path_factory, device):
     path = str(tmp_path_factory.mktemp("m") / "tiny.gguf")
     write_random_gguf(path, preset("tiny-llama"), FileType.MOSTLY_Q4_0, seed=3)
-    r = Runner(path, device="cuda:0", max_batch=80, max_seqs=3)
+    r = Runner(path, device=device, max_batch=80, max_seqs=3)
     yield r
     r.close()
 
 
-@pytest.mark.parametrize("n,first", [(1, 0), (1, 79), (3, 5), (64, 0), (65, 2), (80, 0)])
+@pytest.fixture(scope="module")
+def runner(tmp_path_factory):
+    yield from make(tmp_path_factory, "cuda:0")
+
+
+@pytest.fixture(scope="module")
+def cpu_runner(tmp_path_factory):
+    yield from make(tmp_path_factory, "cpu")
+
+
+ROWS = [(1, 0), (1, 79), (3, 5), (64, 0), (65, 2), (80, 0)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,first", ROWS)
 def test_sampler_rows(runner, n, first):
-    r, rng = runner, np.random.default_rng(n + first)
+    check_sampler_rows(runner, n, first)
+
+
+@pytest.mark.parametrize("n,first", ROWS)
+def test_sampler_rows_cpu(cpu_runner, n, first):
+    check_sampler_rows(cpu_runner, n, first)
+
+
+def check_sampler_rows(r, n, first):
+    rng = np.random.default_rng(n + first)
     first = min(first, 80 - n)
     r.s_temp.fill_(-1.0)
     rows = [(SamplingOptions(temperature=0.5 + i, top_k=i, top_p=0.25 * (i % 4), min_p=0.01 * i, repeat_penalty=1.0 + i,
@@ -42,10 +61,13 @@ def test_sampler_rows(runner, n, first):
         assert r.s_hist[b].tolist() == h + [0] * (HIST_CAP - len(h))
     others = [b for b in range(80) if not first <= b < first + n]
     assert all(float(r.s_temp[b]) == -1.0 for b in others)
-    with pytest.raises(RuntimeError):
-        r._set_samplers([(SamplingOptions(temperature=1e300), [], 0, 0)])
+    for o, hist, seed in ((dict(temperature=1e300), [], 0), (dict(top_k=1 << 31), [], 0), (dict(repeat_last_n=-(1 << 31) - 1), [], 0),
+                          ({}, [1, 1 << 31], 0), ({}, [], 1 << 64), ({}, [], -(1 << 63) - 1)):
+        with pytest.raises(RuntimeError):  # what the arrays cannot hold
+            r._set_samplers([(SamplingOptions(**o), hist, seed, 0)])
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("B,nt", [(1, 0), (1, 1), (79, 79), (80, 80), (0, 5), (3, 0)])
 def test_step_inputs(runner, B, nt):
     """Uploads in a row that the device has not read yet: each arrives whole and in order."""
