@@ -24,6 +24,9 @@ STACK_SRC = os.path.join(CSRC, "stack")
 BUILD = os.path.join(ROOT, "build", "native")
 ARCH = os.environ.get("OMX_ARCH", "gfx950")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+# HIP device code is compiled without packed-float32 instructions: the compiler forms them from ordinary float code, and
+# some of their forms have given wrong results now and then
+NO_PK_F32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
 
 def _ext_suffix() -> str:
@@ -48,7 +51,7 @@ def _torch_lib() -> str | None:
 
 
 def _headers() -> list[str]:
-    return glob.glob(os.path.join(CSRC, "**", "*.h"), recursive=True)
+    return glob.glob(os.path.join(CSRC, "**", "*.h"), recursive=True) + [os.path.abspath(__file__)]  # and the flags here
 
 
 def _needs(obj: str, src: str, hdr_mtime: float) -> bool:
@@ -92,7 +95,7 @@ def build(jobs: int | None = None, clean: bool = False, verbose: bool = False, d
         objs.append(obj)
         if _needs(obj, s, hdr_mtime):
             if s.endswith(".hip"):
-                cmd = [HIPCC, *common, "-c", s, "-o", obj]
+                cmd = [HIPCC, *common, *NO_PK_F32, "-c", s, "-o", obj]
             else:  # host-only translation unit
                 cmd = [HIPCC, *common, "-x", "c++", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-c", s, "-o", obj,
                        "-fvisibility=hidden"]
@@ -142,11 +145,6 @@ def build(jobs: int | None = None, clean: bool = False, verbose: bool = False, d
 
 def stack_target_path() -> str:
     return os.path.join(ROOT, "ollama_operator_amd", "_stack" + _ext_suffix())
-
-
-# HIP device code is compiled without packed-float32 instructions (the compiler otherwise forms them from
-# ordinary float code)
-NO_PK_F32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
 
 def build_stack(verbose: bool = False, force: bool = False) -> str:

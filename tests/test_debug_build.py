@@ -30,3 +30,18 @@ def test_debug_kernels_compile_with_asserts(tmp_path, monkeypatch):
     if shutil.which("strings"):
         txt = _strings(objs[0]) + _strings(objs[1])
         assert "blk >= 0" in txt and "tile < (w.N + 15) / 16" in txt
+
+
+@pytest.mark.parametrize("debug", [False, True])
+def test_hip_units_compile_without_packed_float32(tmp_path, monkeypatch, debug):
+    """Some packed-float32 instructions have given wrong results now and then: the compiler must not form them."""
+    import sys
+    sys.path.insert(0, ROOT)
+    import build_native
+    cmds = []
+    monkeypatch.setattr(build_native, "BUILD", str(tmp_path / "native"))
+    monkeypatch.setattr(build_native, "DEBUG_BUILD", str(tmp_path / "debug"))
+    monkeypatch.setattr(build_native.subprocess, "run", lambda c, **kw: cmds.append(c) or subprocess.CompletedProcess(c, 0, "", ""))
+    build_native.build(debug=debug, sources=["kernels/attention.hip", "bindings.cpp"], jobs=1)
+    hip, host = cmds
+    assert "-target-feature -Xclang -packed-fp32-ops" in " ".join(hip) and "-packed-fp32-ops" not in host
