@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("D", [64, 80, 96, 112, 128, 256])
 @pytest.mark.parametrize("start,NQ,window,whole", [
     (0, 16, 0, False), (0, 63, 0, False), (0, 65, 0, False), (31, 64, 0, False), (129, 33, 0, False),
-    (0, 577, 0, True), (70, 321, 32, False), (3, 200, 97, False), (0, 1100, 0, False), (0, 16, 0, True)])
+    (0, 577, 0, True), (70, 321, 32, False), (3, 200, 97, False), (0, 1100, 0, False), (0, 16, 0, True), (0, 32, 0, False),
+    (1, 32, 0, False), (15, 17, 0, True), (100, 16, 12, False), (96, 20, 13, False)])
 def test_prefill_attention(D, start, NQ, window, whole):
     """Queries, keys and weights are fp16 with float32 sums: the result is off by a few 2^-11 of its size (3e-3, as for the
     decode kernels); keys and values come from the cache as they are stored."""
