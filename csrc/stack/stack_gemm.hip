@@ -150,26 +150,15 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(const bf16* __res
 // 34 -> 16, 12 x 32,000 x 1,024 22.7 -> 14.0 (four columns of blocks: 29 with one).
 template <int NT, int MT>
 __global__ __launch_bounds__(512) void gemm_rows_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W, int M, int N,
-                                                        int K, Epi e, Group G) {
+                                                        int K, Epi e) {
   __shared__ float red[8][NT * MT][256];
-  int m0 = 0;
-  if (G.tiles) {
-    if ((int)blockIdx.y >= *G.ntiles) return;
-    const int* t = G.tiles + 3 * blockIdx.y;
-    W += (long long)t[0] * G.w_stride;
-    m0 = t[1];
-    M = t[1] + t[2];
-  }
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n0 = blockIdx.x * 16 * NT, fr = lane & 15, fq = lane >> 4;
-  const int mt = (M - m0 + 15) >> 4;  // row tiles of 16
+  const int mt = (M + 15) >> 4;  // row tiles of 16
   const bf16* pa[MT];
   const bf16* pw[NT];
 #pragma unroll
-  for (int i = 0; i < MT; ++i) {
-    const int m = min(m0 + 16 * i + fr, M - 1);
-    pa[i] = A + (long long)(G.gather ? G.gather[m] / G.gdiv : m) * lda + 8 * fq;
-  }
+  for (int i = 0; i < MT; ++i) pa[i] = A + (long long)min(16 * i + fr, M - 1) * lda + 8 * fq;
 #pragma unroll
   for (int j = 0; j < NT; ++j) pw[j] = W + (long long)min(n0 + 16 * j + fr, N - 1) * K + 8 * fq;
   f32x4 acc[MT][NT];
@@ -215,7 +204,7 @@ __global__ __launch_bounds__(512) void gemm_rows_kernel(const bf16* __restrict__
     float v = 0.f;
 #pragma unroll
     for (int w = 0; w < 8; ++w) v += red[w][f][x & 255];
-    const int m = m0 + 16 * (f / NT) + 4 * (l >> 4) + r, nn = n0 + 16 * (f % NT) + (l & 15);
+    const int m = 16 * (f / NT) + 4 * (l >> 4) + r, nn = n0 + 16 * (f % NT) + (l & 15);
     if (m < M && nn < N) epi_store(e, m, nn, v);
   }
 }
@@ -230,21 +219,24 @@ void launch_ring(const Operands& o, const Epi& e, const Group& G, int mtiles, hi
   ring::launch_ring<ring::Bf16, Store, BM, BN, WM, WN, KS, RD, TAIL>(o, Store{e}, G, mtiles, s);
 }
 template <int NT, int MT>
-void launch_rows(const Operands& o, const Epi& e, const Group& G, int mtiles, hipStream_t s) {
-  hipLaunchKernelGGL((gemm_rows_kernel<NT, MT>), dim3((o.N + 16 * NT - 1) / (16 * NT), mtiles), dim3(512), 0, s, (const bf16*)o.A,
-                     o.lda, (const bf16*)o.W, o.M, o.N, o.K, e, G);
+void launch_rows(const Operands& o, const Epi& e, hipStream_t s) {
+  hipLaunchKernelGGL((gemm_rows_kernel<NT, MT>), dim3((o.N + 16 * NT - 1) / (16 * NT)), dim3(512), 0, s, (const bf16*)o.A, o.lda,
+                     (const bf16*)o.W, o.M, o.N, o.K, e);
+}
+// 64 x 64 tiles of four waves, no split of K: many blocks of a few steps each
+void launch_many(const Operands& o, const Epi& e, const Group& G, int mtiles, hipStream_t s) {
+  launch_ring<64, 64, 2, 2, 1, 2, true>(o, e, G, mtiles, s);
 }
 void gemm_plain(const Operands& o, const Epi& e, hipStream_t s) {
   const int M = o.M, N = o.N;
+  if (M <= 16) {
+    if (N >= 4096) launch_rows<4, 1>(o, e, s);
+    else launch_rows<1, 1>(o, e, s);
+    return;
+  }
   if (M <= 64) {
-    if (M <= 16) {
-      if (N >= 4096) launch_rows<4, 1>(o, e, Group{}, 1, s);
-      else launch_rows<1, 1>(o, e, Group{}, 1, s);
-    } else if (N <= 4096) {
-      launch_rows<1, 4>(o, e, Group{}, 1, s);
-    } else {
-      launch_rows<2, 4>(o, e, Group{}, 1, s);
-    }
+    if (N <= 4096) launch_rows<1, 4>(o, e, s);
+    else launch_rows<2, 4>(o, e, s);
     return;
   }
   if (o.K % RG_BK) {
@@ -289,10 +281,13 @@ void gemm_bf16_grouped(const bf16* A, int lda, const bf16* W, int rows, int grou
                        const Group& G, hipStream_t s) {
   check((long long)rows * lda < (1LL << 31) && (long long)N * K < (1LL << 31), "grouped gemm: operands of over 2^31 elements");
   const Operands o{(const uint16_t*)A, lda, (const uint16_t*)W, rows, N, K};
-  if (rows / groups < 48) {
-    launch_rows<1, 4>(o, e, G, max_tiles, s);
-  } else if (gemm_group_tile(rows, groups) == 64) {
-    if (K % RG_BK) launch_ring<64, 64, 2, 1, 4, 4, true>(o, e, G, max_tiles, s);
+  if (gemm_group_tile(rows, groups) == 64) {
+    // few blocks: K split over a block's waves; many (two a CU and more): the lighter blocks. Measured, gate / up and down together,
+    // 100 rows: 8 experts of 1,024 x 2,048, top 2 (256 blocks) 48.0 us split, 49.4 light; 64 of 512 x 1,024, top 8 (1,024 and
+    // more) 62.1 and 57.9. (16-column blocks without LDS, as in gemm_rows_kernel, read every expert's activations too often: 75.7, 130.)
+    const long long blocks = (long long)(rows < groups ? rows : rows / 64 > groups ? rows / 64 : groups) * ((N + 63) / 64);
+    if (blocks > 512) launch_many(o, e, G, max_tiles, s);
+    else if (K % RG_BK) launch_ring<64, 64, 2, 1, 4, 4, true>(o, e, G, max_tiles, s);
     else launch_ring<64, 64, 2, 1, 4, 4, false>(o, e, G, max_tiles, s);
   } else if (K % RG_BK) {
     launch_ring<128, 128, 2, 2, 2, 4, true>(o, e, G, max_tiles, s);

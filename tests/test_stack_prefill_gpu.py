@@ -63,10 +63,10 @@ def test_gemm_tiles(M, N, K):
     assert float((out.double() - 5.0 * torch.tanh(ref / 5.0)).abs().max()) < lim + 1e-5
 
 
-@pytest.mark.parametrize("rows,experts,ff", [(40, 6, 24), (150, 4, 72), (500, 4, 64), (700, 3, 40)])
+@pytest.mark.parametrize("rows,experts,ff", [(40, 6, 24), (150, 4, 72), (500, 4, 64), (700, 3, 40), (60, 40, 448), (200, 40, 424)])
 def test_grouped_experts(tmp_path, rows, experts, ff):
-    """Routed feed-forwards with few, some and many rows per expert (16-row, 64-row and 128-row tiles; K = ff and K = 64 with
-    and without a remainder of 64) against the float64 implementation."""
+    """Routed feed-forwards with few, some and many rows per expert (64-row and 128-row tiles, few and many blocks; K = ff and
+    K = 64 with and without a remainder of 64) against the float64 implementation."""
     m = bc.Model(tmp_path, bc.config([(bc.attn(dim=16, vdim=16), bc.moe(experts=experts, top=2, ff=ff, shared_ff=0))], cap=0.0))
     r = m.runner("cuda", "bfloat16", max_batch=1024, kv_tokens=2048)
     toks = bc.tokens(rows, 96, seed=rows)
