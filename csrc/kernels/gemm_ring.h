@@ -71,8 +71,8 @@ constexpr int ring_lds() { return 2 * (BM + BN) * RG_BK * 2; }  // two buffers o
 // LDS read, products of a step (0.16 us at 64 x 64, 0.40 at 128 x 128, 0.76 at 256 x 128), on full ones the operands' way from
 // L2 and the Infinity Cache (0.45 / 0.62 / 1.09). Measured, 128 x 128 or 64 x 64 tiles without the ring
 // -> now: 2,048^3 47 -> 27 us, 4,096 x 2,048 x 2,048 61 -> 44, 500 x 2,048 x 2,048 26 -> 12, 128 x 7,177 x 2,048 34 -> 15.
-// TAIL: K is no multiple of 64 (the predicate breaks the loop into pieces that each wait for all loads, so the others go
-// without it).
+// TAIL: K is no multiple of 64: the pieces of the last step past K are loaded from K - 8 and zeroed on their way to LDS (a
+// condition around the loads would break the loop into pieces that each wait for all of them).
 // Out: a functor out(m, n, value, value of column n ^ 1).
 template <typename T, typename Out, int BM, int BN, int WM, int WN, int KS, int RD, bool TAIL>
 __global__ __launch_bounds__(64 * WM * WN * KS, BM * BN <= 64 * 64 ? 4 : 2) void gemm_ring_kernel(const uint16_t* __restrict__ A, int lda,
@@ -109,29 +109,30 @@ __global__ __launch_bounds__(64 * WM * WN * KS, BM * BN <= 64 * 64 ? 4 : 2) void
 #pragma unroll
   for (int i = 0; i < AL; ++i) {  // rows past the end repeat the last one (their results are not stored)
     const int m = min(m0 + xr + XR * i, M - 1);
-    oa[i] = 2u * ((unsigned)(G.gather ? G.gather[m] / G.gdiv : m - mb) * (unsigned)lda + 8 * xc);
+    oa[i] = 2u * ((unsigned)(G.gather ? G.gather[m] / G.gdiv : m - mb) * (unsigned)lda + (TAIL ? 0 : 8 * xc));
   }
 #pragma unroll
-  for (int i = 0; i < WL; ++i) ow[i] = 2u * ((unsigned)min(xr + XR * i, N - 1 - n0) * (unsigned)K + 8 * xc);
+  for (int i = 0; i < WL; ++i) ow[i] = 2u * ((unsigned)min(xr + XR * i, N - 1 - n0) * (unsigned)K + (TAIL ? 0 : 8 * xc));
   const int n = (K + RG_BK - 1) / RG_BK;
   u32x4 ra[RD][AL], rw[RD][WL];
   auto load = [&](int step, u32x4 (&a)[AL], u32x4 (&w)[WL]) {
     const int k0 = min(step, n - 1) * RG_BK;  // steps past the end: a repeated load that nobody multiplies
-    const char* ca = (const char*)A + 2 * k0;
-    const char* cw = (const char*)W + 2 * k0;
-    const bool in = !TAIL || k0 + 8 * xc < K;
+    const char* ca = (const char*)A + (TAIL ? 0 : 2 * k0);
+    const char* cw = (const char*)W + (TAIL ? 0 : 2 * k0);
+    const unsigned kc = TAIL ? 2u * min(k0 + 8 * xc, K - 8) : 0u;  // pieces past K: the last one, zeroed on its way to LDS
 #pragma unroll
-    for (int i = 0; i < AL; ++i) a[i] = in ? *(const u32x4*)(ca + oa[i]) : u32x4{0, 0, 0, 0};
+    for (int i = 0; i < AL; ++i) a[i] = *(const u32x4*)(ca + (oa[i] + kc));
 #pragma unroll
-    for (int i = 0; i < WL; ++i) w[i] = in ? *(const u32x4*)(cw + ow[i]) : u32x4{0, 0, 0, 0};
+    for (int i = 0; i < WL; ++i) w[i] = *(const u32x4*)(cw + (ow[i] + kc));
   };
   auto at = [](int r, int c) { return r * RG_BK + 8 * (c ^ ((r >> 1) & 7)); };
-  auto write = [&](const u32x4 (&a)[AL], const u32x4 (&w)[WL], int buf) {
+  auto write = [&](int step, const u32x4 (&a)[AL], const u32x4 (&w)[WL], int buf) {
     uint16_t* d = sm + buf * BUF;
+    const bool past = TAIL && step * RG_BK + 8 * xc >= K;
 #pragma unroll
-    for (int i = 0; i < AL; ++i) *(u32x4*)(d + at(xr + XR * i, xc)) = a[i];
+    for (int i = 0; i < AL; ++i) *(u32x4*)(d + at(xr + XR * i, xc)) = past ? u32x4{0, 0, 0, 0} : a[i];
 #pragma unroll
-    for (int i = 0; i < WL; ++i) *(u32x4*)(d + AS + at(xr + XR * i, xc)) = w[i];
+    for (int i = 0; i < WL; ++i) *(u32x4*)(d + AS + at(xr + XR * i, xc)) = past ? u32x4{0, 0, 0, 0} : w[i];
   };
   f32x16 acc[TM][TN];
 #pragma unroll
@@ -162,7 +163,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS, BM * BN <= 64 * 64 ? 4 : 2) void
   };
 #pragma unroll
   for (int u = 0; u < RD; ++u) load(u, ra[u], rw[u]);
-  write(ra[0], rw[0], 0);
+  write(0, ra[0], rw[0], 0);
   load(RD, ra[0], rw[0]);
   // at step s: LDS buffer s & 1 holds it, registers s + 1 .. s + RD the steps after it; behind the barrier the other buffer's
   // readers are done, the next step goes in and its registers take the step RD later
@@ -171,7 +172,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS, BM * BN <= 64 * 64 ? 4 : 2) void
 #pragma unroll
     for (int u = 0; u < RD; ++u) {
       __syncthreads();
-      write(ra[(u + 1) % RD], rw[(u + 1) % RD], (u + 1) & 1);
+      write(s + u + 1, ra[(u + 1) % RD], rw[(u + 1) % RD], (u + 1) & 1);
       load(s + u + 1 + RD, ra[(u + 1) % RD], rw[(u + 1) % RD]);
       compute(u & 1);
     }
@@ -180,7 +181,7 @@ __global__ __launch_bounds__(64 * WM * WN * KS, BM * BN <= 64 * 64 ? 4 : 2) void
   for (int u = 0; u < RD; ++u) {
     if (s + u < n) {
       __syncthreads();
-      if (s + u + 1 < n) write(ra[(u + 1) % RD], rw[(u + 1) % RD], (u + 1) & 1);
+      if (s + u + 1 < n) write(s + u + 1, ra[(u + 1) % RD], rw[(u + 1) % RD], (u + 1) & 1);
       compute(u & 1);
     }
   }

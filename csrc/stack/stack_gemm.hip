@@ -228,7 +228,8 @@ void launch_many(const Operands& o, const Epi& e, const Group& G, int mtiles, hi
   launch_ring<64, 64, 2, 2, 1, 2, true>(o, e, G, mtiles, s);
 }
 void gemm_plain(const Operands& o, const Epi& e, hipStream_t s) {
-  const int M = o.M, N = o.N;
+    const int M = o.M, N = o.N, K = o.K;
+  const long long b64 = (long long)((M + 63) / 64) * ((N + 63) / 64), b128 = (long long)((M + 127) / 128) * ((N + 127) / 128);
   if (M <= 16) {
     if (N >= 4096) launch_rows<4, 1>(o, e, s);
     else launch_rows<1, 1>(o, e, s);
@@ -239,9 +240,10 @@ void gemm_plain(const Operands& o, const Epi& e, hipStream_t s) {
     else launch_rows<2, 4>(o, e, s);
     return;
   }
-  if (o.K % RG_BK) {
-    if ((long long)((M + 127) / 128) * ((N + 127) / 128) >= 128) launch_ring<128, 128, 2, 2, 2, 4, true>(o, e, Group{}, (M + 127) / 128, s);
-    else launch_ring<64, 64, 2, 1, 4, 4, true>(o, e, Group{}, (M + 63) / 64, s);
+  if (K % RG_BK) {  // (2,048 x 5,000 x 2,056 in this order: 126, 82.7 and 97 us; 1,000 x 4,096 x 2,056: 57, 35 and 32)
+    if (b64 <= 512) launch_ring<64, 64, 2, 1, 4, 4, true>(o, e, Group{}, (M + 63) / 64, s);
+    else if (b128 > 256) launch_ring<128, 128, 2, 2, 1, 2, true>(o, e, Group{}, (M + 127) / 128, s);
+    else launch_ring<128, 128, 2, 2, 2, 4, true>(o, e, Group{}, (M + 127) / 128, s);
     return;
   }
   switch (ring::choose_tile(M, N, o.K, 0)) {
