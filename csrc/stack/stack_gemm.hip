@@ -235,7 +235,9 @@ void gemm_plain(const Operands& o, const Epi& e, hipStream_t s) {
     else launch_rows<1, 1>(o, e, s);
     return;
   }
-  if (M <= 64) {
+  // 17 .. 64 rows: each block of the row kernel reads all activations, which many columns (blocks) pay for. K = 2,048, rows against
+  // tiles: 33 rows x 7,177 columns 13.0 and 14.2 us, x 11,264 23.2 and 15.2; 64 rows 17.1 and 15.7, 30.4 and 16.8, x 32,000 59.6 and 31.8
+  if (M <= 64 && N < 8192) {
     if (N <= 4096) launch_rows<1, 4>(o, e, s);
     else launch_rows<2, 4>(o, e, s);
     return;
