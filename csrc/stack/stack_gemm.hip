@@ -1,9 +1,10 @@
 // bfloat16 matrix products of prompt portions and of decode steps with more than 8 rows: C[M][N] = epi(A[M][K] . W[N][K]^T),
 // plain or grouped by expert (Group, stack_device.h). K % 8 == 0 and 16-byte aligned rows (checked by the callers).
-// float32 accumulation in all of them; only the order of the sums differs. Three kernels:
+// float32 accumulation in all of them; only the order of the sums differs. Four kernels:
 //   gemm_pingpong_kernel  256 x 256 tiles, two groups of four waves in turns at the LDS and at the matrix cores
 //   gemm_ring_kernel      256 x 128 .. 64 x 64 tiles, loads several steps ahead in registers (csrc/kernels/gemm_ring.h)
 //   gemm_rows_kernel      up to 64 rows: weights straight from memory, K split over a block's waves
+//   gemm_short_kernel     K of a few hundred and less
 #include "../kernels/gemm_ring.h"
 #include "stack_device.h"
 
@@ -209,6 +210,84 @@ __global__ __launch_bounds__(512) void gemm_rows_kernel(const bf16* __restrict__
   }
 }
 
+// ---- K of a few steps (gemm_plain): 64 x 64 or 128 x 128 tiles of four waves, 32 of K a step, one step of look-ahead. With nothing to
+// overlap, a launch lasts as long as its fixed part: few threads, few registers to fill, no shares of K to add up. Measured
+// against the other kernels here: 300 x 1,024 x 64 4.1 against 5.1 us, 2,048 x 5,000 x 200 19.7 against 29.5.
+constexpr int SH_BK = 32, SH_LD = 40;  // LDS rows padded to 40 elements: 32 rows' 16-byte reads spread over the banks
+template <int TM, int TN>
+__global__ __launch_bounds__(256) void gemm_short_kernel(const bf16* __restrict__ A, int lda, const bf16* __restrict__ W, int M, int N,
+                                                         int K, Epi e) {
+  constexpr int BM = 64 * TM, BN = 64 * TN;
+  __shared__ __attribute__((aligned(16))) uint16_t As[2][BM * SH_LD];
+  __shared__ __attribute__((aligned(16))) uint16_t Ws[2][BN * SH_LD];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave >> 1, wn = wave & 1, fr = lane & 31, fq = lane >> 5;
+  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+  const int sr = tid >> 2, sk = (tid & 3) * 8;  // staging: 4 threads per row, 64 rows per pass
+  u32x4 ra[TM], rw[TN];
+  auto fetch = [&](int k0) {
+    const int k = k0 + sk;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int m = m0 + sr + 64 * i;
+      ra[i] = (m < M && k < K) ? *(const u32x4*)(A + (long long)m * lda + k) : u32x4{0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int n = n0 + sr + 64 * j;
+      rw[j] = (n < N && k < K) ? *(const u32x4*)(W + (long long)n * K + k) : u32x4{0, 0, 0, 0};
+    }
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) *(u32x4*)(&As[buf][(sr + 64 * i) * SH_LD + sk]) = ra[i];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) *(u32x4*)(&Ws[buf][(sr + 64 * j) * SH_LD + sk]) = rw[j];
+  };
+  f32x16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  fetch(0);
+  stage(0);
+  __syncthreads();
+  int buf = 0;
+  for (int k0 = 0; k0 < K; k0 += SH_BK) {
+    const bool more = k0 + SH_BK < K;
+    if (more) fetch(k0 + SH_BK);
+#pragma unroll
+    for (int kk = 0; kk < SH_BK / 16; ++kk) {
+      bf16x8 a[TM], b[TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) a[i] = *(const bf16x8*)(&As[buf][(wm * 32 * TM + 32 * i + fr) * SH_LD + kk * 16 + fq * 8]);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) b[j] = *(const bf16x8*)(&Ws[buf][(wn * 32 * TN + 32 * j + fr) * SH_LD + kk * 16 + fq * 8]);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+    }
+    if (more) stage(buf ^ 1);  // the other buffer's readers finished before the previous barrier
+    __syncthreads();
+    buf ^= 1;
+  }
+  // C fragment: as in the kernels above
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int n = n0 + wn * 32 * TN + 32 * j + fr;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int m = m0 + wm * 32 * TM + 32 * i + (r & 3) + 8 * (r >> 2) + 4 * fq;
+        if (m < M && n < N) epi_store(e, m, n, acc[i][j][r]);
+      }
+    }
+}
+
 struct Store {
   Epi e;
   __device__ __forceinline__ void operator()(int m, int n, float v, float) const { epi_store(e, m, n, v); }
@@ -223,16 +302,29 @@ void launch_rows(const Operands& o, const Epi& e, hipStream_t s) {
   hipLaunchKernelGGL((gemm_rows_kernel<NT, MT>), dim3((o.N + 16 * NT - 1) / (16 * NT)), dim3(512), 0, s, (const bf16*)o.A, o.lda,
                      (const bf16*)o.W, o.M, o.N, o.K, e);
 }
+template <int TM, int TN>
+void launch_short(const Operands& o, const Epi& e, hipStream_t s) {
+  hipLaunchKernelGGL((gemm_short_kernel<TM, TN>), dim3((o.N + 64 * TN - 1) / (64 * TN), (o.M + 64 * TM - 1) / (64 * TM)), dim3(256), 0, s,
+                     (const bf16*)o.A, o.lda, (const bf16*)o.W, o.M, o.N, o.K, e);
+}
 // 64 x 64 tiles of four waves, no split of K: many blocks of a few steps each
 void launch_many(const Operands& o, const Epi& e, const Group& G, int mtiles, hipStream_t s) {
   launch_ring<64, 64, 2, 2, 1, 2, true>(o, e, G, mtiles, s);
 }
 void gemm_plain(const Operands& o, const Epi& e, hipStream_t s) {
-    const int M = o.M, N = o.N, K = o.K;
+  const int M = o.M, N = o.N, K = o.K;
   const long long b64 = (long long)((M + 63) / 64) * ((N + 63) / 64), b128 = (long long)((M + 127) / 128) * ((N + 127) / 128);
   if (M <= 16) {
     if (N >= 4096) launch_rows<4, 1>(o, e, s);
     else launch_rows<1, 1>(o, e, s);
+    return;
+  }
+  // short K: up to 64 rows the row kernel is level from K = 72 (17 rows x 1,024 columns 3.9 us both), the tiles below from 264, on
+  // two and more waves of blocks from 384 (2,048 x 4,096 x 320 18.0 against 18.8 us), with a remainder from 584 (2,048 x 5,000 x 520
+  // 29.3 against 31.5)
+  if (K <= (M <= 64 ? 64 : b128 < 512 ? 256 : K % RG_BK ? 520 : 320)) {
+    if (b128 >= 256) launch_short<2, 2>(o, e, s);
+    else launch_short<1, 1>(o, e, s);
     return;
   }
   // 17 .. 64 rows: each block of the row kernel reads all activations, which many columns (blocks) pay for. K = 2,048, rows against
@@ -240,6 +332,10 @@ void gemm_plain(const Operands& o, const Epi& e, hipStream_t s) {
   if (M <= 64 && N < 8192) {
     if (N <= 4096) launch_rows<1, 4>(o, e, s);
     else launch_rows<2, 4>(o, e, s);
+    return;
+  }
+  if (K < 512) {  // up to seven steps: 1,000 x 5,000 x 320 13.6 us, 22.0 on the model's choice
+    launch_many(o, e, Group{}, (M + 63) / 64, s);
     return;
   }
   if (K % RG_BK) {  // (2,048 x 5,000 x 2,056 in this order: 126, 82.7 and 97 us; 1,000 x 4,096 x 2,056: 57, 35 and 32)
