@@ -232,13 +232,15 @@ void launch_ring(const Operands& o, const Out& out, const Group& G, int mtiles, 
   hipLaunchKernelGGL((gemm_ring_kernel<T, Out, BM, BN, WM, WN, KS, RD, TAIL>), dim3(grid), dim3(64 * WM * WN * KS), (ring_lds<BM, BN>()), s,
                      o.A, o.lda, o.W, o.M, o.N, o.K, out, G, mtiles);
 }
-// The tile with the least time by a model of measured steps: a launch and its first and last step cost `fixed`, a step of 64 K
-// c0 while few blocks run and c1 on a full chip (us; 14 shapes of 128 .. 4096 rows, within 15 %). Tile 0 is the 256 x 256
-// ping-pong kernel, for callers that have it.
+// The tile with the least time by a model of measured steps: a launch with its first and last step costs `fixed`, every further
+// wave of blocks `again`, a step of 64 K c0 while few blocks run and c1 on a full chip (us). Over 65 .. 4,096 rows x 256 .. 32,000
+// columns x K = 512 .. 5,632 (700 shapes, all tiles timed) the choice is 1.0 % from the best on average; without `again` 2.6 %, and
+// up to 1.45 times the best where a few steps of K meet several waves (1,500 x 5,632 x 512: 37.2 -> 24.8 us). Tile 0 is the
+// 256 x 256 ping-pong kernel, for callers that have it.
 inline int choose_tile(int M, int N, int K, int first) {
-  struct Tile { int bm, bn, slots; double fixed, c0, c1; };
-  static const Tile tiles[6] = {{256, 256, 256, 12.0, 1.03, 1.95}, {256, 128, 256, 8.0, 0.76, 1.09}, {128, 128, 256, 7.0, 0.40, 0.62},
-                                {128, 128, 512, 7.0, 0.45, 1.25},  {128, 64, 256, 6.3, 0.275, 0.36}, {64, 64, 512, 5.5, 0.16, 0.45}};
+  struct Tile { int bm, bn, slots; double fixed, again, c0, c1; };
+  static const Tile tiles[6] = {{256, 256, 256, 12.0, 4.0, 1.03, 1.95}, {256, 128, 256, 8.0, 5.0, 0.76, 1.09}, {128, 128, 256, 7.0, 6.0, 0.40, 0.62},
+                                {128, 128, 512, 7.0, 2.0, 0.45, 1.25},  {128, 64, 256, 6.3, 3.0, 0.275, 0.36}, {64, 64, 512, 5.5, 2.0, 0.16, 0.45}};
   const int n = (K + RG_BK - 1) / RG_BK;
   int best = first;
   double least = 0.0;
@@ -246,7 +248,7 @@ inline int choose_tile(int M, int N, int K, int first) {
     const Tile& t = tiles[i];
     const double blocks = (double)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
     const double waves = (double)(long long)((blocks + t.slots - 1) / t.slots), fill = blocks < t.slots ? blocks / t.slots : 1.0;
-    const double us = t.fixed + waves * n * (t.c0 + (t.c1 - t.c0) * fill);
+    const double us = t.fixed + (waves - 1) * t.again + waves * n * (t.c0 + (t.c1 - t.c0) * fill);
     if (i == first || us < least) best = i, least = us;
   }
   return best;
