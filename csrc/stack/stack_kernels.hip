@@ -1048,7 +1048,7 @@ struct FlashLds {
   static constexpr int LDK = 16 * KD + 8;                            // halves; 16-byte rows offset by 4 banks
   static constexpr int VROW = (32 * NV + 127) / 128 * 256;           // bytes
   static constexpr int KB = FL_KEYS * LDK * 2, BUF = KB + FL_KEYS * VROW;
-  static constexpr int MERGE = 2 * (16 * NV + 2) * 64 * 4;           // the odd groups' outputs, maxima and sums
+  static constexpr int MERGE = 2 * (16 * NV + 4) * 64 * 4;           // the odd groups' outputs, maxima and sums
   static constexpr int BYTES = 2 * BUF > MERGE ? 2 * BUF : MERGE;    // then the tiles' pool rows
   static constexpr int ALL = BYTES + 2 * 2 * FL_KEYS * 4;
 };
@@ -1247,23 +1247,35 @@ __global__ __launch_bounds__(256, (KD <= 8 && NV <= 4) ? 2 : 1) void flash_prefi
       }
     }
   }
-  // the odd groups' share joins the even groups' (the tiles' buffers are free once everybody is here)
-  __syncthreads();
-  float* mg = (float*)flash_smem + (qw * (16 * NV + 2)) * 64 + lane;
-  if (set == 1) {
-    mg[0] = mi;
-    mg[64] = li;
+  // the odd groups' share, if there is one, joins the even groups' (the tiles' buffers are free once everybody is here)
+  if (kmax - kmin > 32) {
+    __syncthreads();
+    f32x4* mg = (f32x4*)flash_smem + (qw * (4 * NV + 1)) * 64 + lane;
+    if (set == 1) {
+      mg[0] = f32x4{mi, li, 0.f, 0.f};
 #pragma unroll
-    for (int j = 0; j < NV; ++j)
+      for (int j = 0; j < NV; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) mg[64 * (2 + 16 * j + r)] = o[j][r];
+        for (int k = 0; k < 4; ++k) mg[64 * (1 + 4 * j + k)] = f32x4{o[j][4 * k], o[j][4 * k + 1], o[j][4 * k + 2], o[j][4 * k + 3]};
+    }
+    __syncthreads();
+    if (set == 0) {
+      const float m1 = mg[0][0], mn = fmaxf(mi, m1);
+      const float c0 = __builtin_amdgcn_exp2f(fmaxf(mi - mn, -140.f)), c1 = __builtin_amdgcn_exp2f(fmaxf(m1 - mn, -140.f));
+      li = li * c0 + mg[0][1] * c1;
+      mi = mn;
+#pragma unroll
+      for (int j = 0; j < NV; ++j)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const f32x4 w = mg[64 * (1 + 4 * j + k)];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[j][4 * k + i] = o[j][4 * k + i] * c0 + w[i] * c1;
+        }
+    }
   }
-  __syncthreads();
   if (set == 0 && qi < nrows) {  // register r of tile j: value dim 32 j + (r & 3) + 8 (r >> 2) + 4 hf of this lane's query
-    const float m1 = mg[0], mn = fmaxf(mi, m1);
-    const float c0 = __builtin_amdgcn_exp2f(fmaxf(mi - mn, -140.f)), c1 = __builtin_amdgcn_exp2f(fmaxf(m1 - mn, -140.f));
-    li = li * c0 + mg[64] * c1;
-    if (P.sink) li += __builtin_amdgcn_exp2f(P.sink[h] * 1.44269504088896341f - mn);  // a term of the denominator without key or value
+    if (P.sink) li += __builtin_amdgcn_exp2f(P.sink[h] * 1.44269504088896341f - mi);  // a term of the denominator without key or value
     const float inv = attn_head_gate(P, qrow, h) / li;
     float* out32 = P.out32 ? P.out32 + (long long)qrow * P.ld_out32 + oh * DV : nullptr;
     bf16* out = P.out32 ? nullptr : (bf16*)P.out + (long long)qrow * P.ld_out + oh * DV;
@@ -1274,7 +1286,7 @@ __global__ __launch_bounds__(256, (KD <= 8 && NV <= 4) ? 2 : 1) void flash_prefi
       for (int k = 0; k < 4; ++k) {
         float v[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = (o[j][4 * k + i] * c0 + mg[64 * (2 + 16 * j + 4 * k + i)] * c1) * inv;
+        for (int i = 0; i < 4; ++i) v[i] = o[j][4 * k + i] * inv;
         const int d = 32 * j + 8 * k + 4 * hf;
         if (out32) {
 #pragma unroll
