@@ -769,57 +769,68 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(AttnParams P, Ste
   const long long ldk = P.ldk ? P.ldk : P.D, ldv = P.ldv ? P.ldv : P.Dv;
   const int kq = lane >> 4, dq = lane & 15;
   const float slope = P.slopes ? P.slopes[h] : 0.f;
-  const float hgate = P.hgate ? P.hgate[(long long)b * P.ld_hgate + h] : 0.f, sink = P.sink ? P.sink[h] : 0.f;
+  // keys (and 16-bit values) ahead of their turn only where the registers hold them: with wide values or float32 past 64 dims the
+  // loads ahead cost more than they hide (float32, 4 rows of 16 heads of 128 on 300 keys 15.2 -> 17.0 us; of 64 19.0 -> 12.9)
+  constexpr bool AHEAD = DPL * sizeof(T) <= 16, EARLY = AHEAD && sizeof(T) == 2;
+  const float hgate = AHEAD && P.hgate ? P.hgate[(long long)b * P.ld_hgate + h] : 0.f, sink = AHEAD && P.sink ? P.sink[h] : 0.f;
   float m = -INFINITY, l = 0.f, acc[DPL];
 #pragma unroll
   for (int c = 0; c < DPL; ++c) acc[c] = 0.f;
   const int lo = attn_first_key(P, n);  // the row sees the keys lo .. n - 1
   int t0 = lo + 64 * (split * 4 + wv);
   auto find = [&](int t) { return bt[max(min(t, n - 1), 0) / R.bs]; };  // lanes past the end: the last key, with weight 0
-  int blk = t0 < n ? find(t0 + lane) : 0;
+  int blk = AHEAD && t0 < n ? find(t0 + lane) : 0;
   __syncthreads();
   for (; t0 < n; t0 += 256 * nsplit) {
-    const int t = t0 + lane, tc = min(t, n - 1);
+    const int t = t0 + lane;
     const bool valid = t < n;
-    const int off = tc % R.bs;
-    rs[wv][lane] = (blk * P.G + gv) * R.bs + off;  // the value's row; the key's may sit in a pool of another shape
-    const T* kr = kc + (long long)((blk * KG + kg) * R.bs + off) * ldk + koff;
-    if (t0 + 256 * nsplit < n) blk = find(t + 256 * nsplit);
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's LDS writes have landed
-    constexpr bool EARLY = sizeof(T) == 2 && DPL <= 8;
-    uint32_t raw[EARLY ? 16 : 1][DPL / 2];
-    if constexpr (EARLY) {
-      if (vvec) {
-        const int d = min(dq * DPL, P.Dv - DPL);  // lanes past the last dim repeat it; nobody stores theirs
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const T* vr = vc + (long long)rs[wv][kq * 16 + i] * ldv + d;
-          typedef uint32_t piece __attribute__((ext_vector_type(DPL / 2)));
-          const piece w = *(const piece*)vr;
-#pragma unroll
-          for (int c = 0; c < DPL / 2; ++c) raw[i][c] = w[c];
-        }
-      }
-    }
     float dot = 0.f;
-    if (vec) {
-      for (int d0 = 0; d0 < P.D; d0 += 64) {
-        float k8[8][8];
+    auto score = [&](const T* kr) {
+      if (vec) {
+        for (int d0 = 0; d0 < P.D; d0 += 64) {
+          float k8[8][8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) load8<T>(kr + min(d0 + 8 * u, P.D - 8), k8[u]);
+          for (int u = 0; u < 8; ++u) load8<T>(kr + min(d0 + 8 * u, P.D - 8), k8[u]);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const int d = d0 + 8 * u;
-          if (d < P.D) {
-            const f32x4 qa = *(const f32x4*)&qs[d], qb = *(const f32x4*)&qs[d + 4];
-            dot += qa[0] * k8[u][0] + qa[1] * k8[u][1] + qa[2] * k8[u][2] + qa[3] * k8[u][3] + qb[0] * k8[u][4] +
-                   qb[1] * k8[u][5] + qb[2] * k8[u][6] + qb[3] * k8[u][7];
+          for (int u = 0; u < 8; ++u) {
+            const int d = d0 + 8 * u;
+            if (d < P.D) {
+              const f32x4 qa = *(const f32x4*)&qs[d], qb = *(const f32x4*)&qs[d + 4];
+              dot += qa[0] * k8[u][0] + qa[1] * k8[u][1] + qa[2] * k8[u][2] + qa[3] * k8[u][3] + qb[0] * k8[u][4] +
+                     qb[1] * k8[u][5] + qb[2] * k8[u][6] + qb[3] * k8[u][7];
+            }
+          }
+        }
+      } else {
+        for (int d = 0; d < P.D; ++d) dot += qs[d] * ld(kr + d);
+      }
+    };
+    uint32_t raw[EARLY ? 16 : 1][DPL / 2];
+    const int off = min(t, n - 1) % R.bs;
+    if constexpr (AHEAD) {
+      rs[wv][lane] = (blk * P.G + gv) * R.bs + off;  // the value's row; the key's may sit in a pool of another shape
+      const T* kr = kc + (long long)((blk * KG + kg) * R.bs + off) * ldk + koff;
+      if (t0 + 256 * nsplit < n) blk = find(t + 256 * nsplit);
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's LDS writes have landed
+      if constexpr (EARLY) {
+        if (vvec) {
+          const int d = min(dq * DPL, P.Dv - DPL);  // lanes past the last dim repeat it; nobody stores theirs
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const T* vr = vc + (long long)rs[wv][kq * 16 + i] * ldv + d;
+            typedef uint32_t piece __attribute__((ext_vector_type(DPL / 2)));
+            const piece w = *(const piece*)vr;
+#pragma unroll
+            for (int c = 0; c < DPL / 2; ++c) raw[i][c] = w[c];
           }
         }
       }
+      score(kr);
     } else {
-      for (int d = 0; d < P.D; ++d) dot += qs[d] * ld(kr + d);
+      blk = find(t);  // (the last key again for lanes past the end, with weight 0)
+      if (valid) score(kc + (long long)((blk * KG + kg) * R.bs + off) * ldk + koff);
+      rs[wv][lane] = (blk * P.G + gv) * R.bs + off;
     }
     float sc = -INFINITY;
     if (valid) {
@@ -910,8 +921,8 @@ __global__ __launch_bounds__(256) void attention_decode_kernel(AttnParams P, Ste
       if (dq * DPL + c < P.Dv) w[2 + dq * DPL + c] = acc[c];
     return;
   }
-  if (P.sink) L += expf(sink - M);
-  const float inv = (P.hgate ? P.out_scale * sigmoidf(hgate) : 1.f) / L;
+  if (P.sink) L += expf((AHEAD ? sink : P.sink[h]) - M);
+  const float inv = (!AHEAD ? attn_head_gate(P, b, h) : P.hgate ? P.out_scale * sigmoidf(hgate) : 1.f) / L;
   if (P.out32) {
     float* out = P.out32 + (long long)b * P.ld_out32 + oh * P.Dv;
 #pragma unroll
