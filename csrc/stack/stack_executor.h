@@ -205,6 +205,7 @@ class StackExecutor {
   StackInputs in;
   const int* tiles = nullptr;  // attention query tiles of the NEXT step {first row, rows}, n_tiles of them (0: none)
   int n_tiles = 0, max_tiles = 0;
+  bool on_tiles(const AttnParams& A, int B) const;  // whether a step's attention runs on query tiles (flash_prefill)
   int n_splits = 1;        // blocks per (row, head) of the NEXT steps' decode attention (long contexts)
   bool h_ready = false;    // ws.h holds the stream's rows in the matrix dtype (layers with output norms)
   int n_chunks = 0;        // chunks in ws.ret.chunks for the NEXT step (0: none bound, retention runs token by token)

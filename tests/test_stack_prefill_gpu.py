@@ -91,3 +91,20 @@ def test_decode_attention(tmp_path, dim, vdim, dtype):
         got = bc.run_cuts(r, toks[:n], [n] if n == 1 else [n - 1, n])
         e = bc.rel_err(got[-1:], want[n - 1:n])
         assert e.max() < (1e-2 if dtype == "bfloat16" else 1e-4), f"{n} keys: off by {e.max():.3g}"
+
+
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (192, 64), (256, 128), (192, 160)])
+def test_many_single_rows(tmp_path, dim, vdim):
+    """A step of 20 sequences with a row each (decode steps of more than 16 users), short and long contexts side by side: on query
+    tiles, or wide keys on a block per row and head. Limits as for the prompts."""
+    m = bc.Model(tmp_path, bc.config([(bc.attn(heads=4, kv_heads=2, dim=dim, vdim=vdim, scale=dim ** -0.5), None)], cap=0.0))
+    r = m.runner("cuda", "bfloat16", max_batch=512, max_seqs=20, kv_tokens=4096)
+    toks = bc.tokens(300, 96, seed=dim + vdim)
+    want, _ = m.oracle(toks)
+    ctx = [1, 2, 31, 32, 33, 63, 64, 65, 299] + list(range(100, 111))
+    ids = [r.new_sequence() for _ in ctx]
+    for i, n in zip(ids, ctx):
+        r.step_entries([(i, toks[:n], [])])
+    out = r.step_entries([(i, [toks[n]], [0]) for i, n in zip(ids, ctx)]).float().cpu().numpy()
+    e = bc.rel_err(out, want[ctx])
+    assert e.max() < 1e-2, f"{ctx[int(e.argmax())]} keys: off by {e.max():.3g}"
