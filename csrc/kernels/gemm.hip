@@ -565,9 +565,9 @@ static bool lib_glu() {
 
 void set_gemm_lib_min_m(int m) { g_lib_min_m = m; }
 
-// MoE prefill (default 256 pairs = 128 tokens at top-2): the per-expert GEMMs are plain dense GEMMs over
-// contiguous sorted rows, and the grouped tile kernel (moe_gemm) they replace has no register-ring
-// edition -- Mixtral's 2048-token TTFT is 196 ms on it vs 116 ms per expert on hipBLASLt (profiles/r6_models)
+// MoE prefill of the experts that the grouped register-ring launches do not take (gemm_dq.hip moe_grouped; default 256
+// pairs = 128 tokens at top-2): the per-expert GEMMs are plain dense GEMMs over contiguous sorted rows, ahead of the
+// grouped tile kernel (moe_gemm) -- Mixtral's 2048-token TTFT was 196 ms on that and 116 ms per expert on hipBLASLt
 static int g_moe_lib_min_m = -1;
 int moe_lib_min_m() {
   if (g_moe_lib_min_m < 0) {

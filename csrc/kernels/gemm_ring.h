@@ -235,7 +235,7 @@ void launch_ring(const Operands& o, const Out& out, const Group& G, int mtiles, 
 // The tile with the least time by a model of measured steps: a launch with its first and last step costs `fixed`, every further
 // wave of blocks `again`, a step of 64 K c0 while few blocks run and c1 on a full chip (us). Over 65 .. 4,096 rows x 256 .. 32,000
 // columns x K = 512 .. 5,632 (700 shapes, all tiles timed) the choice is 1.0 % from the best on average; without `again` 2.6 %, and
-// up to 1.45 times the best where a few steps of K meet several waves (1,500 x 5,632 x 512: 37.2 -> 24.8 us). Tile 0 is the
+// up to 1.45 times the best where a few steps of K meet several waves (1,500 x 5,632 x 512: 37.2 -> 19.8 us). Tile 0 is the
 // 256 x 256 ping-pong kernel, for callers that have it.
 inline int choose_tile(int M, int N, int K, int first) {
   struct Tile { int bm, bn, slots; double fixed, again, c0, c1; };

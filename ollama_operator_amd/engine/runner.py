@@ -129,9 +129,9 @@ def kv_cache_type() -> str:
 
 class PinnedRing:
     """Pinned host buffers that uploads pass through. `take(words)` hands out the next one (int32 words) once the
-    copies that read it last are done; `sent()` marks the copies issued since. Uploads then neither wait for the
-    stream (as copies from pageable memory do) nor overwrite what a copy still reads. Used by one thread at a time,
-    like the runner that owns it."""
+    copies that read it last are done; `sent()` marks the copies issued since. Up to `slots` uploads in a row then
+    do not wait for the stream (as copies from pageable memory do), one more waits for the oldest of them; none
+    overwrites what a copy still reads. Used by one thread at a time, like the runner that owns it."""
 
     def __init__(self, words: int, slots: int = 8):
         self.bufs = [torch.zeros(words, dtype=torch.int32, pin_memory=True) for _ in range(slots)]
@@ -790,7 +790,7 @@ class Runner:
         # short prompts through the prefill path (GEMM + prep/finalize kernels resolved once); one per
         # hipBLASLt M bucket too -- a bucket's first GEMM also loads its kernel's code object (~0.1 s),
         # which must not land in a request's TTFT
-        lens = [min(self.max_batch, 32), min(self.max_batch, 128)]  # the tile and the dq GEMM paths
+        lens = [min(self.max_batch, 32), min(self.max_batch, 128)]  # gemm_rows.hip and gemm_dq.hip
         if self.w16 is not None and self.lib_min > 0:
             m = self.lib_min
             while m <= min(self.max_batch, self.ctx - 1):  # every hipBLASLt M bucket (blas.cpp bucket_of)

@@ -1,7 +1,7 @@
 """GPU numerics of the prefill MFMA dequant GEMM paths: the same `gemv` entry with an fp16 activation
 workspace and B >= GEMM_MIN_B, against a plain fp32 PyTorch reference on the dequantised weights.
-path "dq": the stream-order kernel (csrc/kernels/gemm_dq.hip, the default from 128 rows); "old": the
-128 x 128 natural-order tile (gemm.hip, below 128 rows); "lib": hipBLASLt (the oracle / A-B baseline).
+path "dq": the stream-order kernels (csrc/kernels/gemm_dq.hip, the default from 65 rows, gemm_rows.hip below); "old": the
+128 x 128 natural-order tile (gemm.hip); "lib": hipBLASLt (the oracle / A-B baseline).
 Covers every quant type, partial M/N tiles, K padding (Q4_0/Q8_0 with K % 256 != 0), split-K and
 every fused epilogue."""
 import math
@@ -19,7 +19,7 @@ def gemm(m, x, norm=0, nw=None, nb=None, epi=0, y=None, bias=None, extra=None, e
          path="old"):
     """split=True gives the kernel a split-K workspace (small M then runs split-K + finalize).
     lib=True: the hipBLASLt path (dequantised fp16 weight scratch + fp32 slab) from M = 16 on.
-    path: "dq" enables the stream-order kernel (gemm_dq.hip, B >= 128), "old" disables it."""
+    path: "dq" enables the stream-order kernels (gemm_dq.hip, gemm_rows.hip), "old" disables them."""
     B, K = x.shape
     Kp = (K + 255) // 256 * 256
     xws = torch.empty(B * Kp, device="cuda", dtype=torch.float16)
