@@ -314,7 +314,8 @@ PYBIND11_MODULE(_C, m) {
   m.def("moe_lib_min_m", &moe_lib_min_m);
   m.def("moe_grouped", [](py::object gu, py::object down) { return moe_grouped(qmat(gu), qmat(down)); },
         "whether a layer's routed experts take the grouped launches (gemm_dq_moe.hip) for prompts");
-  m.def("set_dq_gemm", &set_dq_gemm, "1: prefill GEMMs on the stream-order dequant kernels (gemm_dq.hip from 65 rows, gemm_rows.hip from 16)");
+  m.def("set_dq_gemm", &set_dq_gemm,
+        "1: prefill GEMMs on the stream-order dequant kernels (gemm_dq.hip from 65 rows, gemm_rows.hip from 16)");
   m.def("set_dq_tuning", &set_dq_tuning, "microbenchmarks: force the dq GEMM tile config (0..3, -1 auto) and split-K factor (0 auto)");
   m.def("dq_gemm_enabled", &dq_gemm_enabled);
   m.def("set_gemv8_geo", [](int nsb, int ks) { set_gemv8_geo(nsb, ks); });

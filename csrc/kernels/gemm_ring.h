@@ -239,8 +239,9 @@ void launch_ring(const Operands& o, const Out& out, const Group& G, int mtiles, 
 // 256 x 256 ping-pong kernel, for callers that have it.
 inline int choose_tile(int M, int N, int K, int first) {
   struct Tile { int bm, bn, slots; double fixed, again, c0, c1; };
-  static const Tile tiles[6] = {{256, 256, 256, 12.0, 4.0, 1.03, 1.95}, {256, 128, 256, 8.0, 5.0, 0.76, 1.09}, {128, 128, 256, 7.0, 6.0, 0.40, 0.62},
-                                {128, 128, 512, 7.0, 2.0, 0.45, 1.25},  {128, 64, 256, 6.3, 3.0, 0.275, 0.36}, {64, 64, 512, 5.5, 2.0, 0.16, 0.45}};
+  static const Tile tiles[6] = {{256, 256, 256, 12.0, 4.0, 1.03, 1.95}, {256, 128, 256, 8.0, 5.0, 0.76, 1.09},
+                                {128, 128, 256, 7.0, 6.0, 0.40, 0.62},  {128, 128, 512, 7.0, 2.0, 0.45, 1.25},
+                                {128, 64, 256, 6.3, 3.0, 0.275, 0.36},  {64, 64, 512, 5.5, 2.0, 0.16, 0.45}};
   const int n = (K + RG_BK - 1) / RG_BK;
   int best = first;
   double least = 0.0;

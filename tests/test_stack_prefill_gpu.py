@@ -38,9 +38,10 @@ def test_flash_prefill_tile_edges(tmp_path, dim, heads, kv, cap):
 # at 17 .. 64 rows, to 256 above) in small and large tiles; up to 511, and no multiple of 64 beyond; few rows of many columns
 GEMMS = [(9, 1, 8), (16, 4100, 264), (16, 40, 72), (17, 33, 2048), (64, 4100, 1032), (64, 15, 96), (65, 64, 64), (65, 65, 72),
          (100, 700, 192), (129, 1024, 704), (300, 3600, 1024), (500, 7177, 2048), (1000, 2048, 2048), (1030, 7177, 2048),
-         (2000, 7177, 2112), (2048, 1030, 200), (4096, 2048, 1088), (17, 70, 8), (64, 4100, 64), (33, 65, 72), (65, 100, 8), (70, 1030, 256),
-         (2050, 4100, 40), (2048, 4096, 256), (65, 33, 264), (1030, 4100, 320), (64, 8200, 448), (66, 130, 504), (65, 40, 520), (1030, 4100, 1032),
-         (3000, 700, 584), (2050, 2100, 520), (17, 8192, 512), (64, 8200, 1088), (33, 9000, 72), (50, 8193, 64)]
+         (2000, 7177, 2112), (2048, 1030, 200), (4096, 2048, 1088), (17, 70, 8), (64, 4100, 64), (33, 65, 72), (65, 100, 8),
+         (70, 1030, 256), (2050, 4100, 40), (2048, 4096, 256), (65, 33, 264), (1030, 4100, 320), (64, 8200, 448), (66, 130, 504),
+         (65, 40, 520), (1030, 4100, 1032), (3000, 700, 584), (2050, 2100, 520), (17, 8192, 512), (64, 8200, 1088), (33, 9000, 72),
+         (50, 8193, 64)]
 
 
 @pytest.mark.parametrize("M,N,K", GEMMS)
