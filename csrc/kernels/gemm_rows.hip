@@ -131,7 +131,8 @@ void run_rows(const GemvParams& P, f16* xp, int Kp, hipStream_t s) {
   const int N = P.w.N;
   // columns per block by what still leaves a block for most CUs (Q4_K, 48 rows: N = 22016 43 us at 48 columns, 49 at 64, 47
   // at 32; 6144 17.9 at 32, 21.5 at 48, 22.8 at 16; 4096 14.7 at 16, 16.9 at 32); at 64 rows three column tiles do not fit
-  // the registers
+  // the registers. Over 22 matrices of 512 .. 32,000 rows, five weight types and 16 .. 64 rows the launch takes 0.51 of the
+  // tile kernel's time on average, and no point takes more
   const bool wide = N >= 48 * 208, middle = N >= 32 * 160;
   if (P.B <= 48) {
     if (wide) launch_rows<QT, 3, 3>(P, xp, Kp, s);
