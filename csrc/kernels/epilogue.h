@@ -75,21 +75,21 @@ __device__ __forceinline__ void epi_apply_t(const GemvParams& P, int bb, int vn,
 
 // The same in two parts for kernels whose threads have many outputs: what an output needs from memory (a store before a load keeps
 // the load behind it, so all of a thread's loads go first), then the rest. Experts (expert_ids) take epi_apply_t.
-struct EpiPre {
+struct EpiOperands {
   float was;   // EPI_ADD: the sum so far
   float bias;
   int slot;    // EPI_QKV
 };
 template <int E>
-__device__ __forceinline__ EpiPre epi_fetch(const GemvParams& P, int bb, int vn) {
-  EpiPre f{0.f, 0.f, 0};
+__device__ __forceinline__ EpiOperands epi_fetch(const GemvParams& P, int bb, int vn) {
+  EpiOperands f{0.f, 0.f, 0};
   if (E != EPI_GLU && E != EPI_GEGLU && P.bias) f.bias = P.bias[vn];
   if constexpr (E == EPI_ADD) f.was = P.y[(long long)bb * P.ldy + vn];
   if constexpr (E == EPI_QKV) f.slot = vn >= P.Eq ? P.slot[bb] : 0;
   return f;
 }
 template <int E>
-__device__ __forceinline__ void epi_put(const GemvParams& P, int bb, int vn, float v, float pv, EpiPre f) {
+__device__ __forceinline__ void epi_put(const GemvParams& P, int bb, int vn, float v, float pv, EpiOperands f) {
   if constexpr (E == EPI_GLU || E == EPI_GEGLU) {
     epi_apply_t<E>(P, bb, vn, v, pv, 0);
     return;

@@ -421,7 +421,7 @@ __global__ __launch_bounds__(256) void gemm_finalize_kernel(GemvParams P, int sk
     const int n0 = 4 * q, vn = n0 + P.row_offset;
     const bool quad = simple && v4 && (E == EPI_ADD || E == EPI_STORE);
     f32x4 was = {0.f, 0.f, 0.f, 0.f};
-    EpiPre pre[4];
+    EpiOperands pre[4];
     if (quad && E == EPI_ADD) was = *(const f32x4*)(P.y + (long long)bb * P.ldy + vn);
     if (simple && !quad) {
 #pragma unroll

@@ -79,7 +79,7 @@ __global__ __launch_bounds__(256) void prep_f16_kernel(GemvParams P, f16* out, i
 template <int E>
 struct Out {
   GemvParams P;
-  typedef EpiPre Pre;
+  typedef EpiOperands Pre;
   __device__ __forceinline__ Pre fetch(int m, int n) const { return epi_fetch<E>(P, m, n + P.row_offset); }
   __device__ __forceinline__ void put(int m, int n, float v, float pv, Pre f) const { epi_put<E>(P, m, n + P.row_offset, v, pv, f); }
 };

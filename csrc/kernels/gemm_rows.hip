@@ -157,7 +157,7 @@ __global__ __launch_bounds__(64 * NW, 2) void dq_rows_kernel(GemvParams P, const
     }
   auto out = [&](auto ec) {  // element r of lane l: row 4 (l >> 4) + r, column l & 15; what the elements need from memory goes first
     constexpr int E = decltype(ec)::value, XN = (MT * NT * 4 + NW - 1) / NW;
-    EpiPre pre[XN];
+    EpiOperands pre[XN];
     auto place = [&](int u, int& x, int& m, int& n) {
       x = tid + 64 * NW * u;
       const int f = x >> 8, r = (x >> 6) & 3, l = x & 63;
