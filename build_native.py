@@ -1,9 +1,9 @@
 """In-tree build of the native core `ollama_operator_amd/_C*.so` for gfx950.
 
 hipcc compiles every `csrc/**/*.hip` (device code) and `csrc/**/*.cpp` (host code: loader,
-executor, pybind11 bindings) in parallel, incrementally, then links one shared object against the
-HIP runtime that torch ships (same SONAME, so one runtime instance per process). No torch headers
-are used, which keeps a full rebuild to well under a minute on 8 cores.
+executor, pybind11 bindings) in parallel, those whose content, headers or command changed, then
+links one shared object against the HIP runtime that torch ships (same SONAME, so one runtime
+instance per process). A full rebuild takes five minutes on 8 cores.
 
     python build_native.py [--clean] [--jobs N]
 """
@@ -12,7 +12,9 @@ from __future__ import annotations
 import argparse
 import concurrent.futures as cf
 import glob
+import hashlib
 import os
+import re
 import subprocess
 import sys
 import sysconfig
@@ -24,6 +26,7 @@ STACK_SRC = os.path.join(CSRC, "stack")
 BUILD = os.path.join(ROOT, "build", "native")
 STACK_BUILD = os.path.join(ROOT, "build", "stack")
 DEBUG_BUILD = os.path.join(ROOT, "build", "debug")
+DEBUG_FLAGS = ["-O1", "-g", "-DOMX_DEBUG_KERNELS"]
 ARCH = os.environ.get("OMX_ARCH", "gfx950")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # HIP device code is compiled without packed-float32 instructions: the compiler forms them from ordinary float code, and
@@ -52,18 +55,49 @@ def _torch_lib() -> str | None:
     return None
 
 
-def _headers() -> list[str]:
-    return glob.glob(os.path.join(CSRC, "**", "*.h"), recursive=True) + [os.path.abspath(__file__)]  # and the flags here
+def _hash(*parts: str | bytes) -> str:
+    h = hashlib.sha256()
+    for x in parts:
+        x = x if isinstance(x, bytes) else x.encode()
+        h.update(len(x).to_bytes(8, "little") + x)
+    return h.hexdigest()
 
 
-def _needs(obj: str, src: str, hdr_mtime: float) -> bool:
-    if not os.path.exists(obj):
-        return True
-    m = os.path.getmtime(obj)
-    return m < os.path.getmtime(src) or m < hdr_mtime
+def _read(path: str) -> bytes:
+    with open(path, "rb") as f:
+        return f.read()
 
 
-DEBUG_FLAGS = ["-O1", "-g", "-DOMX_DEBUG_KERNELS"]
+def _unit_text(src: str) -> list[bytes]:
+    """A unit's source and all headers of the tree that it includes, directly or not, by name and content."""
+    seen: dict[str, bytes] = {}
+    todo = [os.path.abspath(src)]
+    while todo:
+        f = todo.pop()
+        if f in seen:
+            continue
+        seen[f] = _read(f)
+        for name in re.findall(rb'^[ \t]*#[ \t]*include[ \t]*"([^"]+)"', seen[f], re.M):
+            for d in (os.path.dirname(f), CSRC):
+                h = os.path.normpath(os.path.join(d, name.decode()))
+                if os.path.exists(h):
+                    todo.append(h)
+                    break
+    return [x for f in sorted(seen) for x in (os.path.relpath(f, CSRC).encode(), seen[f])]
+
+
+# A product (object, library) is current when the record beside it names what it was made of and the product itself, both by
+# content: times say nothing about an object that was copied, touched or compiled while a header changed.
+def _current(product: str, inputs: str, record: str) -> bool:
+    if not os.path.exists(product) or not os.path.exists(record):
+        return False
+    return _read(record).decode().split() == [inputs, _hash(_read(product))]
+
+
+def _record(product: str, inputs: str, record: str) -> None:
+    if os.path.exists(product):
+        with open(record, "w") as f:
+            f.write(f"{inputs} {_hash(_read(product))}\n")
 
 
 def _core_sources() -> list[str]:
@@ -100,10 +134,19 @@ def all_units() -> list[tuple[str, str, list[str]]]:
     return units(_core_sources(), BUILD, ["-O3"]) + units(_stack_sources(), STACK_BUILD, ["-O3"])
 
 
-def _compile(todo: list[tuple[str, str, list[str]]], jobs: int, verbose: bool, what: str) -> None:
+def _compile(all_: list[tuple[str, str, list[str]]], jobs: int, verbose: bool, what: str, force: bool = False) -> None:
+    version, todo = "/opt/rocm/.info/version", []
+    compiler = _read(version) if os.path.exists(version) else b""
+    for s, obj, cmd in all_:
+        inputs = _hash(compiler, *_unit_text(s), *cmd)
+        if force or not _current(obj, inputs, obj + ".sha256"):
+            todo.append((s, obj, cmd, inputs))
+
     def run(item):
-        s, _, cmd = item
+        s, obj, cmd, inputs = item
         r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode == 0:
+            _record(obj, inputs, obj + ".sha256")
         return s, r.returncode, r.stdout + r.stderr, " ".join(cmd)
 
     failed = []
@@ -120,8 +163,11 @@ def _compile(todo: list[tuple[str, str, list[str]]], jobs: int, verbose: bool, w
         raise RuntimeError(f"{what} build failed ({len(failed)} translation units)")
 
 
-def _link(objs: list[str], out: str, libs: list[str], what: str) -> None:
+def _link(objs: list[str], out: str, libs: list[str], what: str, record: str) -> None:
     """Linked beside the target, then renamed: a reader of the tree (a test, a tree snapshot) never sees a half-written library."""
+    inputs = _hash(*(_hash(_read(o)) for o in objs), *libs)
+    if _current(out, inputs, record):
+        return
     tmp = out + ".tmp"
     link = [HIPCC, "-shared", f"--offload-arch={ARCH}", "-o", tmp, *objs, "-lpthread"]
     tl = _torch_lib()
@@ -131,6 +177,7 @@ def _link(objs: list[str], out: str, libs: list[str], what: str) -> None:
     if r.returncode != 0:
         raise RuntimeError(f"{what} link failed:\n" + " ".join([*link, *libs]) + "\n" + r.stdout + r.stderr)
     os.replace(tmp, out)
+    _record(out, inputs, record)
 
 
 def build(jobs: int | None = None, clean: bool = False, verbose: bool = False, debug: bool = False,
@@ -144,23 +191,20 @@ def build(jobs: int | None = None, clean: bool = False, verbose: bool = False, d
         for f in glob.glob(os.path.join(build_dir, "*.o")):
             os.remove(f)
     srcs = _core_sources() if sources is None else [os.path.join(CSRC, x) for x in sources]
-    hdr_mtime = max((os.path.getmtime(h) for h in _headers()), default=0.0)
     all_ = units(srcs, build_dir, DEBUG_FLAGS if debug else ["-O3"])
-    objs = [obj for _, obj, _ in all_]
-    todo = [u for u in all_ if _needs(u[1], u[0], hdr_mtime)]
-    _compile(todo, jobs or min(8, os.cpu_count() or 4), verbose, "native")
+    _compile(all_, jobs or min(8, os.cpu_count() or 4), verbose, "native")
     if sources is not None:
         return build_dir
     out = target_path()
     if debug:
         os.makedirs(os.path.join(build_dir, "ollama_operator_amd"), exist_ok=True)
         out = os.path.join(build_dir, "ollama_operator_amd", os.path.basename(out))
-    if not os.path.exists(out) or todo or any(os.path.getmtime(o) > os.path.getmtime(out) for o in objs):
-        # hipBLASLt for the large-M prefill GEMM (csrc/runtime/blas.cpp): torch's copy when present
-        # (one instance per process), else the ROCm one
-        tl = _torch_lib()
-        torch_has = tl and os.path.exists(os.path.join(tl, "libhipblaslt.so"))
-        _link(objs, out, ["-lhipblaslt"] + ([] if torch_has else ["-L/opt/rocm/lib"]), "native")
+    # hipBLASLt for the large-M prefill GEMM (csrc/runtime/blas.cpp): torch's copy when present
+    # (one instance per process), else the ROCm one
+    tl = _torch_lib()
+    torch_has = tl and os.path.exists(os.path.join(tl, "libhipblaslt.so"))
+    _link([obj for _, obj, _ in all_], out, ["-lhipblaslt"] + ([] if torch_has else ["-L/opt/rocm/lib"]), "native",
+          os.path.join(build_dir, "module.sha256"))
     return out
 
 
@@ -173,14 +217,10 @@ def build_stack(verbose: bool = False, force: bool = False) -> str:
     the on-device sampler (csrc/kernels/sampling.hip). Its own small library: a checkout that serves only
     such a model compiles these few files (about a minute), not the quantised-GEMV families of `_C`."""
     os.makedirs(STACK_BUILD, exist_ok=True)
-    hdr_mtime = max((os.path.getmtime(h) for h in _headers()), default=0.0)
     all_ = units(_stack_sources(), STACK_BUILD, ["-O3"])
-    objs = [obj for _, obj, _ in all_]
-    todo = [u for u in all_ if force or _needs(u[1], u[0], hdr_mtime)]
-    _compile(todo, min(8, max(1, len(todo))), verbose, "stack module")
+    _compile(all_, min(8, len(all_)), verbose, "stack module", force)
     out = stack_target_path()
-    if not os.path.exists(out) or todo or any(os.path.getmtime(o) > os.path.getmtime(out) for o in objs):
-        _link(objs, out, [], "stack module")
+    _link([obj for _, obj, _ in all_], out, [], "stack module", os.path.join(STACK_BUILD, "module.sha256"))
     return out
 
 
@@ -193,18 +233,20 @@ def build_cpu(verbose: bool = False) -> str:
     runtime dependency, so it loads on a CPU-only node). AVX2 + FMA + F16C baseline, OpenMP threads."""
     import pybind11
     srcs = sorted(glob.glob(os.path.join(CPU_SRC, "*.cpp")))
-    hdrs = glob.glob(os.path.join(CPU_SRC, "*.h"))
+    hdrs = sorted(glob.glob(os.path.join(CPU_SRC, "*.h")))
     out = cpu_target_path()
-    newest = max(os.path.getmtime(f) for f in srcs + hdrs)
-    if os.path.exists(out) and os.path.getmtime(out) >= newest:
-        return out
     cxx = os.environ.get("CXX", "g++")
     cmd = [cxx, "-O3", "-std=c++17", "-fPIC", "-shared", "-fopenmp", "-mavx2", "-mfma", "-mf16c",
            "-fvisibility=hidden", "-I", CPU_SRC, "-I", pybind11.get_include(), "-I", sysconfig.get_paths()["include"],
            *srcs, "-o", out]
+    inputs, record = _hash(*(_read(f) for f in srcs + hdrs), *cmd), os.path.join(ROOT, "build", "cpu.sha256")
+    if _current(out, inputs, record):
+        return out
+    os.makedirs(os.path.dirname(record), exist_ok=True)
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("CPU backend build failed:\n" + " ".join(cmd) + "\n" + r.stdout + r.stderr)
+    _record(out, inputs, record)
     if verbose:
         print("built", os.path.relpath(out, ROOT))
     return out

@@ -44,3 +44,75 @@ def test_every_unit_of_the_tracked_sources_compiles(tmp_path, monkeypatch):
     with cf.ThreadPoolExecutor(max_workers=min(8, os.cpu_count() or 4)) as ex:
         failed = [x for x in ex.map(check, units) if x[1] != 0]
     assert not failed, failed
+
+
+@pytest.fixture
+def small(tmp_path, monkeypatch):
+    """A tree of two units over two headers, and a compiler that writes down what it is asked for."""
+    csrc = tmp_path / "csrc"
+    (csrc / "kernels").mkdir(parents=True)
+    (csrc / "kernels" / "a.hip").write_text('#include "k.h"\n')
+    (csrc / "b.cpp").write_text("#include <vector>\n")
+    (csrc / "kernels" / "k.h").write_text('#include "kernels/deep.h"\n')
+    (csrc / "kernels" / "deep.h").write_text("struct P { int x; };\n")
+    (tmp_path / "ollama_operator_amd").mkdir()
+    for name, value in (("ROOT", str(tmp_path)), ("CSRC", str(csrc)), ("CPU_SRC", str(csrc / "cpu")),
+                        ("STACK_SRC", str(csrc / "stack")), ("BUILD", str(tmp_path / "build"))):
+        monkeypatch.setattr(build_native, name, value)
+    ran = []
+
+    def run(cmd, **kw):
+        out = cmd[cmd.index("-o") + 1]
+        ran.append(os.path.basename(out))
+        with open(out, "w") as f:
+            f.write(" ".join(cmd))
+        return subprocess.CompletedProcess(cmd, 0, "", "")
+
+    monkeypatch.setattr(build_native.subprocess, "run", run)
+
+    def build():
+        ran.clear()
+        build_native.build(jobs=1)
+        return sorted(ran)
+
+    return csrc, build
+
+
+LIB = "_C" + build_native._ext_suffix() + ".tmp"
+
+
+def _age(path, seconds):
+    t = os.path.getmtime(path) + seconds
+    os.utime(path, (t, t))
+
+
+def test_build_decides_by_content(small):
+    csrc, build = small
+    obj = os.path.join(build_native.BUILD, "kernels_a.hip.o")
+    assert build() == [LIB, "b.cpp.o", "kernels_a.hip.o"]
+    assert build() == []
+    # a header changed, its time and the objects' say otherwise (the objects were touched afterwards)
+    (csrc / "kernels" / "deep.h").write_text("struct P { long x; };\n")
+    for o in (obj, os.path.join(build_native.BUILD, "b.cpp.o")):
+        _age(o, 3600)
+    assert build() == ["kernels_a.hip.o"]  # (this compiler's output is the same: nothing to link)
+    # a newer time alone is no change
+    _age(csrc / "kernels" / "deep.h", 7200)
+    assert build() == []
+    # an object from elsewhere, newer than everything
+    with open(obj, "w") as f:
+        f.write("another")
+    _age(obj, 9000)
+    assert build() == ["kernels_a.hip.o"]
+    # a module from elsewhere
+    with open(build_native.target_path(), "w") as f:
+        f.write("another")
+    _age(build_native.target_path(), 9000)
+    assert build() == [LIB]
+
+
+def test_build_follows_flags(small, monkeypatch):
+    _, build = small
+    build()
+    monkeypatch.setattr(build_native, "NO_PK_F32", ["-other"])
+    assert build() == [LIB, "kernels_a.hip.o"]
