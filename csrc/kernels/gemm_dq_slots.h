@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "gemm_dq_impl.h"
+#include "gemm_dq_places.h"
 #include "gemm_ring.h"
 
 namespace omx {
@@ -53,10 +54,10 @@ __device__ __forceinline__ void ds_tile(const GemvParams& P, const f16* __restri
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const QMat& w = P.w;
   const int N = w.N, SB = Kp >> 8;
-  const int ks0 = 4 * (int)((long long)z * SB / sk), ks1 = 4 * (int)((long long)(z + 1) * SB / sk);
+  const int ks0 = 4 * (int)((long long)z * SB / sk), ks1 = 4 * (int)((long long)(z + 1) * SB / sk), kl = ks1 - 1;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int fr = lane & 31, fq = lane >> 5, xr = tid >> 3, xc = tid & 7;
-  // operands through buffer descriptors of the tile's rows: places advance in scalar registers, reads past the end give zeros
+  // operands through buffer descriptors of the tile's rows: places advance in scalar registers
   auto rsrc = [](const void* p, long long bytes) {
     return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)(unsigned)(bytes < 0xFFFFFFF0LL ? bytes : 0xFFFFFFF0LL), 0x00027000);
   };
@@ -69,7 +70,7 @@ __device__ __forceinline__ void ds_tile(const GemvParams& P, const f16* __restri
   const auto b2 = rsrc(B2 ? w.s2 + wf * B2 : w.s1, wl * B2), b3 = rsrc(B3 ? w.s3 + wf * B3 : w.s1, wl * B3);
   unsigned ox[TM], rw[TN];
 #pragma unroll
-  for (int i = 0; i < TM; ++i) ox[i] = 2u * ((unsigned)min(xr + 32 * i, rows - 1) * (unsigned)Kp + 8 * xc);
+  for (int i = 0; i < TM; ++i) ox[i] = ds_x_at(min(xr + 32 * i, rows - 1), Kp, xc);
 #pragma unroll
   for (int j = 0; j < TN; ++j) rw[j] = (unsigned)min(32 * TN * wave + 32 * j + fr, N - 1 - n0) * (unsigned)SB;
   u32x4 xv[2][TM];
@@ -80,16 +81,17 @@ __device__ __forceinline__ void ds_tile(const GemvParams& P, const f16* __restri
   const unsigned da = SB == 1 ? 0 : 2, db = SB == 1 ? 2 : 0;
   auto load_x = [&](int ks, auto b, auto c) {
     constexpr int C = decltype(c)::value;
-    xv[decltype(b)::value][C] = b128(bx, ox[C], 128u * ks);
+    xv[decltype(b)::value][C] = b128(bx, ox[C], ds_x_step(ks, kl));
   };
   auto load_w = [&](int ks, int j, int part, int slot) {
     Piece<QT>& q = wv[slot][j];
     if (part == 0) {
-      const unsigned at = rw[j] * CB + (CB / 8) * fq;
-      q.a = b128(bc, at, (unsigned)ks * (CB / 4));
-      if constexpr (K8) q.b = b128(bc, at + 16, (unsigned)ks * (CB / 4));
-      if constexpr (QT == QT_Q5_K) q.e = __builtin_amdgcn_raw_buffer_load_b32(b2, rw[j] * 32 + 4 * fq, 8u * ks, 0);
-      if constexpr (Q6) q.h = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(b1, rw[j] * 64 + 8 * fq, 16u * ks, 0));
+      const unsigned at = ds_w_at(rw[j], CB, fq);
+      q.a = b128(bc, at, ds_w_step(ks, kl, CB));
+      if constexpr (K8) q.b = b128(bc, at + 16, ds_w_step(ks, kl, CB));
+      if constexpr (QT == QT_Q5_K) q.e = __builtin_amdgcn_raw_buffer_load_b32(b2, ds_w_at(rw[j], 32, fq), ds_w_step(ks, kl, 32), 0);
+      if constexpr (Q6)
+        q.h = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(b1, ds_w_at(rw[j], 64, fq), ds_w_step(ks, kl, 64), 0));
     } else {
       const unsigned at = rw[j] + lsb;
       if constexpr (KM) q.m = b128(b1, 16 * at, 0);
@@ -97,7 +99,7 @@ __device__ __forceinline__ void ds_tile(const GemvParams& P, const f16* __restri
         q.m = b128(b2, 16 * at, 0);
         q.e = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(b3, 2 * at, 0, 0);
       }
-      if constexpr (K8 || QT == QT_Q4_0) q.e = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(b1, 16 * at + 2 * lt, 0, 0);
+      if constexpr (K8 || QT == QT_Q4_0) q.e = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(b1, ds_scale_at(at, lt), 0, 0);
       if (j == TN - 1) {  // two pieces of the stream further
         wt[slot] = lt;
         lsb += da, lt += db;
