@@ -219,8 +219,9 @@ void Executor::attn_block(int i, const StepInputs& in, hipStream_t s) {
   P.n_rot = cfg.n_rot;
   P.n_kv = cfg.Hkv;
   P.bs = in.bs;  // the next GEMV of the step (gemv.hip cross-launch prefetch)
-  if (in.prefill && B >= GEMM_MIN_B && ws.rope) {  // every layer turns by the same angles
-    if (i == 0) rope_table(in.pos, inv_freq, B, cfg.n_rot / 2, ws.rope, s);
+  if (in.prefill && B >= GEMM_MIN_B && ws.rope) {
+    // every layer of a pass turns by the same angles; a stage call by itself knows of no layer before it
+    if (i == 0 || !in_pass_) rope_table(in.pos, inv_freq, B, cfg.n_rot / 2, ws.rope, s);
     P.rope = ws.rope;
   }
   const bool ch = chain(in);
@@ -575,16 +576,20 @@ bool Executor::ar_fits(int B) const {
   return ws.ar_on && (long long)B * cfg.E <= ws.ar.slab_floats && (long long)B * cfg.V <= ws.ar.slab_floats;
 }
 
+namespace {
+struct Active {
+  int& f;
+  explicit Active(int& x) : f(x) { f = 1; }
+  ~Active() { f = 0; }
+};
+}  // namespace
+
 void Executor::forward_tp(const StepInputs& in, hipStream_t s) {
   if (cfg.tp <= 1 || !ws.ar_on) throw std::runtime_error("forward_tp needs tp > 1 and the custom all-reduce");
   if (!ar_fits(in.B)) throw std::runtime_error("forward_tp: batch exceeds the all-reduce slabs");
   if (in.B > ws.max_B) throw std::runtime_error("batch exceeds workspace");
   const int n = in.B * cfg.E;
-  struct Active {  // the stages write partial sums to the slabs only inside forward_tp
-    int& f;
-    explicit Active(int& x) : f(x) { f = 1; }
-    ~Active() { f = 0; }
-  } active(ar_active_);
+  Active active(ar_active_), pass(in_pass_);  // the stages write partial sums to the slabs only inside forward_tp
   embed(in, s);
   const bool q8 = x8(in);
   for (int i = 0; i < cfg.n_layer; ++i) {
@@ -618,6 +623,7 @@ void Executor::forward_tp(const StepInputs& in, hipStream_t s) {
 void Executor::forward(const StepInputs& in, hipStream_t s) {
   if (cfg.tp != 1) throw std::runtime_error("Executor::forward is the TP=1 path; TP steps are driven per block");
   if (in.B > ws.max_B) throw std::runtime_error("batch exceeds workspace");
+  Active pass(in_pass_);
   embed(in, s);
   for (int i = 0; i < cfg.n_layer; ++i) {
     attn_block(i, in, s);

@@ -78,7 +78,7 @@ struct Workspace {
   long long w16_elems = 0;
   float* yws = nullptr;      //   and its fp32 output slab [M][N]
   long long yws_elems = 0;
-  float* rope = nullptr;     // [maxB][n_rot / 2] {cosine, sine} of a prompt's positions, written in layer 0
+  float* rope = nullptr;     // [maxB][n_rot / 2] {cosine, sine} of a prompt's positions, written in a pass's layer 0
   int max_B = 0;
   int n_splits = 1;
   int defer = 0;             // B == 1: attention leaves n_splits partials, the O GEMV merges them
@@ -164,6 +164,7 @@ class Executor {
   GemvParams phi_down_params(int i, const StepInputs& in) const;  // phi2 layer i's ffn_down GEMV
   bool phi_pair(int i, const StepInputs& in) const;               // phi2: O + down as one launch
   int ar_active_ = 0;
+  int in_pass_ = 0;  // inside forward / forward_tp: all layers in order on the same inputs
 };
 
 }  // namespace omx
