@@ -572,6 +572,12 @@ class Runner:
         else:
             dst.copy_(torch.tensor(s.blocks, dtype=torch.int32))
 
+    def _reserve(self, sid: int, n_total: int) -> None:
+        try:
+            self.kv.reserve(sid, n_total)
+        finally:  # a reservation that fails may have taken blocks: the sequence keeps them, and is not asked again
+            self._sync_block_table(sid)
+
     def _sync_block_tables(self, sids: list[int]) -> None:
         """Block-table rows of several sequences, as one copy: the span of table rows from the first to the last
         of them as the host holds it (rows of the sequences between are what the device has already, free rows
@@ -652,8 +658,7 @@ class Runner:
         n = len(tokens)
         if start + n > self.ctx:
             raise ValueError(f"context overflow: {start + n} > {self.ctx}")
-        self.kv.reserve(sid, start + n)
-        self._sync_block_table(sid)
+        self._reserve(sid, start + n)
         C = self.max_batch
         for c0 in range(0, n, C):
             chunk = tokens[c0:c0 + C]
@@ -871,8 +876,7 @@ class Runner:
         s = self.kv.seqs[sid]
         reserved = False
         if pos + k > len(s.blocks) * self.block_size:
-            self.kv.reserve(sid, min(self.ctx, pos + k + 4 * self.block_size))
-            self._sync_block_table(sid)
+            self._reserve(sid, min(self.ctx, pos + k + 4 * self.block_size))
             reserved = True
         if not (not reserved and self._adv_next == (sid, pos)):
             self._upload(np.array([[pos], [self.kv.slot(sid, pos)], [pos + 1], [s.row], [0]], np.int32), None)
@@ -904,8 +908,8 @@ class Runner:
             for b, (sid, pos) in enumerate(zip(sids, poss)):
                 s = self.kv.seqs[sid]
                 if pos + 1 > len(s.blocks) * self.block_size:
+                    grown.append(sid)  # first: a reservation that fails may have taken blocks
                     self.kv.reserve(sid, min(self.ctx, pos + 4 * self.block_size))
-                    grown.append(sid)
                 arr[:, b] = (pos, self.kv.slot(sid, pos), pos + 1, s.row, b)
         finally:  # also where a later sequence finds no blocks: these hold theirs, and are not asked again
             if grown:
@@ -1009,8 +1013,8 @@ class Runner:
                 start = s.length
                 if start + len(tokens) > self.ctx:
                     raise ValueError(f"context overflow: {start + len(tokens)} > {self.ctx}")
-                self.kv.reserve(sid, start + len(tokens))
                 grown.append(sid)
+                self.kv.reserve(sid, start + len(tokens))
                 pos = np.arange(start, start + len(tokens))
                 pos_l.append(pos)
                 slot_l.append(self._slots(sid, pos))
@@ -1059,8 +1063,8 @@ class Runner:
                 start, n = s.length, len(tokens)
                 if start + n > self.ctx:
                     raise ValueError(f"context overflow: {start + n} > {self.ctx}")
-                self.kv.reserve(sid, start + n)
                 grown.append(sid)
+                self.kv.reserve(sid, start + n)
                 ws = set(int(i) for i in want)
                 if any(i < 0 or i >= n for i in ws):
                     raise ValueError("a wanted place lies outside the entry's tokens")

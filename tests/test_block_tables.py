@@ -69,3 +69,28 @@ def test_a_refused_row_leaves_the_others_in_place(tiny_models, device):
     with pytest.raises(OutOfBlocks):
         r.admit_many([(a[0], r.block_size, [5] * 3, O, [1] * r.block_size, 0), (a[2], r.block_size, [5] * 90, O, [1] * r.block_size, 0)])
     same(r, a[:2])
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_a_reservation_that_fails_midway_leaves_its_blocks_on_the_device(tiny_models, device):
+    """The pool runs out within a row's reservation: the blocks it took are the row's, and a step that needs no more goes through."""
+    r = Runner(tiny_models["tiny-llama"], device=device, max_batch=64, max_seqs=4, ctx=128, kv_tokens=6 * 16)
+    assert r.block_size == 16
+    a = admit(r, [16, 16, 16], np.random.default_rng(5))
+    poss = [16, 16, 16]
+    r.recompose([(O, [1, 7], 0, 0)] * 3, [7] * 3)
+    r.d_block_table[:] = -1  # whatever is not uploaded again is no page
+    for sid in a:
+        r._sync_block_table(sid)
+    with pytest.raises(OutOfBlocks):
+        r.decode_batch(a, poss)  # asks for four blocks a row: three are left
+    s = r.kv.seqs[a[0]]
+    assert len(s.blocks) > 1 and r.kv.alloc.n_free == 0
+    same(r, a)
+    r.free_sequence(a[2])
+    with pytest.raises(OutOfBlocks):
+        r.admit_many([(a[1], 16, [5] * 40, O, [1] * 16, 0), (r.new_sequence(), 0, [5] * 60, O, [5] * 60, 0)])
+    same(r, a[:2])
+    with pytest.raises(OutOfBlocks):
+        r.step_entries([(a[1], [5] * 90, [1])])
+    same(r, a[:2])
