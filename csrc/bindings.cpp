@@ -317,6 +317,18 @@ PYBIND11_MODULE(_C, m) {
         "whether a layer's routed experts take the grouped launches (gemm_dq_moe.hip) for prompts");
   m.def("set_dq_gemm", &set_dq_gemm,
         "1: prefill GEMMs on the stream-order dequant kernels (gemm_dq.hip from 65 rows, gemm_rows.hip from 16)");
+  m.def("dq_choice", [](int qtype, int M, int N, int K, long long gws_elems) {
+    GemvParams P{};
+    P.w.qtype = qtype;
+    P.w.N = N;
+    P.w.K = K;
+    P.B = M;
+    float slab;  // (never read)
+    P.gws = gws_elems > 0 ? &slab : nullptr;
+    P.gws_elems = gws_elems;
+    const DqChoice c = dq_choose(P);
+    return py::make_tuple(c.tile, c.sk);
+  }, "(tile, K splits) that the dq GEMM takes for M rows with slabs of gws_elems floats");
   m.def("set_dq_tuning", &set_dq_tuning, "microbenchmarks: force the dq GEMM tile config (0..3, -1 auto) and split-K factor (0 auto)");
   m.def("dq_gemm_enabled", &dq_gemm_enabled);
   m.def("set_gemv8_geo", [](int nsb, int ks) { set_gemv8_geo(nsb, ks); });

@@ -1,6 +1,8 @@
-// Stream-order dequant prefill GEMM: dispatcher and knobs. Kernels and the tile x split-K chooser are in
+// Stream-order dequant prefill GEMM: dispatcher and knobs. Kernels are in
 // gemm_dq_slots.h (shared parts in gemm_dq_impl.h), instantiated once per weight type in gemm_dq_<type>.hip.
 #include <cstdlib>
+#include <stdexcept>
+#include <string>
 
 #include "common.h"
 #include "ops.h"
@@ -39,6 +41,46 @@ void set_dq_tuning(int cfg, int sk) {
   dq_gemm_enabled();  // env defaults read first, then overridden
   g_dq_cfg = cfg;
   g_dq_sk = sk;
+}
+
+// tile x K split with the least time by a model of measured launches: the first and last steps of a wave of blocks cost `fixed`,
+// every further wave `again`, a step of 64 K c0 while few blocks run and c1 on a full chip, on 128 x 128 tiles c2 with two blocks a
+// CU (us); a split adds a launch that sums the slabs. Over 65 .. 2,048 rows x 7 matrices of 1,024 .. 22,016 rows and K = 4,096 ..
+// 14,336 (all tiles and splits timed) the choice takes 0.3 % more time than the best on average and 5 % at most, Q6_K, whose
+// unpacking is longer, with values of its own the same.
+struct DsTile {
+  int bm, bn;
+  double fixed, again, c0, c1, c2;
+};
+constexpr DsTile DS_TILES[4] = {{256, 256, 12.0, 6.1, 1.14, 1.51, 0}, {256, 128, 10.0, 1.3, 0.59, 0.92, 0},
+                                {128, 256, 6.9, 0.8, 0.78, 1.05, 0},  {128, 128, 6.7, 0.0, 0.42, 0.62, 1.05}};
+constexpr DsTile DS_TILES6[4] = {{256, 256, 9.8, 3.8, 1.34, 1.99, 0}, {256, 128, 4.3, 2.8, 0.77, 1.13, 0},
+                                 {128, 256, 5.7, 1.4, 1.08, 1.50, 0}, {128, 128, 2.6, 0.0, 0.64, 0.91, 1.51}};
+DqChoice dq_choose(const GemvParams& P) {
+  dq_gemm_enabled();  // OMX_DQ_CFG is read
+  const bool q6 = P.w.qtype == QT_Q6_K;
+  const int M = P.B, N = P.w.N, SB = (P.w.K + 255) >> 8;
+  const int rule[6] = {1, 2, 3, 4, 6, 8}, *ks = g_dq_sk > 0 ? &g_dq_sk : rule, n_ks = g_dq_sk > 0 ? 1 : 6;
+  const double g = q6 ? 8.4 : 3.0, bw = q6 ? 8.6e6 : 5.4e6;
+  double least = -1.0;
+  DqChoice best{3, 1};
+  for (int c = 0; c < 4; ++c) {
+    if (g_dq_cfg >= 0 && g_dq_cfg <= 3 && c != g_dq_cfg) continue;
+    const DsTile& t = q6 ? DS_TILES6[c] : DS_TILES[c];
+    for (int i = 0; i < n_ks; ++i) {
+      const int k = ks[i];
+      const long long units = (long long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * k;
+      if (k > 1 && (!P.gws || (long long)k * M * N > P.gws_elems || SB < k || (units > 640 && g_dq_sk <= 0))) break;
+      const double slots = c == 3 ? 512 : 256, waves = (double)(long long)((units + slots - 1) / slots);
+      const double fill = units < 256 ? units / 256.0 : 1.0, step = t.c2 > 0 && units > 256 ? t.c2 : t.c0 + (t.c1 - t.c0) * fill;
+      const double us = t.fixed + (waves - 1) * t.again + waves * 4 * SB / k * step + (k > 1 ? g + 8.0 * k * M * N / bw : 0.0);
+      if (least < 0.0 || us < least) least = us, best = {c, k};
+    }
+  }
+  if (least < 0.0)  // a forced split
+    throw std::runtime_error("dq GEMM: " + std::to_string(g_dq_sk) + " splits of K do not fit " + std::to_string(SB) +
+                             " super-blocks or the slabs");
+  return best;
 }
 
 bool dq_gemm(const GemvParams& P, hipStream_t s) {

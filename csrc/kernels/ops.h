@@ -203,6 +203,11 @@ void set_dq_ring(int on);  // no effect (gemm_dq.hip)
 // cosine and sine of pos[b] * inv_freq[i], i < half, to out [B][half][2] (GemvParams::rope)
 void rope_table(const int* pos, const float* inv_freq, int B, int half, float* out, hipStream_t s);
 void set_dq_tuning(int cfg, int sk);  // microbenchmarks: force tile config (-1 auto) and split-K (0 auto)
+// tile (0..3: 256 x 256, 256 x 128, 128 x 256, 128 x 128) and K splits of a product; throws where a forced split does not fit
+struct DqChoice {
+  int tile, sk;
+};
+DqChoice dq_choose(const GemvParams& P);
 void gemm_finalize(const GemvParams& P, int sk, hipStream_t s);  // sums sk split-K slabs + epilogue
 
 // launch-shape knobs for the decode GEMV (tuned on MI355X; see scripts/bench_gemv.py)

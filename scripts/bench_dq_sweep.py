@@ -1,6 +1,6 @@
 """dq GEMM tile / split-K sweep (csrc/kernels/gemm_dq.hip) on Llama-2-7B Q4_K_M shapes: for every shape and
 M, each forced (tile config, split-K) pair next to the automatic choice, time per call (prep + GEMM +
-finalize) and TFLOP/s. Feeds the chooser in run_dq. On the GPU box: python scripts/bench_dq_sweep.py"""
+finalize) and TFLOP/s. Feeds the chooser (dq_choose). On the GPU box: python scripts/bench_dq_sweep.py"""
 import os
 import sys
 
@@ -37,6 +37,10 @@ def main():
             res = []
             for cfg, sk in [(-1, 0)] + [(c, k) for c in CFGS for k in sks]:
                 C.set_dq_tuning(cfg, sk)
+                try:
+                    C.dq_choice(int(qt), M, N, K, gws.numel())
+                except RuntimeError:  # this split does not fit
+                    continue
                 for _ in range(3):
                     fn()
                 torch.cuda.synchronize()
