@@ -334,7 +334,6 @@ PYBIND11_MODULE(_C, m) {
   m.def("set_gemv8_geo", [](int nsb, int ks) { set_gemv8_geo(nsb, ks); });
   m.def("set_gemv8_kb", [](int mode) { set_gemv8_kb(mode); });
   m.def("gemv8_merge_supported", &gemv8_merge_supported);
-  m.def("set_dq_ring", &set_dq_ring, "no effect: both kernels it chose between are gone");
   // launch counters (ops.h LC_*): tests assert which kernel family a call enqueued
   m.def("launch_counts", []() {
     static const char* names[LC_N] = {"dq_gemm", "gemm_tile", "gemm_lib", "gemv8_row1", "gemv8_rows", "gemv8_dual",

@@ -35,8 +35,6 @@ bool dq_gemm_enabled() {
 
 void set_dq_gemm(int on) { g_dq_enable = on ? 1 : 0; }
 
-void set_dq_ring(int) {}  // chose between two kernels that gemm_dq_slots.h has replaced; callers may still set it
-
 void set_dq_tuning(int cfg, int sk) {
   dq_gemm_enabled();  // env defaults read first, then overridden
   g_dq_cfg = cfg;

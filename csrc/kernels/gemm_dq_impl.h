@@ -144,27 +144,6 @@ struct Piece {
   unsigned e;                                // Q5_K 5th bits; Q6_K / Q4_0 / Q8_0: fp16 d (low half)
 };
 
-template <int QT>
-__device__ __forceinline__ void load_piece(const QMat& w, long long row, int SB, int pc, Piece<QT>& R) {
-  const int t = pc / SB, sb = pc - t * SB;
-  if constexpr (QT == QT_Q8_0) {
-    const uint8_t* q = w.s0 + row * SB * 256 + 32LL * pc;
-    R.a = *(const u32x4*)q;
-    R.b = *(const u32x4*)(q + 16);
-    R.e = *(const uint16_t*)(w.s1 + row * SB * 16 + 16LL * sb + 2 * t);
-  } else {
-    R.a = *(const u32x4*)(w.s0 + row * SB * 128 + 16LL * pc);
-    if constexpr (QT == QT_Q4_K || QT == QT_Q5_K) R.m = *(const u32x4*)(w.s1 + row * SB * 16 + 16LL * sb);
-    if constexpr (QT == QT_Q5_K) R.e = *(const unsigned*)(w.s2 + row * SB * 32 + 4LL * pc);
-    if constexpr (QT == QT_Q6_K) {
-      R.h = *(const u32x2*)(w.s1 + row * SB * 64 + 8LL * pc);
-      R.m = *(const u32x4*)(w.s2 + row * SB * 16 + 16LL * sb);
-      R.e = *(const uint16_t*)(w.s3 + row * SB * 2 + 2LL * sb);
-    }
-    if constexpr (QT == QT_Q4_0) R.e = *(const uint16_t*)(w.s1 + row * SB * 16 + 16LL * sb + 2 * t);
-  }
-}
-
 // Q4_K / Q5_K 6-bit scale and min of sub-block j (no branch: j differs between the lanes of a wave)
 __device__ __forceinline__ void k_scale(const u32x4& m, int j, float& sc, float& mn) {
   const float d = h2f(m.x & 0xFFFF), dmin = h2f(m.x >> 16);
@@ -208,27 +187,6 @@ __device__ __forceinline__ void dq_scale(const u32x4& m, unsigned e, int t, int 
     S = dq_splat(h2f((uint16_t)e) * (float)(int8_t)(m.x & 0xFF));
   } else {
     S = dq_splat(h2f((uint16_t)e));
-  }
-}
-
-// dequantise a piece to 32 fp16 in stream order: o[0..7] = lo half pairs, o[8..15] = hi half pairs
-template <int QT>
-__device__ __forceinline__ void dq_piece(const Piece<QT>& R, int t, unsigned (&o)[16]) {
-#pragma unroll
-  for (int half = 0; half < 2; ++half) {
-    u32x4 m = R.m;
-    if constexpr (QT == QT_Q6_K) {  // int8 scales 8 n + sub (lo codes) and 8 n + sub + 4 (hi codes): dwords 2 n / 2 n + 1, byte sub
-      const int n = t >> 2, sub = t & 3;
-      m.x = (half ? (n ? R.m.w : R.m.y) : (n ? R.m.z : R.m.x)) >> (8 * sub);
-    }
-    dh2 S, C;
-    dq_scale<QT>(m, R.e, t, half, S, C);
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-#pragma unroll
-      for (int odd = 0; odd < 2; ++odd)
-        o[8 * half + 2 * e + odd] = dq_word<QT>(dsel(QT == QT_Q8_0 && half ? R.b : R.a, e), QT == QT_Q6_K ? (half ? R.h.y : R.h.x) : R.e,
-                                                half, e, odd, S, C);
   }
 }
 

@@ -199,7 +199,6 @@ bool dq_moe_covered(const GemvParams& P);
 void dq_moe(const GemvParams& P, hipStream_t s);
 bool dq_gemm_enabled();
 void set_dq_gemm(int on);
-void set_dq_ring(int on);  // no effect (gemm_dq.hip)
 // cosine and sine of pos[b] * inv_freq[i], i < half, to out [B][half][2] (GemvParams::rope)
 void rope_table(const int* pos, const float* inv_freq, int B, int half, float* out, hipStream_t s);
 void set_dq_tuning(int cfg, int sk);  // microbenchmarks: force tile config (-1 auto) and split-K (0 auto)

@@ -393,15 +393,14 @@ def test_ffn_down_k_padding(tiny_models, monkeypatch, name):
     assert ta == tb
 
 
-@pytest.mark.parametrize("ring", [0, 1])
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
 @pytest.mark.parametrize("name", ["tiny-llama", "tiny-llama-q40", "tiny-llama-q8", "tiny-llama-q5km", "tiny-phi2"])
-def test_prefill_dq_ring_and_glds_kernels(tiny_models, name, ring):
-    """Both editions of the hand-written prefill GEMM (gemm_dq_impl.h: the register-ring default and the
-    glds kernel, set_dq_ring) over 240 prompt rows (128- and 256-row tiles with a partial last tile,
-    split-K for the narrow shapes): logits match the torch twin and every dense projection ran on the dq
-    kernel."""
+def test_prefill_dq_tiles(tiny_models, name, tile):
+    """Each tile of the hand-written prefill GEMM (gemm_dq_slots.h, set_dq_tuning) over 240 prompt rows (128- and 256-row
+    tiles with a partial last tile, split-K for the narrow shapes): logits match the torch twin and every dense projection
+    ran on the dq kernel."""
     C = native()
-    C.set_dq_ring(ring)
+    C.set_dq_tuning(tile, 0)
     try:
         path = tiny_models[name]
         g = Runner(path, device="cuda", max_batch=256, max_seqs=2, ctx=256)
@@ -417,4 +416,4 @@ def test_prefill_dq_ring_and_glds_kernels(tiny_models, name, ring):
         V = g.cfg.n_vocab
         assert rel(g.logits[0, :V].cpu(), c.logits[0, :V]) < 3e-2
     finally:
-        C.set_dq_ring(1)
+        C.set_dq_tuning(-1, 0)
