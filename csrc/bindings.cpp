@@ -268,7 +268,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("attention", [](uintptr_t q, int ldq, uintptr_t kc, uintptr_t vc, uintptr_t block_table, int max_blocks,
                         uintptr_t q_seq, uintptr_t q_len, int NQ, int H, int n_kv, int D, int bs, float scale,
                         int window, uintptr_t out, int ldo, uintptr_t ws, int n_splits, uintptr_t counters,
-                        uintptr_t stream, int prefill, int Dv) {
+                        uintptr_t stream, int prefill, int Dv, int heads) {
     if (n_splits < 1 || n_splits > 64) throw std::runtime_error("n_splits must be in [1, 64]");
     if (n_splits > 1 && (!ws || !counters)) throw std::runtime_error("split attention needs ws and counters");
     check_attn(H, n_kv, D, Dv);
@@ -295,11 +295,14 @@ PYBIND11_MODULE(_C, m) {
     A.counters = Pp<int>(counters);
     A.prefill = prefill;
     A.Dv = Dv;
+    A.heads = heads;
     attention_decode(A, S(stream));
   }, py::arg("q"), py::arg("ldq"), py::arg("kc"), py::arg("vc"), py::arg("block_table"), py::arg("max_blocks"),
      py::arg("q_seq"), py::arg("q_len"), py::arg("NQ"), py::arg("H"), py::arg("n_kv"), py::arg("D"), py::arg("bs"),
      py::arg("scale"), py::arg("window"), py::arg("out"), py::arg("ldo"), py::arg("ws"), py::arg("n_splits"),
-     py::arg("counters"), py::arg("stream"), py::arg("prefill") = 0, py::arg("Dv") = 0);
+     py::arg("counters"), py::arg("stream"), py::arg("prefill") = 0, py::arg("Dv") = 0, py::arg("heads") = 0);
+  m.def("attention_heads", &attention_heads, "query heads per decode block for rows of `keys` keys on average", py::arg("NQ"),
+        py::arg("H"), py::arg("n_kv"), py::arg("D"), py::arg("keys"));
   m.def("attention_ws_floats", &attention_ws_floats);
   m.def("set_attn_tuning", &set_attn_tuning, py::arg("kps"), py::arg("hpb") = -1);
   m.def("gemv_merge_supported", &gemv_merge_supported);
@@ -517,10 +520,11 @@ PYBIND11_MODULE(_C, m) {
       .def_property_readonly("x8_on", [](const Executor& e) { return e.ws.x8_ok; })
       .def_property_readonly("x8_bmax", [](const Executor& e) { return e.ws.x8_ok ? e.ws.x8_bmax : 0; })
       .def("set_segments", [](Executor& e, std::vector<std::pair<int, int>> segs) { e.segments = std::move(segs); })
-      .def("set_splits", [](Executor& e, int n, int defer) {
+      .def("set_splits", [](Executor& e, int n, int defer, int heads) {
         e.ws.n_splits = n;
         e.ws.defer = defer;
-      }, py::arg("n"), py::arg("defer") = 0)
+        e.ws.attn_heads = heads;
+      }, py::arg("n"), py::arg("defer") = 0, py::arg("heads") = 0)
       .def("run", [](Executor& e, const std::string& what, int layer, py::dict d, uintptr_t stream) {
         static const std::pair<const char*, int> names[] = {{"forward", ST_FORWARD}, {"embed", ST_EMBED},
             {"attn", ST_ATTN}, {"ffn", ST_FFN}, {"head", ST_HEAD}, {"forward_tp", ST_FORWARD_TP}};

@@ -785,21 +785,33 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void attn_prefill_kernel(Att
 
 // query heads per block: as many of a GQA group as leave a block for each of the 256 CUs. A head more is a second pass of
 // arithmetic over the same rows (a step of 128 keys takes 1.2 us with one head, 1.6 with two, 2.5 with four), blocks that
-// share a KV head read its rows from L2. Measured (us at 1 / 2 / 4 heads, 32 heads on 8, 400 keys): 4 rows 7.9 / 10.5 / 15.9,
-// 8 rows 8.2 / 10.8 / 16.1, 16 rows 13.3 / 11.9 / 16.7; 64 heads on 8: 8 rows 13.1 / 12.1 / 16.1. The whole group reads
-// least and wins from some 1,300 keys in every row on (8 rows, 3,000 keys: 37 / 29 / 27; 8,000: 99 / 65 / 54), so it stays
-// where the sequences may grow past 4,096 keys and the launch is 64 blocks or more: the lengths are known on the device only.
-static int heads_per_block(const AttnParams& P) {
-  const int G = P.H / P.n_kv;
-  const bool grown = (long long)P.max_blocks * P.bs > 4096 && (P.window <= 0 || P.window > 4096);
-  int hpb = g_attn_hpb;
-  if (hpb <= 0) hpb = (long long)P.NQ * P.n_kv < 64 ? 1 : grown ? G : std::clamp((int)((long long)P.NQ * P.H / 256), 1, G);
-  if (P.D > 128 && hpb > 2) hpb = 2;  // head dim 256: the per-wave merge tile [8][G][D + 2] fits LDS for G <= 2
+// share a KV head read its rows from L2. From some 1,300 keys in the mean row on, the reads weigh more: the whole group, up to four
+// heads (eight were behind four at every length). Launches of fewer than 64 blocks take one head in any case. Measured, us at 1 / 2 / 4 / 8
+// heads, 128 dims, heads / KV heads x rows:
+//   32 / 8 x 8:  400 keys 8.5 / 11.1 / 16.3, 800 13.9 / 15.4 / 18.1, 1,300 19.9 / 19.4 / 19.3, 2,000 27.1 / 23.0 / 22.2, 4,000 50 / 39 / 35
+//   32 / 8 x 16: 400 14.2 / 12.2 / 17.0, 1,300 35 / 26.0 / 27.1, 2,000 52 / 35.5 / 33.9, 4,000 104 / 66 / 55
+//   64 / 8 x 8:  400 12.9 / 12.2 / 16.1 / 26.8, 1,300 31 / 26.8 / 26.0 / 28.8, 4,000 86 / 63 / 53 / 58;  x 16, 400: 21 / 21 / 17.7 / 27.0
+// keys: of the mean row, as the host knows it.
+int attention_heads(int NQ, int H, int n_kv, int D, long long keys) {
+  const int G = H / n_kv, most = std::min(G, 4);
+  int hpb = (long long)NQ * n_kv < 64 ? 1 : keys > 1300 ? most : std::clamp((int)((long long)NQ * H / 256), 1, most);
+  if (D > 128 && hpb > 2) hpb = 2;  // head dim 256: the per-wave merge tile [8][G][D + 2] fits LDS for G <= 2
   // head dims 80 / 96 / 112 (an fp8 row of 5-7 bytes per lane is widened at load): at 4+ heads per block
   // the kernel spills, so those dims take at most 2 (K/V re-reads of a wider group hit L2)
-  if (P.D % 64 && hpb > 2) hpb = 2;
-  while (hpb > 1 && (G % hpb || (hpb != 1 && hpb != 2 && hpb != 4 && hpb != 8))) --hpb;
-  return hpb < 1 ? 1 : hpb;
+  if (D % 64 && hpb > 2) hpb = 2;
+  while (hpb > 1 && (G % hpb || hpb == 3)) --hpb;
+  return hpb;
+}
+
+// a caller that names neither heads nor lengths (AttnParams::heads 0) gets the heads for the longest rows that the table holds
+static int heads_per_block(const AttnParams& P) {
+  const int G = P.H / P.n_kv;
+  const long long most = (long long)P.max_blocks * P.bs;
+  int hpb = g_attn_hpb > 0 ? g_attn_hpb : P.heads;
+  if (hpb <= 0) return attention_heads(P.NQ, P.H, P.n_kv, P.D, P.window > 0 ? std::min<long long>(P.window, most) : most);
+  if ((P.D > 128 || P.D % 64) && hpb > 2) hpb = 2;  // (as above)
+  while (hpb > 1 && (G % hpb || (hpb != 2 && hpb != 4 && hpb != 8))) --hpb;
+  return hpb;
 }
 
 template <int D, bool KV8>

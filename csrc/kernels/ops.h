@@ -258,10 +258,12 @@ struct AttnParams {
   int defer;                   // write exactly n_splits unmerged partials (attention_ws_floats layout
                                // [NQ][S][H*D] then [NQ][S][H][2] {m, l}); the consumer merges them
   int kv8;                     // kc / vc hold fp8 e4m3 (OCP e4m3fn) instead of fp16
+  int heads;                   // decode: query heads per block (attention_heads; 0: for the longest rows the table holds)
   int kvw, kvn, hpk;           // KV heads in x, their groups in z, query heads per KV head (set by attention_decode)
 };
 void attention_decode(const AttnParams& P, hipStream_t s);
 size_t attention_ws_floats(int NQ, int H, int D, int n_splits);
+int attention_heads(int NQ, int H, int n_kv, int D, long long keys);  // query heads per decode block, keys of the mean row
 extern int g_attn_kps;  // least decode keys per flash-decode split (scripts/bench_attn.py sweep)
 void set_attn_tuning(int kps, int hpb = -1);
 

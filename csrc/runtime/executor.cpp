@@ -292,6 +292,7 @@ void Executor::attn_block(int i, const StepInputs& in, hipStream_t s) {
   A.ws = ws.attn_ws;
   A.n_splits = ws.n_splits;
   A.counters = ws.attn_cnt;
+  A.heads = in.prefill ? 0 : ws.attn_heads;
   A.prefill = in.prefill;
   // deferred split merge (B == 1): the O projection's prologue merges the partial slabs
   const bool defer = ws.defer && B == 1 && ws.n_splits > 1;

@@ -81,6 +81,7 @@ struct Workspace {
   float* rope = nullptr;     // [maxB][n_rot / 2] {cosine, sine} of a prompt's positions, written in a pass's layer 0
   int max_B = 0;
   int n_splits = 1;
+  int attn_heads = 0;        // AttnParams::heads of decode steps
   int defer = 0;             // B == 1: attention leaves n_splits partials, the O GEMV merges them
   // TP decode: one-shot all-reduce over peer-mapped slabs (allreduce.hip). The O / down projections
   // write their partial sums into this rank's slab 0 / 1, the vocab-sharded LM head into slab 2.

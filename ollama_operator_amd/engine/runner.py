@@ -116,7 +116,7 @@ class NativeExec:
     def run(self, stage: str, layer: int, B: int, n_logits: int = 0, use_idx: bool = False,
             prefill: bool = False):
         S, defer = self.r.split_plan(B)
-        self.exe.set_splits(S, defer)
+        self.exe.set_splits(S, defer, self.r._decode_heads)
         self.exe.step(self.stages[stage], layer, B, n_logits, use_idx, prefill, stream_handle() if self.on_gpu else 0)
 
 
@@ -339,6 +339,7 @@ class Runner:
                           (native().gemv_merge_supported(1, Eq, loc["D"], 8) or
                            (ksplit and tp_size == 1 and native().gemv8_merge_supported(Eq, loc["D"], 8))))
         self._decode_S = 0
+        self._decode_heads = 0
         self._adv_next = None  # (sid, pos) the device step inputs were advanced to by the last decode
         # TP decode collectives: one-shot all-reduce over peer-mapped slabs (parallel/custom_ar.py),
         # decode-size messages only (<= ~1 MB); prefill chunks keep RCCL
@@ -481,6 +482,18 @@ class Runner:
         if S:
             return S, int(S > 1)
         return self.n_splits(B), 0
+
+    def decode_heads(self, poss: list[int]) -> int:
+        """Query heads per attention block of a decode step whose rows sit at `poss` (csrc/kernels/attention.hip
+        attention_heads, by the mean length; part of the step graph's key). 0: the kernel's own choice, where
+        lengths make no difference to it."""
+        loc, B = self.w.local, len(poss)
+        if not self.is_gpu or loc["H"] == loc["Hkv"] or B * loc["Hkv"] < 64:
+            return 0
+        keys = sum(poss) // B + 1
+        if self.cfg.sliding_window > 0:
+            keys = sum(min(p + 1, self.cfg.sliding_window) for p in poss) // B
+        return native().attention_heads(B, loc["H"], loc["Hkv"], self.Dc, keys)
 
     def decode_splits(self, length: int) -> int:
         """Flash-decode split bucket for a B == 1 step over `length` visible keys: 1 / 2 / 4 / 8
@@ -775,11 +788,14 @@ class Runner:
         if not self.is_gpu:
             self.d_tokens[:B].copy_(self.s_out[:B])
 
+    def _graph_key(self, B: int, steps: int, inst: int) -> tuple:
+        return B, self._decode_S, steps, inst, self._decode_heads
+
     def _graph(self, B: int, steps: int = 1, inst: int = 0):
         """The decode graph of `steps` consecutive steps for B rows (one replay = `steps` tokens per row:
         the feedback kernel advances every row on device between them, so no host work sits in between).
         inst: which of the two instances (graph_pair)."""
-        key = (B, self._decode_S, steps, inst)
+        key = self._graph_key(B, steps, inst)
         g = self.graphs.get(key)
         if g is None:
             s = torch.cuda.Stream()
@@ -920,6 +936,7 @@ class Runner:
         if not (self.is_gpu and not grown and self._adv_next == nxt):
             self._upload(arr, None)
         self._decode_S = self.decode_splits(poss[0] + 1) if B == 1 else 0
+        self._decode_heads = self.decode_heads(poss) if B > 1 else 0
         try:
             with trace_range(f"decode B={B}"):
                 if self.use_graphs:
@@ -930,7 +947,7 @@ class Runner:
                 self._adv_next = (sids[0], poss[0] + 1) if B == 1 else (tuple(sids), tuple(p + 1 for p in poss))
             self.steps_issued += 1
         finally:
-            self._decode_S = 0
+            self._decode_S = self._decode_heads = 0
 
     def sampler_error(self) -> bool:
         """True (and the word re-armed) when a sample since the last check met non-finite logits: the
@@ -1124,7 +1141,10 @@ class Runner:
         """Load-time capture of the B = 2..max_B decode graphs (continuous batching)."""
         if self.use_graphs:
             for B in range(2, max_B + 1):
-                self._graph(B)
+                for heads in sorted({self.decode_heads([0] * B), self.decode_heads([self.ctx - 1] * B)}):
+                    self._decode_heads = heads
+                    self._graph(B)
+            self._decode_heads = 0
             torch.cuda.synchronize()
 
     def _generate_pipelined(self, sid: int, st, first: int, max_tokens: int, stop, times, t1,

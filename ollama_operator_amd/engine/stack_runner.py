@@ -347,7 +347,7 @@ class StackRunner(Runner):
         self._alloc_step_state(V, n_blocks)
         self.decode_group, self.graph_pair, self.steps_issued = 1, False, 0
         self.ring_fence = 1 if os.environ.get("OMX_RING_FENCE", "0") == "1" else 0
-        self._defer_ok, self._decode_S, self._adv_next = False, 0, None
+        self._defer_ok, self._decode_S, self._decode_heads, self._adv_next = False, 0, 0, None
         if self.is_gpu:
             self.exe = StackExec(self)
         else:
@@ -380,6 +380,9 @@ class StackRunner(Runner):
 
     def split_plan(self, B: int) -> tuple[int, int]:
         return 1, 0
+
+    def decode_heads(self, poss: list[int]) -> int:
+        return 0
 
     def decode_splits(self, length: int) -> int:
         """Blocks per (row, head) of the decode attention over `length` keys: 1 up to 512 keys, then a power of
@@ -422,7 +425,7 @@ class StackRunner(Runner):
         """A graph captured in mid-generation: the warm-up forward that precedes the capture really runs, and a
         second run of the same rows would advance their recurrent states twice (a K/V write is the same write
         again, a state update is not). The states are put back after it."""
-        key = (B, self._decode_S, steps, inst)
+        key = self._graph_key(B, steps, inst)
         if key in self.graphs:
             return self.graphs[key]
         saved = [st.clone() if st is not None else None for st in self.states]
