@@ -301,6 +301,8 @@ PYBIND11_MODULE(_C, m) {
      py::arg("q_seq"), py::arg("q_len"), py::arg("NQ"), py::arg("H"), py::arg("n_kv"), py::arg("D"), py::arg("bs"),
      py::arg("scale"), py::arg("window"), py::arg("out"), py::arg("ldo"), py::arg("ws"), py::arg("n_splits"),
      py::arg("counters"), py::arg("stream"), py::arg("prefill") = 0, py::arg("Dv") = 0, py::arg("heads") = 0);
+  m.def("attention_even_splits", &attention_even_splits, "splits of decode rows of one length", py::arg("blocks"), py::arg("keys"),
+        py::arg("most"));
   m.def("attention_heads", &attention_heads, "query heads per decode block for rows of `keys` keys on average", py::arg("NQ"),
         py::arg("H"), py::arg("n_kv"), py::arg("D"), py::arg("keys"));
   m.def("attention_ws_floats", &attention_ws_floats);

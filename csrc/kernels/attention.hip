@@ -187,20 +187,32 @@ struct KVStep {
   Row k[U], v[U];
 };
 
-// Splits of a query's nk keys. The merge costs some 6 us (partials written through, a ticket, read back), so splits
-// are for CUs that would idle: a split takes about a 256th of the launch's work, kps keys at least, and up to 2 kps nothing is
-// split. Measured with heads_per_block and the block order below, before (splits of 256 keys whatever the launch, a
-// query's blocks on one XCD) -> now, us, 128 dims, rows x heads / KV heads:
-//   1 x 32 / 8: 400 keys 9.4 -> 7.6, 3,000 16.2 -> 10.6;  1 x 32 / 32: 1,500 11.7 -> 10.7;  4 x 32 / 8: 1,500 19.2 -> 14.3
-//   8 x 32 / 8: 400 17.0 -> 8.5, 1,500 32.2 -> 21.0;  16 x 32 / 8: 400 18.7 -> 12.1, 1,500 37.5 -> 27.8
-//   8 x 32 / 32: 400 14.6 -> 12.5;  8 x 64 / 8: 400 27.8 -> 12.2;  one row of 3,000 and 15 of 375, 32 / 8: 50.2 -> 27.2
-__device__ __forceinline__ int split_count(const AttnParams& P, int nk, int heads, int most) {
+// Splits of a query's nk keys. A split takes kps keys at least, and up to 2 kps nothing is split.
+//  * Rows of different lengths: a split takes about a 256th of the launch's work, the merge (some 6 us: partials written through, a
+//    ticket, read back) being for CUs that would idle. Which rows a query is served beside so decides where its sums are cut.
+//  * Rows around the mean length (a quarter): their blocks are of one size, and a few more than 256 of them take a round for
+//    themselves, so the splits are those of even_splits: rounds of blocks times what a block takes, a round's start and the merge
+//    put into keys (400, 150; one head: 4.9 us + 12.3 us per 1,000 keys, merged 6.4 us; four heads: 6.8 us + 20.8, merged 12.6).
+//    For up to 2,304 keys and more, on the host, which knows all of it but the lengths.
+// Measured with attention_heads and the block order below, us, 128 dims, rows x heads / KV heads: splits of 256 keys whatever the
+// launch, a query's blocks on one XCD / a 256th of the work for all rows / now
+//   3 x 32 / 32: 1,500 keys 19.0 / 22.5 / 18.0;  5 x 32 / 32: 4,000 57.3 / 68.4 / 57.3;  9 x 32 / 8: 4,000 49.6 / 57.0 / 39.0
+//   12 x 32 / 8: 1,500 37.2 / 37.2 / 26.1, 4,000 60.1 / 70.5 / 51.0;  17 x 32 / 8: 1,500 42.2 / 46.2 / 37.0, 4,000 79.5 / 95.6 / 75.6
+//   1 x 32 / 8: 4,000 16.8 / 12.4 / 12.4;  16 x 32 / 8, one of 4,000 and 15 of 500: 61.8 / 31 / 31.1
+// Over 340 points (1 to 24 rows, four groupings, 700 to 4,000 keys, even and ragged) 0.78 of the first's time; behind it by 3 to 6 %: 32
+// heads on 32, one row of 4,000 keys alone or beside one to four of 500.
+// first: q_len of row lane (0 past the rows), requested ahead.
+__device__ __forceinline__ int split_count(const AttnParams& P, int nk, int heads, int most, int first) {
   if (most == 1 || nk <= 2 * P.kps) return 1;
-  const int lane = threadIdx.x & 63;
-  float total = 0.f;
-  for (int i = lane; i < P.NQ; i += 64) total += (float)(P.window > 0 ? min(P.window, P.q_len[i]) : P.q_len[i]);
-  const int share = max(P.kps, (int)(wave_sum(total) * (float)heads * (1.f / 256.f)));
-  return max(1, min(most, (nk + share / 2) / share));
+  auto seen = [&](int len) { return (float)(P.window > 0 ? min(P.window, len) : len); };
+  float total = seen(first);
+  for (int i = (threadIdx.x & 63) + 64; i < P.NQ; i += 64) total += seen(P.q_len[i]);
+  total = wave_sum(total);
+  const float n = (float)nk;
+  const int share = max(P.kps, (int)(total * (float)heads * (1.f / 256.f)));
+  int S = (nk + share / 2) / share;
+  if (fabsf(n * (float)P.NQ - total) <= 0.25f * total) S = min(nk > 2304 ? P.even_long : P.even, (nk + P.kps / 2) / P.kps);
+  return max(1, min(most, S));
 }
 
 // U key slots per lane group per step: 4, or 2 when 8 query heads share a KV head or the head dim is
@@ -225,13 +237,15 @@ __global__ __launch_bounds__(ATT_NT) void attn_decode_kernel(AttnParams P) {
   const int split = P.kvn == 1 ? (int)blockIdx.z : (int)blockIdx.z / P.kvn;
   const int kvh = ((int)blockIdx.z - split * P.kvn) * P.kvw + col;  // KV head of this block's G query heads
   const int h0 = kvh * P.hpk + mem * G;  // the first of them
+  const int first = splits > 1 && !P.defer && (int)(threadIdx.x & 63) < P.NQ ? P.q_len[threadIdx.x & 63] : 0;
   const int seq = P.q_seq ? P.q_seq[qi] : qi;
   const int len = P.q_len[qi];
   const int kstart = P.window > 0 ? max(0, len - P.window) : 0;
   const int nk = len - kstart;
+  if (!P.defer && (split - 0.5f) * (float)P.kps > (float)nk) return;  // (split_count gives no row that many)
   // deferred merge: exactly n_splits splits (empty ones publish m = -inf, l = 0) and the consumer
   // (the O-projection GEMV prologue) merges them; otherwise the split count follows the length
-  const int S = P.defer ? splits : split_count(P, nk, P.H / G, splits);
+  const int S = P.defer ? splits : split_count(P, nk, P.H / G, splits, first);
   if (split >= S) return;  // block-uniform: surplus splits of a short query leave immediately
   const int chunk = (nk + S - 1) / S;
   const int t0 = kstart + split * chunk;
@@ -814,6 +828,18 @@ static int heads_per_block(const AttnParams& P) {
   return hpb;
 }
 
+// splits of rows of one length: b blocks a split, `keys` each row
+int attention_even_splits(int b, int keys, int most) {
+  auto rounds = [](int blocks) { return (blocks + 255) / 256; };
+  int best = 1;
+  double least = rounds(b) * (keys + 400.);
+  for (int k = 2; k <= most; ++k) {
+    const double t = rounds(b * k) * ((double)keys / k + 400.) + 150.;
+    if (t < 0.93 * least || (best > 1 && t < least)) least = t, best = k;
+  }
+  return best;
+}
+
 template <int D, bool KV8>
 static void launch_dk(const AttnParams& P0, hipStream_t s) {
   const int G = heads_per_block(P0);
@@ -821,6 +847,11 @@ static void launch_dk(const AttnParams& P0, hipStream_t s) {
   P.kvw = P.n_kv % 8 ? P.n_kv : 8;  // the blocks of a KV head are 8 apart
   P.kvn = P.n_kv / P.kvw;
   P.hpk = P.H / P.n_kv;
+  // no row is split further than into a block for each CU (split_count), and blocks that find nothing to do are not free
+  const int heads = P.H / G;
+  if (!P.defer) P.n_splits = std::min(P.n_splits, std::max(3, (256 + heads / 2) / heads));
+  P.even = attention_even_splits(P.NQ * heads, 1500, P.n_splits);
+  P.even_long = attention_even_splits(P.NQ * heads, 4000, P.n_splits);
   dim3 grid(P.kvw * (P.hpk / G), P.NQ, P.kvn * P.n_splits);
   // 8 lanes per key: fp8 rows at D = 128 (8 lanes x 16 B), and fp16 rows of head dims 80 / 96 / 112 (20-28 B
   // per lane in 2-3 vector loads; at 16 lanes a lane's 10-14 B are 2-B aligned: one load per element)

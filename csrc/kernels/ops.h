@@ -259,10 +259,12 @@ struct AttnParams {
                                // [NQ][S][H*D] then [NQ][S][H][2] {m, l}); the consumer merges them
   int kv8;                     // kc / vc hold fp8 e4m3 (OCP e4m3fn) instead of fp16
   int heads;                   // decode: query heads per block (attention_heads; 0: for the longest rows the table holds)
-  int kvw, kvn, hpk;           // KV heads in x, their groups in z, query heads per KV head (set by attention_decode)
+  int kvw, kvn, hpk;           // KV heads in x, their groups in z, query heads per KV head (set by attention_decode,
+  int even, even_long;         // as the splits of rows of one length, up to 2,304 keys and longer)
 };
 void attention_decode(const AttnParams& P, hipStream_t s);
 size_t attention_ws_floats(int NQ, int H, int D, int n_splits);
+int attention_even_splits(int b, int keys, int most);  // splits of decode rows of one length, b blocks a split
 int attention_heads(int NQ, int H, int n_kv, int D, long long keys);  // query heads per decode block, keys of the mean row
 extern int g_attn_kps;  // least decode keys per flash-decode split (scripts/bench_attn.py sweep)
 void set_attn_tuning(int kps, int hpb = -1);

@@ -19,6 +19,19 @@ def test_rule(NQ, H, n_kv, D, short, grown):
     assert (H // n_kv) % short == 0 and (H // n_kv) % grown == 0
 
 
+def test_even_rows_fill_whole_rounds():
+    """Splits of rows of one length: no few blocks past a round of 256, which would take a round for themselves."""
+    splits = native().attention_even_splits
+    assert [splits(b, 1500, 16) for b in (32, 64, 72, 96, 128, 160, 200, 256, 257)] == [8, 4, 3, 2, 2, 1, 1, 1, 1]
+    assert [splits(b, 4000, 3) for b in (136, 160, 192, 272)] == [3, 3, 1, 3]  # long rows: two or four rounds of thirds
+    for b in range(1, 600):
+        for keys in (1500, 4000):
+            k = splits(b, keys, 8)
+            rounds = -(-b * k // 256)
+            # one split more would not fit the rounds that there are, and (256 // 86 = 2) two thirds of them are busy
+            assert k in (1, 8) or (b * (k + 1) > 256 * rounds and b * k > 256 * rounds * 2 / 3), (b, keys, k)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("graphs", [True, False])
 def test_steps_follow_the_lengths(tiny_models, monkeypatch, graphs):
