@@ -409,7 +409,7 @@ void Executor::ffn_block(int i, const StepInputs& in, hipStream_t s) {
     }
     if (B >= GEMM_MIN_B && ws.x16 && ws.moe_rows) {
       // prefill: grouped MFMA GEMM over expert-homogeneous tiles of the sorted (token, expert)
-      // pairs -- each expert's weights stream once per 128 routed rows, not once per pair
+      // pairs -- each expert's weights stream once per tile of routed rows, not once per pair
       const int pairs = B * k;
       auto grouped = [&](GemvParams& P) {
         P.n_sel = k;

@@ -18,7 +18,10 @@ pytestmark = pytest.mark.gpu
     (FileType.MOSTLY_Q4_K_M, 1024, 17, 512), (FileType.MOSTLY_Q4_0, 1280, 129, 512),
     # widths that are no multiple of 256 (padded K) nor of 128 (the last columns of an expert's tile), a full portion among them
     (FileType.MOSTLY_Q4_0, 1056, 640, 576), (FileType.MOSTLY_Q8_0, 1056, 101, 576), (FileType.MOSTLY_Q4_0, 2144, 40, 1088),
-    (FileType.MOSTLY_Q8_0, 1120, 640, 1088)])
+    (FileType.MOSTLY_Q8_0, 1120, 640, 1088),
+    # up to 128 rows an expert on average (tiles in halves): at the limit some experts have more, the second half of a tile a few
+    (FileType.MOSTLY_Q4_K_M, 1024, 256, 512), (FileType.MOSTLY_Q5_K_S, 1280, 250, 512), (FileType.MOSTLY_Q6_K, 1280, 256, 512),
+    (FileType.MOSTLY_Q6_K, 1024, 33, 512), (FileType.MOSTLY_Q8_0, 1056, 256, 576), (FileType.MOSTLY_Q4_0, 1056, 255, 576)])
 def test_grouped_experts(tmp_path, ft, n_ff, rows, n_embd):
     """Against float32 on the CPU, beside the path that is taken with these kernels switched off: both round the same two
     operands to fp16 and add in float32, so neither may be further from float32 than the other by more than the order of sums
