@@ -106,7 +106,8 @@ bool dq_gemm(const GemvParams& P, hipStream_t s) {
 // Whole prompts (Q4_K_M) on this path / on the others (executor.cpp ffn_block), us. Four layers of 8 experts, top 2, of 1,024 x 1,024
 // (width x feed-forward: 2,048 rows of gate and up): 17 rows 335 / 463, 130 463 / 1,606, 400 576 / 1,819; of 2,048 x 4,096: 17 rows 596 /
 // 1,037, 1,000 1,622 / 3,237. Two layers of 64 experts, top 8, of 1,024 x 2,048: 17 rows 365 / 488, 1,000 1,413 / 6,667; of 8 of 4,096 x
-// 14,336: 17 rows 1,039 / 2,265, 64 1,076 / 2,362, 260 1,293 / 4,182, 1,000 2,733 / 5,357. Smaller experts (not measured) stay with the others.
+// 14,336: 17 rows 1,039 / 2,265, 64 1,076 / 2,362, 260 1,293 / 4,182, 1,000 2,733 / 5,357. Smaller experts (not measured) stay with
+// the others.
 static bool moe_matrix(const QMat& w) {
   const int qt = w.qtype;
   return w.K % 4 == 0 && ((w.K + 255) >> 8) * 256 <= PREP_MAX_KP &&

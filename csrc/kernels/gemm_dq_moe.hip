@@ -23,7 +23,7 @@ __global__ __launch_bounds__(256, 1) void dq_moe_kernel(GemvParams P, const f16*
 
 // The same in tiles of 128 x 128, a table's tile in two halves, two blocks a CU: for up to 128 rows an expert, where the products
 // are bound by the weights' way in and 256 columns a block leave CUs without one (8 experts x 4,096 columns: 128 blocks). us, 128 x
-// 128 tiles of eight waves / the kernel above / this, 8 experts, top 2, down 4,096 x 14,336 (Q4_K, Q6_K) and gate / up 28,672 x 4,096 (Q4_K):
+// 128 tiles of eight waves / the kernel above / this, 8 experts, top 2: down 4,096 x 14,336 (Q4_K), (Q6_K), gate / up 28,672 x 4,096:
 //   17 rows 200 / 207 / 132, 241 / 314 / 185, 318 / 271 / 254;  260 rows 210 / 215 / 149, 246 / 347 / 226, 336 / 292 / 275
 //   400 rows 214 / 227 / 171, 251 / 361 / 241, 345 / 303 / 288
 //   600 rows - / 307 / 282, - / 429 / 429, - / 469 / 551;  1,000 rows - / 341 / 424, - / 477 / 672, - / 704 / 808
@@ -43,7 +43,8 @@ void run_moe(const GemvParams& P, f16* xp, int Kp, hipStream_t s) {
   hipLaunchKernelGGL(prep_xp_kernel<QT>, dim3(P.B), dim3(256), (size_t)Kp * sizeof(float), s, P, xp, Kp);
   const int experts = P.moe_max_tiles - (P.B + DQ_MOE_TILE_M - 1) / DQ_MOE_TILE_M;  // (the table's bound: a rest for each)
   if (P.B <= 128 * experts) {
-    hipLaunchKernelGGL(dq_moe_half_kernel<QT>, dim3(P.moe_max_tiles * 2 * ((P.w.N + 127) / 128)), dim3(256), (ds_lds<4, 1>()), s, P, xp, Kp);
+    hipLaunchKernelGGL(dq_moe_half_kernel<QT>, dim3(P.moe_max_tiles * 2 * ((P.w.N + 127) / 128)), dim3(256), (ds_lds<4, 1>()), s, P, xp,
+                       Kp);
     return;
   }
   hipLaunchKernelGGL(dq_moe_kernel<QT>, dim3(P.moe_max_tiles * ((P.w.N + 255) / 256)), dim3(256), (ds_lds<8, 2>()), s, P, xp, Kp);
