@@ -183,7 +183,7 @@ def test_mb_fp16_input_with_rms_partials(qt, B, K):
     parts = torch.zeros(16, K // 16, device="cuda")  # [batch row][16-row tile] as producers write them
     parts[:B] = x.pow(2).reshape(B, K // 16, 16).sum(-1)
     y = torch.zeros(B, N, device="cuda")
-    gemv(m, x, norm=1, nw=nw, y=y, extra=dict(x16=x16.data_ptr(), ld16=ld, zrow16=B, xstat=parts.data_ptr(),
+    gemv(m, x, norm=1, nw=nw, y=y, extra=dict(x16=x16.data_ptr(), ld16=ld, xstat=parts.data_ptr(),
                                               xstat_n=K // 16))
     xn = x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + 1e-5) * nw
     assert rel(y, xn @ m.w.T) < 4e-3, (qt, B, K)
@@ -226,7 +226,7 @@ def test_mb_chain_matches_fused_norm():
     gemv(mo, a, epi=1, y=resid, extra=dict(emit16=e16.data_ptr(), ld_emit=E, emit_nw=nw.data_ptr(),
                                            emit_stat=st.data_ptr()))
     y_chain = torch.zeros(B, F, device="cuda")
-    gemv(mg, resid, norm=1, nw=nw, y=y_chain, extra=dict(x16=e16.data_ptr(), ld16=E, zrow16=B, xstat=st.data_ptr(),
+    gemv(mg, resid, norm=1, nw=nw, y=y_chain, extra=dict(x16=e16.data_ptr(), ld16=E, xstat=st.data_ptr(),
                                                          xstat_n=E // 16))
     y_lds = torch.zeros(B, F, device="cuda")
     gemv(mg, resid, norm=1, nw=nw, y=y_lds)
@@ -275,7 +275,7 @@ def test_mb_chain_range_scale(qt):
     assert bool(torch.isfinite(e16[:B].float()).all())
     assert rel(e16[:B].float() * scale[:, None], resid * nw) < 1e-3
     y_chain = torch.zeros(B, F, device="cuda")
-    gemv(mg, resid, norm=1, nw=nw, y=y_chain, extra=dict(x16=e16.data_ptr(), ld16=E, zrow16=B, xstat=st.data_ptr(),
+    gemv(mg, resid, norm=1, nw=nw, y=y_chain, extra=dict(x16=e16.data_ptr(), ld16=E, xstat=st.data_ptr(),
                                                          xstat_n=n, xscale=st[16 * n:].data_ptr()))
     y_lds = torch.zeros(B, F, device="cuda")
     gemv(mg, resid, norm=1, nw=nw, y=y_lds)
