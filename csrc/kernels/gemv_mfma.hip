@@ -887,15 +887,8 @@ bool gemv_mb2(const GemvParams& A, const GemvParams& Bp, hipStream_t s) {
   ga = ga < 1 ? 1 : ga > ta ? ta : ga;
   int gb = ncu - ga;
   gb = gb < 1 ? 1 : gb > tb ? tb : gb;
-  const size_t lds = mb_lds_bytes(A.B, A.w.K, AM_G16);
-  auto go = [&](auto kern) {
-    static bool attr = false;
-    if (!attr) {
-      (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-      attr = true;
-    }
-    hipLaunchKernelGGL(kern, dim3(ga + gb), dim3(MB_NT), lds, s, A, Bp, ga);
-  };
+  const size_t lds = mb_lds_bytes(A.B, A.w.K, AM_G16);  // 17 KB (the rows are in memory): no attribute needed
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(ga + gb), dim3(MB_NT), lds, s, A, Bp, ga); };
   if (nsbw == 1) go(gemv_mb2_kernel<QT_Q4_K, QT_Q6_K, 1, 4, AM_G16, 7>);
   else if (mb_operands(A) != 4 || mb_operands(Bp) != 4) go(gemv_mb2_kernel<QT_Q4_K, QT_Q6_K, 2, 2, AM_G16, 7>);
   else go(gemv_mb2_kernel<QT_Q4_K, QT_Q6_K, 2, 2, AM_G16, 4>);
