@@ -207,6 +207,10 @@ void run_rows(const GemvParams& P, f16* xp, int Kp, hipStream_t s) {
   // at 32; 6144 17.9 at 32, 21.5 at 48, 22.8 at 16; 4096 14.7 at 16, 16.9 at 32); at 64 rows three column tiles do not fit
   // the registers. Over 22 matrices of 512 .. 32,000 rows, five weight types and 16 .. 64 rows the launch takes 0.51 of the
   // tile kernel's time on average, and no point takes more
+  // Four waves a block instead of eight where 257 to 512 blocks of 48 columns then run at once, two on each of the 256 CUs (33 rows,
+  // us, four / eight: Q4_K x 4,096 N = 12,032 23.0 / 21.3, 12,800 29.0 / 33.2, 22,016 30.9 / 34.5, 24,576 31.6 / 35.7; Q6_K 25.9 / 25.6,
+  // 36.8 / 41.7, 39.3 / 44.1, 39.7 / 45.1). Past 512 blocks four were ahead too when this was measured again (28,672: Q4_K 43.2 / 47.9,
+  // Q6_K 54.2 / 61.7); the line was drawn at the round.
   const bool wide = N >= 48 * 208, middle = N >= 32 * 160;
   if (P.B <= 48) {
     if (wide && N > 48 * 256 && N <= 48 * 512) launch_rows<QT, 3, 3, 4>(P, xp, Kp, s);
