@@ -303,7 +303,10 @@ PYBIND11_MODULE(_C, m) {
      py::arg("counters"), py::arg("stream"), py::arg("prefill") = 0, py::arg("Dv") = 0, py::arg("heads") = 0);
   m.def("attention_even_splits", &attention_even_splits, "splits of decode rows of one length", py::arg("blocks"), py::arg("keys"),
         py::arg("most"));
-  m.def("attention_heads", &attention_heads, "query heads per decode block for rows of `keys` keys on average", py::arg("NQ"),
+  m.def("attention_heads", [](int NQ, int H, int n_kv, int D, long long keys) {
+    if (n_kv < 1 || H < n_kv || H % n_kv) throw std::runtime_error("attention_heads: H must be a multiple of n_kv");
+    return attention_heads(NQ, H, n_kv, D, keys);
+  }, "query heads per decode block for rows of `keys` keys on average", py::arg("NQ"),
         py::arg("H"), py::arg("n_kv"), py::arg("D"), py::arg("keys"));
   m.def("attention_ws_floats", &attention_ws_floats);
   m.def("set_attn_tuning", &set_attn_tuning, py::arg("kps"), py::arg("hpb") = -1);

@@ -19,6 +19,12 @@ def test_rule(NQ, H, n_kv, D, short, grown):
     assert (H // n_kv) % short == 0 and (H // n_kv) % grown == 0
 
 
+@pytest.mark.parametrize("H,n_kv", [(32, 0), (4, 8), (32, 5), (32, -1)])
+def test_heads_without_groups_are_refused(H, n_kv):
+    with pytest.raises(RuntimeError, match="multiple of n_kv"):
+        native().attention_heads(8, H, n_kv, 128, 100)
+
+
 def test_even_rows_fill_whole_rounds():
     """Splits of rows of one length: no few blocks past a round of 256, which would take a round for themselves."""
     splits = native().attention_even_splits
